@@ -176,7 +176,7 @@ class Context:
     # ---- fields (Fortran-ordered numpy arrays, ghosts included) ----
     def get(self, b, fid):
         shp = self.shape(b, fid)
-        out = np.zeros(int(np.prod(shp)))
+        out = np.empty(int(np.prod(shp)))
         _check(lib.snac_download_field(self.h, b, FIELDS[fid], out), "snac_download_field")
         return out.reshape(shp, order="F")
 

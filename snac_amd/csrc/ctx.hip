@@ -16,6 +16,7 @@
 #include "bound_program.hpp"
 #include "case.hpp"
 #include "common.hpp"
+#include "hostcopy.hpp"
 #include "io.hpp"
 #include "mg.hpp"
 
@@ -119,6 +120,7 @@ struct snac_ctx {
   int nparts = 0;
   double dlmin = 0;
   std::vector<void *> owned;
+  snac::HostCopy xfer;  // field uploads and downloads
   // phase timers
   bool timing = false;
   struct TRec { int ph; hipEvent_t a, b; };
@@ -1356,6 +1358,7 @@ void create(snac_ctx *c) {
 
 void destroy(snac_ctx *c) {
   if (c->stream) (void)hipStreamSynchronize(c->stream);
+  c->xfer.release();
   mg_free(c->mg);
   drop_graph(c);
   for (auto &r : c->pending) { (void)hipEventDestroy(r.a); (void)hipEventDestroy(r.b); }
@@ -1660,19 +1663,13 @@ void copy_field(snac_ctx *c, int b, int fid, double *dst_host, const double *src
     // one component's rows, 3 nx apart on the device, contiguous on the host;
     // with FP32 stencils the tendencies live in dto32 and pass through the
     // FP64 array
-    size_t w = (size_t)D.g.nx * sizeof(double), pitch = 3 * w, rows = (size_t)D.g.ny * D.g.nz;
     if (c->st32) launch_cvt_f2d(c->stream, D.dto32, D.dto[0], 3 * D.nin);
-    if (src_host) SNAC_HIP(hipMemcpy2DAsync(d, pitch, src_host, w, w, rows, hipMemcpyHostToDevice, c->stream));
-    else SNAC_HIP(hipMemcpy2DAsync(dst_host, w, d, pitch, w, rows, hipMemcpyDeviceToHost, c->stream));
+    c->xfer.run(c->device, c->stream, d, 3L * D.g.nx, D.g.nx, (long)D.g.ny * D.g.nz, dst_host, src_host);
     if (c->st32 && src_host) launch_cvt_d2f(c->stream, D.dto[0], D.dto32, 3 * D.nin);
   } else if (ghosted) {
-    size_t w = (size_t)(D.g.nx + 2) * sizeof(double), pitch = (size_t)D.g.sx * sizeof(double);
-    size_t rows = (size_t)(D.g.ny + 2) * (D.g.nz + 2);
-    if (src_host) SNAC_HIP(hipMemcpy2DAsync(d, pitch, src_host, w, w, rows, hipMemcpyHostToDevice, c->stream));
-    else SNAC_HIP(hipMemcpy2DAsync(dst_host, w, d, pitch, w, rows, hipMemcpyDeviceToHost, c->stream));
+    c->xfer.run(c->device, c->stream, d, D.g.sx, D.g.nx + 2, (long)(D.g.ny + 2) * (D.g.nz + 2), dst_host, src_host);
   } else {
-    if (src_host) SNAC_HIP(hipMemcpyAsync(d, src_host, n * sizeof(double), hipMemcpyHostToDevice, c->stream));
-    else SNAC_HIP(hipMemcpyAsync(dst_host, d, n * sizeof(double), hipMemcpyDeviceToHost, c->stream));
+    c->xfer.run(c->device, c->stream, d, D.g.nx, D.g.nx, (long)D.g.ny * D.g.nz, dst_host, src_host);
   }
   SNAC_HIP(hipStreamSynchronize(c->stream));
 }
