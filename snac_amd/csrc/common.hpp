@@ -163,12 +163,13 @@ void launch_face_ops(hipStream_t s, const FaceOp *dev_ops, int nops, int max_pla
 struct R2RPlan {
   int n = 0, kind = 0;
   bool fft = false;        // LDS FFT path (n a power of two >= 4, supported kind)
+  bool mfma = false;       // matrix product on the matrix cores (tab: its fragments)
   int lshift = 0;          // FFT tile (autotuned): 0..2 lines per workgroup = max >> lshift;
                            // 3, 4 (R2HC/HC2R): full tiles, 2 / 4 per workgroup, pipelined
                            // 5 (R2HC/HC2R): full tiles, wavefront-local passes;
                            // 6 (R2HC/HC2R): full tiles, the FFT's factors swapped;
                            // 7 (R2HC/HC2R): wavefront-local passes, factors swapped
-  const double *tab = nullptr;  // device twiddles (fft) or dense matrix
+  const double *tab = nullptr;  // device twiddles (fft), matrix fragments (mfma) or dense matrix
 };
 R2RPlan r2r_plan(int kind, int n);  // cached per (kind, n); throws if unsupported
 int r2r_tile_choices(const R2RPlan &pl);  // number of tile choices of the plan's kernel

@@ -1,8 +1,9 @@
 // Batched real-to-real transforms along one axis, the kinds FFTW offers and
 // SNaC selects by boundary condition (fft.f90:96-149): R2HC/HC2R (periodic),
 // REDFT10/REDFT01 (Neumann-Neumann), RODFT10/RODFT01 (Dirichlet-Dirichlet);
-// REDFT11/RODFT11 (mixed) and lengths that are not powers of two go through
-// a dense matrix path.  Unnormalised, as FFTW's; callers scale.
+// REDFT11/RODFT11 (mixed), RODFT00 and lengths that are not powers of two are
+// matrix products on the matrix cores.  Unnormalised, as FFTW's; callers
+// scale.
 //
 // FFT path (n = 4..1024, powers of two): a workgroup stages L whole lines in
 // LDS, forms the kind's n-point complex sequence (halfcomplex unpacking for
@@ -572,6 +573,147 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void k_
   }
 }
 
+// Dense transforms on the FP64 matrix cores: the kinds and lengths without a
+// power-of-two FFT.  A transform of n points is a matrix product Y = M X over
+// the lines; most kinds' matrices are symmetric or antisymmetric under a
+// mirror of the samples (j -> n - j for R2HC / HC2R, n - 1 - j for the cosine
+// and sine kinds), so the product splits into a symmetric and an
+// antisymmetric part of half the size each, half the multiplications:
+//   MODE 1 (R2HC, REDFT10, RODFT10, RODFT00): the input is folded,
+//     s_j = x_j + x_mirror, a_j = x_j - x_mirror as it is loaded;
+//   MODE 2 (HC2R, REDFT01, RODFT01): the output is unfolded,
+//     y_j = E_j + O_j, y_mirror = E_j - O_j;
+//   MODE 0 (REDFT11, RODFT11): no fold.
+// A workgroup holds L = 16 NTL LG lines in LDS; each of its wavefronts takes
+// tiles of 16 matrix rows for 16 NTL of them (v_mfma_f64_16x16x4).  The
+// matrix comes from memory in the instruction's operand order, 512
+// contiguous bytes per load, L2-resident and used for NTL products.  With
+// SWAP (outputs contiguous along the line) the operands change places, so
+// that the 16 lanes of a result row hold consecutive outputs of one line and
+// the stores are 128-byte runs either way.
+// Bound: 2 n (MODE 0) or n FP64 operations per point at the matrix rate (72
+// TFLOP/s measured on a large product) against 16 bytes per point; at n = 192
+// the folded product takes about as long as the memory does.  The form it
+// replaces walked a matrix row per thread (8-byte loads a row apart): 347 us
+// on average over the transforms of a 192x96x96 box, 17-22 us now (1.6 TB/s
+// of the lines' bytes); 146 -> 12-17 us for a 180x77x90 channel's, 8.1 -> 3.4
+// us for two-point lines.
+typedef double double4_ __attribute__((ext_vector_type(4)));
+struct MArgs {
+  const double *in;
+  double *out;
+  long ies, is1, is2, oes, os1, os2;
+  const double *fs, *fa;  // matrix fragments [tile][k / 4][64] of the two parts
+  double scale;
+  int n, nb1, nlines;
+  int half;     // samples up to the mirror (MODE 0: n)
+  int rows;     // matrix rows of the symmetric part (MODE 2: of both)
+  int ks, ka;   // inner lengths of the two parts
+  int na;       // MODE 1: rows of the antisymmetric part
+  int hc;       // 1: R2HC / HC2R index maps, 0: even / odd
+  int ld, ntile, tw, lg;
+};
+
+template <int MODE, bool SWAP, int NTL>
+__global__ __launch_bounds__(512) void k_r2r_mfma(MArgs a) {
+  extern __shared__ double2 S[];
+  const int L = 16 * NTL * a.lg, nthr = 64 * a.tw * a.lg, n = a.n;
+  double *X = reinterpret_cast<double *>(S);  // [L][ld]: symmetric part, then (at ksp) the antisymmetric one
+  long *oin = reinterpret_cast<long *>(X + (size_t)L * a.ld), *oout = oin + L;
+  const int ksp = (a.ks + 3) & ~3, kap = (a.ka + 3) & ~3;
+  const int line0 = blockIdx.x * L;
+  for (int t = threadIdx.x; t < L; t += nthr) {
+    const int line = line0 + t;
+    long oi = -1, oo = -1;
+    if (line < a.nlines) {
+      const int b1 = line % a.nb1, b2 = line / a.nb1;
+      oi = b1 * a.is1 + b2 * a.is2;
+      oo = b1 * a.os1 + b2 * a.os2;
+    }
+    oin[t] = oi;
+    oout[t] = oo;
+  }
+  __syncthreads();
+  // 1. lines into LDS: folded (MODE 1), sorted into the two parts (MODE 2) or
+  // as they are; the inner dimension's padding is zero
+  const bool coal = a.ies != 1;  // consecutive threads on consecutive lines
+  const int cols = MODE == 1 ? a.half : n, lsh = __ffs(L) - 1;  // L is a power of two
+  for (int e = threadIdx.x; e < L * cols; e += nthr) {
+    const int l = coal ? e & (L - 1) : e / cols, j = coal ? e >> lsh : e - l * cols;
+    const long o = oin[l];
+    double *row = X + l * a.ld;
+    const double x = o >= 0 ? a.in[j * a.ies + o] : 0.0;
+    if (MODE == 1) {
+      const int mir = a.hc ? (j == 0 ? 0 : n - j) : n - 1 - j;
+      const double y = mir != j && o >= 0 ? a.in[mir * a.ies + o] : 0.0;
+      row[j] = x + y;
+      if (j < a.ka) row[ksp + j] = mir != j ? x - y : 0.0;
+    } else if (MODE == 2) {
+      if (a.hc) row[j < a.ks ? j : ksp + n - 1 - j] = x;
+      else row[(j & 1) ? ksp + (j >> 1) : j >> 1] = x;
+    } else {
+      row[j] = x;
+    }
+  }
+  for (int l = threadIdx.x; l < L; l += nthr) {
+    double *row = X + l * a.ld;
+    for (int k = a.ks; k < ksp; k++) row[k] = 0.0;
+    for (int k = a.ka; k < kap; k++) row[ksp + k] = 0.0;
+  }
+  __syncthreads();
+  const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), ln = threadIdx.x & 63;
+  const int lq = ln & 15, kq = ln >> 4, l0 = (wv / a.tw) * 16 * NTL;
+  for (int tile = wv % a.tw; tile < a.ntile; tile += a.tw) {
+    double4_ es[NTL], ea[NTL];
+#pragma unroll
+    for (int t = 0; t < NTL; t++) { es[t] = double4_{0, 0, 0, 0}; ea[t] = double4_{0, 0, 0, 0}; }
+    // 2. the two products; operand layout: lane -> (row or column ln & 15, inner ln >> 4)
+    const double *xs = X + (l0 + lq) * a.ld + kq;
+    auto product = [&](const double *f, const double *x, int nk, double4_ (&acc)[NTL]) {
+      auto step = [&](double m, int k) {
+#pragma unroll
+        for (int t = 0; t < NTL; t++) {
+          const double b = x[t * 16 * a.ld + 4 * k];
+          acc[t] = SWAP ? __builtin_amdgcn_mfma_f64_16x16x4f64(b, m, acc[t], 0, 0, 0)
+                        : __builtin_amdgcn_mfma_f64_16x16x4f64(m, b, acc[t], 0, 0, 0);
+        }
+      };
+      f += ln;
+      int k = 0;
+      for (; k + 4 <= nk; k += 4, f += 256) {  // four matrix loads in flight
+        const double m0 = f[0], m1 = f[64], m2 = f[128], m3 = f[192];
+        step(m0, k);
+        step(m1, k + 1);
+        step(m2, k + 2);
+        step(m3, k + 3);
+      }
+      for (; k < nk; k++, f += 64) step(f[0], k);
+    };
+    product(a.fs + (size_t)tile * (ksp / 4) * 64, xs, ksp / 4, es);
+    if (MODE != 0) product(a.fa + (size_t)tile * (kap / 4) * 64, xs + ksp, kap / 4, ea);
+    // 3. results: register v of a lane is row 4 v + (ln >> 4), column ln & 15
+#pragma unroll
+    for (int t = 0; t < NTL; t++)
+#pragma unroll
+      for (int v = 0; v < 4; v++) {
+        const int l = l0 + 16 * t + (SWAP ? 4 * v + kq : lq), r = 16 * tile + (SWAP ? lq : 4 * v + kq);
+        const long o = oout[l];
+        if (o < 0 || r >= a.rows) continue;
+        double *y = a.out + o;
+        if (MODE == 0) {
+          y[r * a.oes] = es[t][v] * a.scale;
+        } else if (MODE == 1) {
+          y[(a.hc ? r : 2 * r) * a.oes] = es[t][v] * a.scale;
+          if (r < a.na) y[(a.hc ? n - 1 - r : 2 * r + 1) * a.oes] = ea[t][v] * a.scale;
+        } else {
+          const int mir = a.hc ? (r == 0 ? 0 : n - r) : n - 1 - r;
+          y[r * a.oes] = (es[t][v] + ea[t][v]) * a.scale;
+          if (mir != r) y[mir * a.oes] = (es[t][v] - ea[t][v]) * a.scale;
+        }
+      }
+  }
+}
+
 __global__ __launch_bounds__(NT) void k_r2r_dense(Args a) {
   extern __shared__ double2 S[];
   double *R = reinterpret_cast<double *>(S);
@@ -708,6 +850,106 @@ void launch_rfft(bool inv, int n, int ls, dim3 grid, size_t lds, hipStream_t s, 
   }
 }
 
+// ---- the matrix-core form: index maps, fragments, launch shape ----
+// the split of kind's matrix under the mirror (k_r2r_mfma); Y[r] of a part is
+// the sum over c of coef(out(r), in(c))
+struct MSplit {
+  int mode, hc, half, rows, na, ks, ka;
+};
+MSplit mfma_split(int kind, int n) {
+  MSplit m{};
+  m.hc = kind == K_R2HC || kind == K_HC2R;
+  m.mode = kind == K_REDFT11 || kind == K_RODFT11                                                 ? 0
+           : kind == K_HC2R || kind == K_REDFT01 || kind == K_RODFT01                             ? 2
+                                                                                                  : 1;
+  if (m.mode == 0) {
+    m.half = m.rows = m.ks = n;
+    return m;
+  }
+  m.half = m.hc ? n / 2 + 1 : (n + 1) / 2;
+  const int sym = m.half, anti = n - m.half;  // the sizes of the two parts on the transformed side
+  if (m.mode == 1) {
+    m.rows = sym;
+    m.na = anti;
+    m.ks = m.ka = m.half;
+  } else {
+    m.rows = m.half;
+    m.ks = sym;
+    m.ka = anti;
+  }
+  return m;
+}
+
+// LDS doubles per line: both parts, padded to a row that is an odd multiple
+// of two doubles, so that the 16 lines of an operand read fall on different banks
+int mfma_ld(const MSplit &m) {
+  const int ld = ((m.ks + 3) & ~3) + ((m.ka + 3) & ~3);
+  return ld + 2;  // a multiple of 4, plus 2
+}
+size_t mfma_lds(int ld, int lines) { return (size_t)lines * (ld * sizeof(double) + 2 * sizeof(long)); }
+constexpr size_t LDS_MAX = 160 * 1024;
+// whether 16 lines fit (n up to about 1270; longer lines keep k_r2r_dense)
+bool mfma_fits(int kind, int n) { return mfma_lds(mfma_ld(mfma_split(kind, n)), 16) <= LDS_MAX; }
+
+std::vector<double> mfma_fragments(int kind, int n) {
+  const MSplit m = mfma_split(kind, n);
+  const int nt = (m.rows + 15) / 16, kb[2] = {(m.ks + 3) / 4, (m.ka + 3) / 4};
+  std::vector<double> f((size_t)nt * 64 * (kb[0] + kb[1]), 0.0);
+  for (int part = 0; part < 2; part++) {
+    const int nr = part == 0 ? m.rows : (m.mode == 1 ? m.na : m.rows), nc = part == 0 ? m.ks : m.ka;
+    auto side = [&](int q) { return m.hc ? (part == 0 ? q : n - 1 - q) : 2 * q + part; };  // transformed side
+    double *out = f.data() + (part == 0 ? 0 : (size_t)nt * kb[0] * 64);
+    for (int r = 0; r < nr; r++)
+      for (int c = 0; c < nc; c++) {
+        // the antisymmetric part has nothing on a sample that is its own mirror
+        const int sample = m.mode == 1 ? c : r;
+        if (m.mode != 0 && part == 1 && sample == (m.hc ? (n - sample) % n : n - 1 - sample)) continue;
+        const double v = m.mode == 0   ? r2r_coef(kind, n, r, c)
+                         : m.mode == 1 ? r2r_coef(kind, n, side(r), c)
+                                       : r2r_coef(kind, n, r, side(c));
+        out[(((size_t)(r / 16) * kb[part] + c / 4) * 4 + c % 4) * 16 + r % 16] = v;
+      }
+  }
+  return f;
+}
+
+void launch_mfma(hipStream_t s, const Args &b, int kind, double scale, const double *frag) {
+  const MSplit m = mfma_split(kind, b.n);
+  MArgs a;
+  a.in = b.in; a.out = b.out;
+  a.ies = b.ies; a.is1 = b.is1; a.is2 = b.is2; a.oes = b.oes; a.os1 = b.os1; a.os2 = b.os2;
+  a.scale = scale;
+  a.n = b.n; a.nb1 = b.nb1; a.nlines = b.nlines;
+  a.half = m.half; a.rows = m.rows; a.ks = m.ks; a.ka = m.ka; a.na = m.na; a.hc = m.hc;
+  a.ld = mfma_ld(m);
+  a.ntile = (m.rows + 15) / 16;
+  a.fs = frag;
+  a.fa = frag + (size_t)a.ntile * ((m.ks + 3) / 4) * 64;
+  // a wavefront per tile of rows up to eight; short lines get more line
+  // groups per workgroup instead (at least four wavefronts)
+  a.tw = std::min(a.ntile, 8);
+  a.lg = a.tw == 1 ? 4 : (a.tw == 2 ? 2 : 1);
+  // two tiles of lines per wavefront (each matrix load used twice) where two
+  // workgroups still fit a CU's LDS and the launch has two workgroups per CU
+  const int ntl = mfma_lds(a.ld, 32 * a.lg) <= LDS_MAX / 2 && a.nlines >= 32 * a.lg * 512 ? 2 : 1;
+  while (a.lg > 1 && mfma_lds(a.ld, 16 * ntl * a.lg) > LDS_MAX) a.lg >>= 1;
+  const int L = 16 * ntl * a.lg;
+  const dim3 grid((unsigned)((a.nlines + L - 1) / L)), blk(64 * a.tw * a.lg);
+  const size_t lds = mfma_lds(a.ld, L);
+  const bool sw = a.oes == 1;
+#define SNAC_MF(M, W, T) hipLaunchKernelGGL((k_r2r_mfma<M, W, T>), grid, blk, lds, s, a)
+#define SNAC_MFM(M)                                                                  \
+  do {                                                                               \
+    if (sw) { if (ntl == 2) SNAC_MF(M, true, 2); else SNAC_MF(M, true, 1); }         \
+    else { if (ntl == 2) SNAC_MF(M, false, 2); else SNAC_MF(M, false, 1); }          \
+  } while (0)
+  if (m.mode == 0) SNAC_MFM(0);
+  else if (m.mode == 1) SNAC_MFM(1);
+  else SNAC_MFM(2);
+#undef SNAC_MFM
+#undef SNAC_MF
+}
+
 std::mutex g_mu;
 std::map<std::pair<int, int>, std::pair<R2RPlan, double *>> g_plans;
 
@@ -718,25 +960,32 @@ bool fft_kind(int kind) {
 
 }  // namespace
 
-double r2r_coef(int kind, int n, int k, int j) {
-  const double pi = std::acos(-1.0);
+namespace {
+// cos and sin of pi p / q, the angle reduced in integers first: p reaches n^2,
+// and rounding the full-size angle would cost n ulps of the coefficient
+double cos_pi(long p, long q) { return std::cos(std::acos(-1.0) * (double)(p % (2 * q)) / (double)q); }
+double sin_pi(long p, long q) { return std::sin(std::acos(-1.0) * (double)(p % (2 * q)) / (double)q); }
+}  // namespace
+
+double r2r_coef(int kind, int n_, int k_, int j_) {
+  const long n = n_, k = k_, j = j_;
   switch (kind) {
   case K_R2HC:
-    if (k <= n / 2) return std::cos(2.0 * pi * (double)j * k / n);
-    return -std::sin(2.0 * pi * (double)j * (n - k) / n);
+    if (k <= n / 2) return cos_pi(2 * j * k, n);
+    return -sin_pi(2 * j * (n - k), n);
   case K_HC2R:
     if (j == 0) return 1.0;
     if (n % 2 == 0 && j == n / 2) return (k % 2) ? -1.0 : 1.0;
-    if (j < (n + 1) / 2) return 2.0 * std::cos(2.0 * pi * (double)j * k / n);
-    return -2.0 * std::sin(2.0 * pi * (double)(n - j) * k / n);
-  case K_REDFT10: return 2.0 * std::cos(pi * (j + 0.5) * k / n);
-  case K_REDFT01: return j == 0 ? 1.0 : 2.0 * std::cos(pi * j * (k + 0.5) / n);
-  case K_RODFT10: return 2.0 * std::sin(pi * (j + 0.5) * (k + 1) / n);
-  case K_RODFT01: return j == n - 1 ? ((k % 2) ? -1.0 : 1.0) : 2.0 * std::sin(pi * (j + 1) * (k + 0.5) / n);
-  case K_REDFT11: return 2.0 * std::cos(pi * (j + 0.5) * (k + 0.5) / n);
-  case K_RODFT11: return 2.0 * std::sin(pi * (j + 0.5) * (k + 0.5) / n);
+    if (j < (n + 1) / 2) return 2.0 * cos_pi(2 * j * k, n);
+    return -2.0 * sin_pi(2 * (n - j) * k, n);
+  case K_REDFT10: return 2.0 * cos_pi((2 * j + 1) * k, 2 * n);
+  case K_REDFT01: return j == 0 ? 1.0 : 2.0 * cos_pi(j * (2 * k + 1), 2 * n);
+  case K_RODFT10: return 2.0 * sin_pi((2 * j + 1) * (k + 1), 2 * n);
+  case K_RODFT01: return j == n - 1 ? ((k % 2) ? -1.0 : 1.0) : 2.0 * sin_pi((j + 1) * (2 * k + 1), 2 * n);
+  case K_REDFT11: return 2.0 * cos_pi((2 * j + 1) * (2 * k + 1), 4 * n);
+  case K_RODFT11: return 2.0 * sin_pi((2 * j + 1) * (2 * k + 1), 4 * n);
   // DST-I: the transform of a staggered Dirichlet-Dirichlet axis (fft.f90:130-133)
-  case K_RODFT00: return 2.0 * std::sin(pi * (j + 1) * (k + 1) / (n + 1));
+  case K_RODFT00: return 2.0 * sin_pi((j + 1) * (k + 1), n + 1);
   default: throw std::runtime_error("unsupported r2r kind " + std::to_string(kind));
   }
 }
@@ -770,9 +1019,15 @@ R2RPlan r2r_plan(int kind, int n) {
     }
   } else {
     if (n > 2048) throw std::runtime_error("r2r: length " + std::to_string(n) + " needs the FFT path (power of two)");
-    h.resize((size_t)n * n);
-    for (int k = 0; k < n; k++)
-      for (int j = 0; j < n; j++) h[(size_t)k * n + j] = r2r_coef(kind, n, k, j);
+    (void)r2r_coef(kind, n, 0, 0);  // refuses unknown kinds
+    pl.mfma = mfma_fits(kind, n);
+    if (pl.mfma) {
+      h = mfma_fragments(kind, n);
+    } else {
+      h.resize((size_t)n * n);
+      for (int k = 0; k < n; k++)
+        for (int j = 0; j < n; j++) h[(size_t)k * n + j] = r2r_coef(kind, n, k, j);
+    }
   }
   double *d = nullptr;
   SNAC_HIP(hipMalloc(&d, h.size() * sizeof(double)));
@@ -817,6 +1072,8 @@ void launch_r2r(hipStream_t s, const R2RPlan &pl, const double *in, long ies, lo
     dim3 grid((unsigned)((a.nlines + L - 1) / L));
     size_t lds = (size_t)L * pl.n * sizeof(double2);
     launch_fft_kind(pl.kind, pl.n, ls, grid, lds, s, a);
+  } else if (pl.mfma) {
+    launch_mfma(s, a, pl.kind, scale, pl.tab);
   } else {
     int L = std::max(1, std::min(2 * LDS_COMPLEX / pl.n, a.nlines));
     a.L = L;
