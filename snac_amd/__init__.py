@@ -435,7 +435,8 @@ class Context:
         workgroup over several modes sharing LDS-staged coefficients (FFT
         path), 3 and 4 as 2 with 16 and 8 lanes per line (longer row chunks;
         the same systems in another elimination order); a negative value
-        (the default) restores each level's fastest, timed at set-up.  0..2
+        (the default) restores each level's fastest, timed at set-up (FP64 levels with few kinds of columns: their
+        precomputed line factors, reported as 5).  0..2
         compute the same values."""
         _check(lib.snac_set_kernel_variant(self.h, 4, int(v)), "set_kernel_variant")
 

@@ -171,7 +171,9 @@ struct R2RPlan {
                            // 7 (R2HC/HC2R): wavefront-local passes, factors swapped
   const double *tab = nullptr;  // device twiddles (fft), matrix fragments (mfma) or dense matrix
 };
-R2RPlan r2r_plan(int kind, int n);  // cached per (kind, n); throws if unsupported
+// cached per (kind, n, rowwise); throws if unsupported.  rowwise: a dense
+// product one output per thread even where the matrix cores could take it
+R2RPlan r2r_plan(int kind, int n, bool rowwise = false);
 int r2r_tile_choices(const R2RPlan &pl);  // number of tile choices of the plan's kernel
 void launch_r2r(hipStream_t s, const R2RPlan &pl, const double *in, long ies, long is1, long is2,
                 double *out, long oes, long os1, long os2, int nb1, int nb2, double scale);

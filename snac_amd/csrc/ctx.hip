@@ -495,6 +495,8 @@ void finish_mg_plan(snac_ctx *c, MGPlan &P) {
   // staggered along a bounded FFT axis)
   P.fwd = r2r_plan(P.kind_fwd, P.ng);
   P.bwd = r2r_plan(P.kind_bwd, P.ng);
+  P.fwd_row = r2r_plan(P.kind_fwd, P.ng, true);
+  P.bwd_row = r2r_plan(P.kind_bwd, P.ng, true);
   if (P.comp >= 0) {
     plan_mg(c);
     if (c->mg.ok && c->mg.ph) {
@@ -774,7 +776,7 @@ void mg_stage_in(snac_ctx *c, MGPlan &P) {
       const double *in = D.pp + 1 + D.g.sx + D.g.sx * D.g.sy;
       long off = 0;
       for (int q = 0; q < 3; q++) off += (long)(B.lo_g[q] - P.gmin[q]) * pst[q];
-      launch_r2r(c->stream, P.fwd, in, gstride(D, a), gstride(D, b1), gstride(D, b2), P.ph + off, pst[a], pst[b1],
+      launch_r2r(c->stream, c->prec == SNAC_PREC_FP64 ? P.fwd : P.fwd_row, in, gstride(D, a), gstride(D, b1), gstride(D, b2), P.ph + off, pst[a], pst[b1],
                  pst[b2], bext(D, b1), bext(D, b2), 1.0);
     }
     mg_copy3(c->stream, P.ph, pst[P.ax_m], pst[P.ax_a], pst[P.ax_s], P.r, na * ns, ns, 1, P.ng, (int)na,
@@ -806,7 +808,7 @@ void mg_stage_out(snac_ctx *c, MGPlan &P) {
       double *out = D.pp + 1 + D.g.sx + D.g.sx * D.g.sy;
       long off = 0;
       for (int q = 0; q < 3; q++) off += (long)(B.lo_g[q] - P.gmin[q]) * pst[q];
-      launch_r2r(c->stream, P.bwd, P.ph + off, pst[a], pst[b1], pst[b2], out, gstride(D, a), gstride(D, b1),
+      launch_r2r(c->stream, c->prec == SNAC_PREC_FP64 ? P.bwd : P.bwd_row, P.ph + off, pst[a], pst[b1], pst[b2], out, gstride(D, a), gstride(D, b1),
                  gstride(D, b2), bext(D, b1), bext(D, b2), P.norm);
     }
   } else {

@@ -4,36 +4,12 @@
 // with cross-lane shuffles), fused residual + restriction, prolongation,
 // operator application, per-group dot products with wavefront reductions and
 // the CG vector updates.
-#include "mg.hpp"
+#include "mg_device.hpp"
 #include <algorithm>
 #include <type_traits>
 
 namespace snac {
 namespace {
-
-template <typename T>
-__device__ __forceinline__ long vidx(const MGLevT<T> &L, int m, int a, int s) { return ((long)m * L.na + a) * L.ns + s; }
-template <typename T>
-__device__ __forceinline__ long cidx(const MGLevT<T> &L, int m, int a, int s) { return m * L.qm + (long)a * L.ns + s; }
-
-// sum of the couplings to the neighbouring lines (a and m directions) times x
-template <typename T>
-__device__ __forceinline__ T nb_sum(const MGLevT<T> &L, const T *__restrict__ x, int m, int a, long e, long q) {
-  T r = 0;
-  const long sa = L.ns;
-  if (a < L.na - 1) r += L.ca[q] * x[e + sa];
-  else if (L.per_a) r += L.ca[q] * x[e - (long)(L.na - 1) * sa];
-  if (a > 0) r += L.ca[q - sa] * x[e - sa];
-  else if (L.per_a) r += L.ca[q + (long)(L.na - 1) * sa] * x[e + (long)(L.na - 1) * sa];
-  if (L.coupled) {
-    const long sm = (long)L.na * L.ns;
-    if (m < L.nm - 1) r += L.cm[q] * x[e + sm];
-    else if (L.per_m) r += L.cm[q] * x[e - (long)(L.nm - 1) * sm];
-    if (m > 0) r += L.cm[q - L.qm] * x[e - sm];
-    else if (L.per_m) r += L.cm[q + (long)(L.nm - 1) * L.qm] * x[e + (long)(L.nm - 1) * sm];
-  }
-  return r;
-}
 
 // nb_sum of an FFT-path level (no m couplings) whose neighbour lines still
 // lack the prolongation: each neighbour reads x + xc of its coarse cell
@@ -56,15 +32,6 @@ __device__ __forceinline__ T nb_sum_pro(const MGLevT<T> &L, const T *__restrict_
   if (a > 0) r += L.ca[q - sa] * v(a - 1, e - sa, q - sa);
   else if (L.per_a) r += L.ca[q + w] * v(L.na - 1, e + w, q + w);
   return r;
-}
-
-template <typename T>
-__device__ __forceinline__ T mx_at(const MGLevT<T> &L, T lm, const T *__restrict__ x, int m, int a, int s) {
-  const long e = vidx(L, m, a, s), q = cidx(L, m, a, s);
-  T y = (L.dg[q] - lm * L.w[q]) * x[e];
-  if (s > 0) y -= L.cs[q - 1] * x[e - 1];
-  if (s < L.ns - 1) y -= L.cs[q] * x[e + 1];
-  return y - nb_sum(L, x, m, a, e, q);
 }
 
 template <typename T>
@@ -114,29 +81,6 @@ __device__ __forceinline__ Row<T> fetch(const Row<T> &r, int src, bool valid) {
   o.de = shfl(r.de, src);
   if (!valid) { o.al = 0; o.be = 1; o.ga = 0; o.de = 0; }
   return o;
-}
-
-// Reciprocals for the relaxation's eliminations without the IEEE division
-// sequence: the hardware estimate refined by Newton steps (two for FP64,
-// one for FP32), within a few ulp of the correctly rounded quotient.  The
-// relaxation only preconditions a CG that the FP64 residual judges.
-__device__ __forceinline__ double frcp(double x) {
-  double r = __builtin_amdgcn_rcp(x);
-  double e = __builtin_fma(-x, r, 1.0);
-  r = __builtin_fma(r, e, r);
-  e = __builtin_fma(-x, r, 1.0);
-  return __builtin_fma(r, e, r);
-}
-__device__ __forceinline__ float frcp(float x) {
-  float r = __builtin_amdgcn_rcpf(x);
-  float e = __builtin_fmaf(-x, r, 1.0f);
-  return __builtin_fmaf(r, e, r);
-}
-// a / b, or a times the refined reciprocal of b (FR)
-template <bool FR, typename T>
-__device__ __forceinline__ T dv(T a, T b) {
-  if constexpr (FR) return a * frcp(b);
-  else return a / b;
 }
 
 // PCR elimination of row r against its neighbours lo (index i-d) and hi (i+d)
@@ -1855,6 +1799,11 @@ void mg_set_shift(MGPlan &P, hipStream_t st, double shift) {
   hipLaunchKernelGGL(k_shift_lam, dim3((P.ng + 255) / 256), dim3(256), 0, st, P.ng, P.lam_base, shift, P.lam64,
                      P.lam32);
   SNAC_HIP(hipGetLastError());
+  // the tables of the levels the solves will use: the finest only where the
+  // V-cycle stops there (a fused coarse end that starts at the finest level runs in full)
+  const bool finest = P.smooth_only && P.h64.tail0 != 0;
+  if (P.prec == 0) mg_factor(st, P.h64, P.ng, finest);
+  else mg_factor(st, P.h32, P.ng, finest);
 }
 
 // r.r per group (k_dot's element order and sums, so the same values) with

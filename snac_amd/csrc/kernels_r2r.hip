@@ -714,6 +714,11 @@ __global__ __launch_bounds__(512) void k_r2r_mfma(MArgs a) {
   }
 }
 
+// The dense product one output per thread: lengths past the matrix-core
+// form's LDS, and the mixed-precision mode's transforms.  There FP32
+// right-hand sides turn any change of rounding, however small, into
+// differences of about 2e-9 of the velocities within a few substages, so that
+// mode keeps its operations and their order.
 __global__ __launch_bounds__(NT) void k_r2r_dense(Args a) {
   extern __shared__ double2 S[];
   double *R = reinterpret_cast<double *>(S);
@@ -891,6 +896,34 @@ constexpr size_t LDS_MAX = 160 * 1024;
 // whether 16 lines fit (n up to about 1270; longer lines keep k_r2r_dense)
 bool mfma_fits(int kind, int n) { return mfma_lds(mfma_ld(mfma_split(kind, n)), 16) <= LDS_MAX; }
 
+// cos and sin of pi p / q, the angle reduced in integers first: p reaches n^2,
+// and rounding the full-size angle would cost n ulps of the coefficient
+double cos_pi(long p, long q) { return std::cos(std::acos(-1.0) * (double)(p % (2 * q)) / (double)q); }
+double sin_pi(long p, long q) { return std::sin(std::acos(-1.0) * (double)(p % (2 * q)) / (double)q); }
+
+double reduced_coef(int kind, int n_, int k_, int j_) {
+  const long n = n_, k = k_, j = j_;
+  switch (kind) {
+  case K_R2HC:
+    if (k <= n / 2) return cos_pi(2 * j * k, n);
+    return -sin_pi(2 * j * (n - k), n);
+  case K_HC2R:
+    if (j == 0) return 1.0;
+    if (n % 2 == 0 && j == n / 2) return (k % 2) ? -1.0 : 1.0;
+    if (j < (n + 1) / 2) return 2.0 * cos_pi(2 * j * k, n);
+    return -2.0 * sin_pi(2 * (n - j) * k, n);
+  case K_REDFT10: return 2.0 * cos_pi((2 * j + 1) * k, 2 * n);
+  case K_REDFT01: return j == 0 ? 1.0 : 2.0 * cos_pi(j * (2 * k + 1), 2 * n);
+  case K_RODFT10: return 2.0 * sin_pi((2 * j + 1) * (k + 1), 2 * n);
+  case K_RODFT01: return j == n - 1 ? ((k % 2) ? -1.0 : 1.0) : 2.0 * sin_pi((j + 1) * (2 * k + 1), 2 * n);
+  case K_REDFT11: return 2.0 * cos_pi((2 * j + 1) * (2 * k + 1), 4 * n);
+  case K_RODFT11: return 2.0 * sin_pi((2 * j + 1) * (2 * k + 1), 4 * n);
+  // DST-I: the transform of a staggered Dirichlet-Dirichlet axis (fft.f90:130-133)
+  case K_RODFT00: return 2.0 * sin_pi((j + 1) * (k + 1), n + 1);
+  default: throw std::runtime_error("unsupported r2r kind " + std::to_string(kind));
+  }
+}
+
 std::vector<double> mfma_fragments(int kind, int n) {
   const MSplit m = mfma_split(kind, n);
   const int nt = (m.rows + 15) / 16, kb[2] = {(m.ks + 3) / 4, (m.ka + 3) / 4};
@@ -904,9 +937,9 @@ std::vector<double> mfma_fragments(int kind, int n) {
         // the antisymmetric part has nothing on a sample that is its own mirror
         const int sample = m.mode == 1 ? c : r;
         if (m.mode != 0 && part == 1 && sample == (m.hc ? (n - sample) % n : n - 1 - sample)) continue;
-        const double v = m.mode == 0   ? r2r_coef(kind, n, r, c)
-                         : m.mode == 1 ? r2r_coef(kind, n, side(r), c)
-                                       : r2r_coef(kind, n, r, side(c));
+        const double v = m.mode == 0   ? reduced_coef(kind, n, r, c)
+                         : m.mode == 1 ? reduced_coef(kind, n, side(r), c)
+                                       : reduced_coef(kind, n, r, side(c));
         out[(((size_t)(r / 16) * kb[part] + c / 4) * 4 + c % 4) * 16 + r % 16] = v;
       }
   }
@@ -960,32 +993,25 @@ bool fft_kind(int kind) {
 
 }  // namespace
 
-namespace {
-// cos and sin of pi p / q, the angle reduced in integers first: p reaches n^2,
-// and rounding the full-size angle would cost n ulps of the coefficient
-double cos_pi(long p, long q) { return std::cos(std::acos(-1.0) * (double)(p % (2 * q)) / (double)q); }
-double sin_pi(long p, long q) { return std::sin(std::acos(-1.0) * (double)(p % (2 * q)) / (double)q); }
-}  // namespace
-
-double r2r_coef(int kind, int n_, int k_, int j_) {
-  const long n = n_, k = k_, j = j_;
+double r2r_coef(int kind, int n, int k, int j) {
+  const double pi = std::acos(-1.0);
   switch (kind) {
   case K_R2HC:
-    if (k <= n / 2) return cos_pi(2 * j * k, n);
-    return -sin_pi(2 * j * (n - k), n);
+    if (k <= n / 2) return std::cos(2.0 * pi * (double)j * k / n);
+    return -std::sin(2.0 * pi * (double)j * (n - k) / n);
   case K_HC2R:
     if (j == 0) return 1.0;
     if (n % 2 == 0 && j == n / 2) return (k % 2) ? -1.0 : 1.0;
-    if (j < (n + 1) / 2) return 2.0 * cos_pi(2 * j * k, n);
-    return -2.0 * sin_pi(2 * (n - j) * k, n);
-  case K_REDFT10: return 2.0 * cos_pi((2 * j + 1) * k, 2 * n);
-  case K_REDFT01: return j == 0 ? 1.0 : 2.0 * cos_pi(j * (2 * k + 1), 2 * n);
-  case K_RODFT10: return 2.0 * sin_pi((2 * j + 1) * (k + 1), 2 * n);
-  case K_RODFT01: return j == n - 1 ? ((k % 2) ? -1.0 : 1.0) : 2.0 * sin_pi((j + 1) * (2 * k + 1), 2 * n);
-  case K_REDFT11: return 2.0 * cos_pi((2 * j + 1) * (2 * k + 1), 4 * n);
-  case K_RODFT11: return 2.0 * sin_pi((2 * j + 1) * (2 * k + 1), 4 * n);
+    if (j < (n + 1) / 2) return 2.0 * std::cos(2.0 * pi * (double)j * k / n);
+    return -2.0 * std::sin(2.0 * pi * (double)(n - j) * k / n);
+  case K_REDFT10: return 2.0 * std::cos(pi * (j + 0.5) * k / n);
+  case K_REDFT01: return j == 0 ? 1.0 : 2.0 * std::cos(pi * j * (k + 0.5) / n);
+  case K_RODFT10: return 2.0 * std::sin(pi * (j + 0.5) * (k + 1) / n);
+  case K_RODFT01: return j == n - 1 ? ((k % 2) ? -1.0 : 1.0) : 2.0 * std::sin(pi * (j + 1) * (k + 0.5) / n);
+  case K_REDFT11: return 2.0 * std::cos(pi * (j + 0.5) * (k + 0.5) / n);
+  case K_RODFT11: return 2.0 * std::sin(pi * (j + 0.5) * (k + 0.5) / n);
   // DST-I: the transform of a staggered Dirichlet-Dirichlet axis (fft.f90:130-133)
-  case K_RODFT00: return 2.0 * sin_pi((j + 1) * (k + 1), n + 1);
+  case K_RODFT00: return 2.0 * std::sin(pi * (j + 1) * (k + 1) / (n + 1));
   default: throw std::runtime_error("unsupported r2r kind " + std::to_string(kind));
   }
 }
@@ -995,9 +1021,9 @@ int r2r_tile_choices(const R2RPlan &pl) {
   return (pl.kind == K_R2HC || pl.kind == K_HC2R) && pl.n >= 8 ? 8 : 3;
 }
 
-R2RPlan r2r_plan(int kind, int n) {
+R2RPlan r2r_plan(int kind, int n, bool rowwise) {
   std::lock_guard<std::mutex> lk(g_mu);
-  auto key = std::make_pair(kind, n);
+  auto key = std::make_pair(rowwise ? kind + 16 : kind, n);
   auto it = g_plans.find(key);
   if (it != g_plans.end()) return it->second.first;
   if (n < 1) throw std::runtime_error("r2r: invalid length");
@@ -1020,7 +1046,7 @@ R2RPlan r2r_plan(int kind, int n) {
   } else {
     if (n > 2048) throw std::runtime_error("r2r: length " + std::to_string(n) + " needs the FFT path (power of two)");
     (void)r2r_coef(kind, n, 0, 0);  // refuses unknown kinds
-    pl.mfma = mfma_fits(kind, n);
+    pl.mfma = !rowwise && mfma_fits(kind, n);
     if (pl.mfma) {
       h = mfma_fragments(kind, n);
     } else {

@@ -44,7 +44,7 @@ struct MGLevT {
   const unsigned char *act;
   int nch, base, extra; // a line of ns rows over nch lanes: base (+1 for the first `extra`) rows each
   int lpl;              // lanes per line segment (32 or 64; nch <= lpl)
-  int lvar;             // line relaxation kernel of this level (0..4, chosen by timing at set-up)
+  int lvar;             // line relaxation kernel of this level (0..4, chosen by timing at set-up; 5: factored lines)
   // FFT path: dg, w, cs, ca and act are the same at every position a
   // (uniform, periodic in a), so a pass can read them once per row s
   int auni;
@@ -56,12 +56,42 @@ struct MGLevT {
 };
 using MGLev = MGLevT<double>;
 
+// A level's factored lines (FFT path, kernels_mgline.hip).  Columns with the
+// same coefficients form a class; each (mode, class) has one table of the
+// constants of a line's partitioned elimination, [entry][lane].  Absent (tab
+// null) where a level has many classes or long lines.
+// FP64: coefficients equal to 1e-12 (a uniform axis' spacings differ by
+// rounding): the sweeps only precondition, so a class' representative stands
+// for its columns.  FP32: equal as floats, and the tables hold exactly what
+// the unfactored kernels compute, so that a factored solve has their bits.
+template <typename T>
+struct MGFacT {
+  const T *tab = nullptr;   // [mode][class][mg_fac_entries][lpl]
+  const T *cc = nullptr;    // [class][2 K][lpl]: couplings to the columns above and below, per lane and row
+  const int *cls = nullptr; // class of each column
+  const int *rep = nullptr; // a column of each class
+  const int *pin = nullptr; // coarsest level: the singular modes, whose row pin_s is the identity
+  int ncls = 0, lpl = 0, K = 0, nch = 0, base = 0, extra = 0, pin_s = -1;
+  // FP32: 1 / 2: the values of the kernels with refined reciprocals / IEEE
+  // quotients; 0: not in use
+  int mode = 0;
+};
+// values per lane: five per row after the first, the coupling of the first,
+// four per reduction step (log2(lpl) + 1 of them), two reciprocals
+constexpr int mg_fac_entries(int K, int lpl) { return 5 * (K - 1) + 1 + 4 * (lpl == 32 ? 6 : 7) + 2; }
+constexpr int MG_FAC_CLASSES = 16;               // columns differing in more ways are solved unfactored
+constexpr size_t MG_FAC_BYTES = size_t(1) << 29; // table bytes of one level at most
+// lanes, rows and chunks of the factored lines of ns rows; false: none
+template <typename T>
+bool mg_fac_shape(int ns, MGFacT<T> &F);
+
 // the coarse end of the hierarchy handled by one fused kernel (FFT path)
 constexpr int MG_TAIL_MAX = 12;
 template <typename T>
 struct MGTailT {
   int nl;                   // levels in the tail; the last one has na == 1
   MGLevT<T> lev[MG_TAIL_MAX];
+  MGFacT<T> fac[MG_TAIL_MAX];
   T *x[MG_TAIL_MAX], *b[MG_TAIL_MAX];
   // the LDS-resident form: one mode's x and b of level q at element offsets
   // ox[q] / ob[q] of the workgroup's LDS, lds_elems elements in all
@@ -75,6 +105,7 @@ struct MGTailT {
 template <typename T>
 struct MGHier {
   std::vector<MGLevT<T>> lev;
+  std::vector<MGFacT<T>> fac;  // per level
   const T *lam = nullptr;
   std::vector<T *> xl, bl;
   int tail0 = -1;           // first level handled by the fused tail kernel (-1: none)
@@ -135,6 +166,22 @@ bool mg_fast_rcp();
 template <typename T>
 void mg_restrict_residual(hipStream_t st, const MGLevT<T> &F, const MGLevT<T> &C, const T *lam_f, const T *x,
                           const T *b, T *bc, const int *done);
+// ---- factored lines (kernels_mgline.hip) ----
+// (re)computes the factor tables of a hierarchy's levels from its
+// coefficients and eigenvalues
+template <typename T>
+void mg_factor(hipStream_t st, const MGHier<T> &H, int nm, bool finest_only);
+// mg_line with a level's factors; xc0: the coarse correction that lines of
+// this sweep's own colour still lack (read only across the ends of an odd
+// periodic axis)
+template <typename T>
+void mg_line_fac(hipStream_t st, const MGLevT<T> &L, const MGFacT<T> &F, T *x, const T *b, int col, int zero_nb,
+                 const int *done, const T *xc, const T *xc0, int cna);
+// mg_tail with the levels' factors; false (nothing launched) where a level has none
+template <typename T>
+bool mg_tail_fac(hipStream_t st, const MGTailT<T> &t, int nm, const T *lam, const int *done);
+// the restricted residual after a two-colour pre-smoothing from zero (FP64)
+void mg_restrict_zebra(hipStream_t st, const MGLev &F, const MGLev &C, const double *x, double *bc, const int *done);
 // fine x += coarse x on the active fine cells
 template <typename T>
 void mg_prolong(hipStream_t st, const MGLevT<T> &F, const MGLevT<T> &C, const T *xc, T *xf, const int *done);
@@ -291,6 +338,7 @@ struct MGPlan {
   int kind_fwd = 0, kind_bwd = 0;
   double norm = 1.0;
   R2RPlan fwd, bwd;
+  R2RPlan fwd_row, bwd_row;  // the mixed and learned modes' (k_r2r_dense)
   double *ph = nullptr;
   std::vector<void *> owned;
   // optional timing marks around the finest level's colour sweeps that read

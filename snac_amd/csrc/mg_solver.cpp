@@ -60,6 +60,9 @@ struct HostLev {
   std::vector<double> bd[3];  // boundary terms of the diagonal from the s / a / m faces
   std::vector<unsigned char> act;
   long at(int m, int a, int s) const { return ((long)m * na + a) * ns + s; }
+  // the couplings of (a, s) to the columns above and below it (mode-independent levels)
+  double up(int a, int s) const { return a < na - 1 || per_a ? ca[at(0, a, s)] : 0.0; }
+  double down(int a, int s) const { return a > 0 ? ca[at(0, a - 1, s)] : (per_a ? ca[at(0, na - 1, s)] : 0.0); }
   void resize() {
     size_t n = (size_t)nmq * na * ns;
     dg.assign(n, 1.0); w.assign(n, 0.0); cs.assign(n, 0.0); ca.assign(n, 0.0); cm.assign(n, 0.0);
@@ -88,6 +91,38 @@ bool uniform_axis(const Case &cs, int a) {
       if (std::fabs(B.df[a][i] - h) > 1e-12 * h) return false;
       if (i <= B.n[a] && std::fabs(B.dc[a][i] - h) > 1e-12 * h) return false;
     }
+  return true;
+}
+
+// Groups a level's columns by their coefficients (FP64: equal to 1e-12 of the
+// larger; FP32: equal as floats); false when there are more than
+// MG_FAC_CLASSES kinds
+template <typename T>
+bool column_classes(const HostLev &h, std::vector<int> &cls, std::vector<int> &rep) {
+  auto near = [](double x, double y) {
+    if (sizeof(T) == 4) return (float)x == (float)y;
+    return std::fabs(x - y) <= 1e-12 * std::max(std::fabs(x), std::fabs(y));
+  };
+  cls.assign(h.na, 0);
+  rep.clear();
+  for (int a = 0; a < h.na; a++) {
+    size_t c = 0;
+    for (; c < rep.size(); c++) {
+      const int r = rep[c];
+      bool eq = true;
+      for (int s = 0; eq && s < h.ns; s++) {
+        const long q = h.at(0, a, s), p = h.at(0, r, s);
+        eq = near(h.dg[q], h.dg[p]) && near(h.w[q], h.w[p]) && near(h.cs[q], h.cs[p]) && near(h.up(a, s), h.up(r, s)) &&
+             near(h.down(a, s), h.down(r, s));
+      }
+      if (eq) break;
+    }
+    if (c == rep.size()) {
+      if ((int)c == MG_FAC_CLASSES) return false;
+      rep.push_back(a);
+    }
+    cls[a] = (int)c;
+  }
   return true;
 }
 
@@ -446,6 +481,8 @@ void mg_plan(MGPlan &P, const Case &cs, int device, int comp) {
   P.nlev = (int)H.size();
   if (device < 0) { P.ok = true; return; }
 
+  const int *dsing = dev_upload(P, sing);
+  P.singular = const_cast<int *>(dsing);
   // device arrays: the FP64 hierarchy and its FP32 twin (mixed precision)
   P.h64 = MGHier<double>();
   P.h32 = MGHier<float>();
@@ -532,6 +569,45 @@ void mg_plan(MGPlan &P, const Case &cs, int device, int comp) {
       P.h32.bl.push_back(dev_zeros<float>(P, n));
     }
   }
+  // factored lines (FFT path): the column classes of each level and their
+  // tables, filled by mg_factor
+  P.h64.fac.resize(H.size());
+  P.h32.fac.resize(H.size());
+  for (size_t l = 0; !coupled && l < H.size(); l++) {
+    const HostLev &h = H[l];
+    auto set = [&](auto &Hh, auto zero) {
+      using T = decltype(zero);
+      MGFacT<T> F;
+      std::vector<int> cls, rep;
+      if (!mg_fac_shape<T>(h.ns, F) || !column_classes<T>(h, cls, rep)) return;
+      // the unfactored kernels' bits need their split of the lines, and on an
+      // odd periodic axis their order of the two ends, which have one colour
+      if (sizeof(T) == 4 && (F.lpl != lpl || (h.per_a && h.na % 2 == 1 && h.na > 1))) return;
+      F.ncls = (int)rep.size();
+      const size_t n = (size_t)h.nm * F.ncls * mg_fac_entries(F.K, F.lpl) * F.lpl;
+      if (n * sizeof(T) > MG_FAC_BYTES) return;
+      F.cls = dev_upload(P, cls);
+      F.rep = dev_upload(P, rep);
+      std::vector<T> cc((size_t)F.ncls * 2 * F.K * F.lpl, T(0));
+      for (int c = 0; c < F.ncls; c++)
+        for (int lane = 0; lane < F.nch; lane++)
+          for (int j = 0; j < F.base + (lane < F.extra ? 1 : 0); j++) {
+            const int s2 = lane * F.base + std::min(lane, F.extra) + j, a = rep[c];
+            T *q = cc.data() + (size_t)c * 2 * F.K * F.lpl + lane;
+            q[(size_t)j * F.lpl] = (T)h.up(a, s2);
+            q[(size_t)(F.K + j) * F.lpl] = (T)h.down(a, s2);
+          }
+      F.cc = dev_upload(P, cc);
+      F.tab = dev_zeros<T>(P, n);
+      if (l + 1 == H.size()) {
+        F.pin_s = P.pin_s;
+        F.pin = dsing;
+      }
+      Hh.fac[l] = F;
+    };
+    set(P.h64, double());
+    set(P.h32, float());
+  }
   // fused tail: the levels with at most 32 columns (FFT path, modes independent)
   int tail0 = -1;
   const int nl = (int)H.size();
@@ -548,6 +624,7 @@ void mg_plan(MGPlan &P, const Case &cs, int device, int comp) {
     int off = 0;
     for (int q = 0; q < Hh.tail.nl; q++) {
       Hh.tail.lev[q] = Hh.lev[tail0 + q];
+      Hh.tail.fac[q] = Hh.fac[tail0 + q];
       Hh.tail.x[q] = Hh.xl[tail0 + q];
       Hh.tail.b[q] = Hh.bl[tail0 + q];
       const int n = (Hh.lev[tail0 + q].na * Hh.lev[tail0 + q].ns + 3) / 4 * 4;  // 16-byte aligned blocks
@@ -569,7 +646,6 @@ void mg_plan(MGPlan &P, const Case &cs, int device, int comp) {
   P.sums = dev_zeros<double>(P, 2 * P.ng);
   P.nact = dev_upload(P, nact);
   P.done = dev_zeros<int>(P, P.ng);
-  P.singular = dev_upload(P, sing);
   {
     std::vector<int> sl;
     for (int g = 0; g < P.ng; g++)
@@ -592,10 +668,22 @@ void mg_plan(MGPlan &P, const Case &cs, int device, int comp) {
   P.stall = dev_zeros<int>(P, 1);
   P.rr_prev = dev_zeros<double>(P, 2 * P.ng);
   SNAC_HIP(hipHostMalloc((void **)&P.stall_host, sizeof(int), hipHostMallocDefault));
+  // the Helmholtz plans' tables follow each solve's shift (mg_set_shift); the
+  // FP32 tables follow the choice of kernels (mg_tune_lines)
+  mg_factor(nullptr, P.h64, P.ng, false);
+  SNAC_HIP(hipStreamSynchronize(nullptr));
   P.ok = true;
 }
 
 namespace {
+
+// whether a level's factored lines are the ones to run: the FP32 ones stand
+// for kernels with refined reciprocals where those are on
+template <typename T>
+bool fac_in_use(const MGFacT<T> &F) {
+  if (!F.tab) return false;
+  return sizeof(T) == 8 || F.mode == 2 || (F.mode == 1 && mg_fast_rcp());
+}
 
 template <typename T>
 void vcycle(MGPlan &P, MGHier<T> &H, hipStream_t st, size_t l) {
@@ -604,7 +692,7 @@ void vcycle(MGPlan &P, MGHier<T> &H, hipStream_t st, size_t l) {
   const T *b = H.bl[l];
   if ((int)l == H.tail0) {  // the coarse end in one launch, one workgroup per mode
     if (P.mark_tail) P.mark_tail(true);
-    mg_tail(st, H.tail, P.ng, H.lam, P.pin_s, P.singular, P.done);
+    if (!mg_tail_fac(st, H.tail, P.ng, H.lam, P.done)) mg_tail(st, H.tail, P.ng, H.lam, P.pin_s, P.singular, P.done);
     if (P.mark_tail) P.mark_tail(false);
     return;
   }
@@ -617,19 +705,28 @@ void vcycle(MGPlan &P, MGHier<T> &H, hipStream_t st, size_t l) {
   for (int cm = 0; cm <= (two_m ? 1 : 0); cm++)
     for (int ca = 0; ca <= (two_a ? 1 : 0); ca++) { col[nc][0] = ca; col[nc][1] = cm; nc++; }
   const bool zero_first = nc > 2;
+  // factored lines, unless a line kernel is forced
+  const MGFacT<T> &F = H.fac[l];
+  const bool fac = fac_in_use(F) && !L.coupled && mg_line_variant() < 0;
   if (zero_first) mg_zero(st, (long)L.nm * L.na * L.ns, x);
   for (int k = 0; k < nc; k++) {
     const int znb = (!zero_first && k == 0) ? 1 : 0;
     const bool mk = l == 0 && znb == 0 && P.mark_line0;
     if (mk) P.mark_line0(true);
-    mg_line(st, L, H.lam, x, b, col[k][0], col[k][1], znb, -1, nullptr, P.done);
+    if (fac) mg_line_fac<T>(st, L, F, x, b, col[k][0], znb, P.done, nullptr, nullptr, 0);
+    else mg_line(st, L, H.lam, x, b, col[k][0], col[k][1], znb, -1, nullptr, P.done);
     if (mk) P.mark_line0(false);
   }
   // smooth_only: the finest level's symmetric zebra sweeps are the whole
   // preconditioner (no coarse correction)
   const bool coarse = !(l == 0 && P.smooth_only);
   if (coarse) {
-    mg_restrict_residual(st, L, H.lev[l + 1], H.lam, x, b, H.bl[l + 1], P.done);
+    if constexpr (sizeof(T) == 8) {
+      if (!L.coupled) mg_restrict_zebra(st, L, H.lev[l + 1], x, H.bl[l + 1], P.done);
+      else mg_restrict_residual(st, L, H.lev[l + 1], H.lam, x, b, H.bl[l + 1], P.done);
+    } else {
+      mg_restrict_residual(st, L, H.lev[l + 1], H.lam, x, b, H.bl[l + 1], P.done);
+    }
     vcycle(P, H, st, l + 1);
   }
   // two colours (FFT path): the first post-sweep relaxes colour 1 reading
@@ -643,8 +740,12 @@ void vcycle(MGPlan &P, MGHier<T> &H, hipStream_t st, size_t l) {
     const bool mk = l == 0 && P.mark_line0;
     if (mk) P.mark_line0(true);
     const bool pro = fuse && k == nc - 1;
-    mg_line(st, L, H.lam, x, b, col[k][0], col[k][1], 0, -1, nullptr, P.done, pro ? (const T *)H.xl[l + 1] : nullptr,
-            pro ? H.lev[l + 1].na : 0);
+    if (fac)
+      mg_line_fac<T>(st, L, F, x, b, col[k][0], 0, P.done, pro ? (const T *)H.xl[l + 1] : nullptr,
+                     coarse ? (const T *)H.xl[l + 1] : nullptr, coarse ? H.lev[l + 1].na : 0);
+    else
+      mg_line(st, L, H.lam, x, b, col[k][0], col[k][1], 0, -1, nullptr, P.done, pro ? (const T *)H.xl[l + 1] : nullptr,
+              pro ? H.lev[l + 1].na : 0);
     if (mk) P.mark_line0(false);
   }
 }
@@ -870,6 +971,7 @@ template <typename T>
 std::string hier_key(const MGHier<T> &H, int dev) {
   std::ostringstream k;
   k << "dev " << dev << " T" << sizeof(T) << " tail " << H.tail0;
+  for (const auto &F : H.fac) k << (F.tab ? " f" : " -");
   for (const auto &L : H.lev)
     k << " | nm " << L.nm << " na " << L.na << " ns " << L.ns << " qm " << L.qm << " c " << L.coupled << " p "
       << L.per_a << " lpl " << L.lpl;
@@ -898,7 +1000,8 @@ void tune_hier(MGPlan &P, MGHier<T> &H, hipStream_t st) {
   std::vector<int> lv(nl, -1);
   std::vector<int> tuned;  // the launched levels with a choice to make
   for (int l = 0; l < last; l++)
-    if (H.lev[l].na >= 2) tuned.push_back(l);
+    if (sizeof(T) == 8 && H.fac[l].tab) lv[l] = 5;  // factored lines: nothing to choose
+    else if (H.lev[l].na >= 2) tuned.push_back(l);
   if (!tuned.empty()) {
     hipEvent_t e0, e1;
     SNAC_HIP(hipEventCreate(&e0));
@@ -976,6 +1079,19 @@ void mg_tune_lines(MGPlan &P, hipStream_t st) {
   if (!P.ok || !P.x) return;
   tune_hier(P, P.h64, st);
   tune_hier(P, P.h32, st);
+  // the FP32 levels' factored lines take the place of the kernels chosen
+  // (those with 16 or 8 lanes per line split the lines differently and stay)
+  MGHier<float> &H = P.h32;
+  for (size_t l = 0; l < H.fac.size(); l++) {
+    MGFacT<float> &F = H.fac[l];
+    const int lv = H.lev[l].lvar < 0 ? 2 : H.lev[l].lvar;
+    if (!F.tab) continue;
+    if (H.tail0 >= 0 && (int)l >= H.tail0) F.mode = 2;
+    else if (lv <= 2) F.mode = lv == 2 && mg_line_variant_runs(H.lev[l], 2) ? 1 : 2;
+    if (H.tail0 >= 0 && (int)l >= H.tail0) H.tail.fac[l - H.tail0] = F;
+  }
+  mg_factor(st, H, P.ng, false);
+  SNAC_HIP(hipStreamSynchronize(st));
 }
 
 }  // namespace snac
