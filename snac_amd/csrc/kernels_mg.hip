@@ -773,6 +773,27 @@ __device__ __forceinline__ double wave_sum(double v) {
   return v;
 }
 
+// Group g's two sums from its chunks' partial sums, in the same order in
+// whichever kernel needs them: the CG passes reduce the partials of the pass
+// before them themselves (nchunk values, cache hits) instead of waiting for a
+// launch that does nothing else (4.3 us each, four per iteration).  Called by
+// every thread of the workgroup.
+__device__ __forceinline__ double2 part_sums(const double *__restrict__ part, int g, int nchunk) {
+  __shared__ double tot[2];
+  if (threadIdx.x < 64) {
+    double a = 0.0, b = 0.0;
+    for (int c = threadIdx.x; c < nchunk; c += 64) {
+      a += part[((long)g * nchunk + c) * 2];
+      b += part[((long)g * nchunk + c) * 2 + 1];
+    }
+    a = wave_sum(a);
+    b = wave_sum(b);
+    if (threadIdx.x == 0) { tot[0] = a; tot[1] = b; }
+  }
+  __syncthreads();
+  return make_double2(tot[0], tot[1]);
+}
+
 // blockIdx.y = group, blockIdx.x = chunk of the group's elements
 template <typename TY, typename TX2>
 __global__ __launch_bounds__(256) void k_dot(long gsize, const double *__restrict__ x, const TY *__restrict__ y,
@@ -963,11 +984,11 @@ __device__ __forceinline__ double mx_r(const MGLev &L, double lm, F &&f, int a, 
   return y - r;
 }
 
-__device__ __forceinline__ double cg_beta(int g, const double *__restrict__ rzn, const double *__restrict__ rzo,
+__device__ __forceinline__ double cg_beta(int g, double rzn, const double *__restrict__ rzo,
                                           const double *__restrict__ cross) {
   if (!rzo) return 0.0;
   const double den = rzo[g * 2];
-  const double num = rzn[g * 2] - (cross ? cross[g * 2 + 1] : 0.0);
+  const double num = rzn - (cross ? cross[g * 2 + 1] : 0.0);
   return den != 0.0 ? num / den : 0.0;
 }
 
@@ -981,7 +1002,8 @@ __device__ __forceinline__ double cg_beta(int g, const double *__restrict__ rzn,
 // group's ends forms its neighbour again.  Same values either way.
 template <typename TZ, typename TP, bool STAGE = false>
 __global__ __launch_bounds__(256) void k_dir_apply_dot(MGLev L, const double *__restrict__ lam, long gsize,
-                                                       const double *__restrict__ rzn, const double *__restrict__ rzo,
+                                                       const double *__restrict__ rzp, double *__restrict__ rzn,
+                                                       const double *__restrict__ rzo,
                                                        const double *__restrict__ cross, const TZ *__restrict__ z,
                                                        const TP *__restrict__ pp, TP *__restrict__ p,
                                                        double *__restrict__ part, int nchunk,
@@ -991,7 +1013,9 @@ __global__ __launch_bounds__(256) void k_dir_apply_dot(MGLev L, const double *__
   const int g = blockIdx.y;
   double s1 = 0.0;
   if (!done[g]) {
-    const double be = cg_beta(g, rzn, rzo, cross);
+    const double2 rz = part_sums(rzp, g, nchunk);
+    if (blockIdx.x == 0 && threadIdx.x == 0) { rzn[g * 2] = rz.x; rzn[g * 2 + 1] = rz.y; }  // for the passes after this one
+    const double be = cg_beta(g, rz.x, rzo, cross);
     auto pnew = [&](long e) -> double {
       if (be == 0.0) return (double)(TP)(double)z[e];
       return (double)(TP)((double)z[e] + be * (double)pp[e]);
@@ -1062,7 +1086,7 @@ __global__ __launch_bounds__(256) void k_dir_apply_dot(MGLev L, const double *__
 // sums, as k_dir_apply_dot.
 template <typename TZ, typename TP>
 __global__ __launch_bounds__(256) void k_dir_apply_dot_lds(MGLev L, const double *__restrict__ lam, long gsize,
-                                                           const double *__restrict__ rzn,
+                                                           const double *__restrict__ rzp, double *__restrict__ rzn,
                                                            const double *__restrict__ rzo,
                                                            const double *__restrict__ cross,
                                                            const TZ *__restrict__ z, const TP *__restrict__ pp,
@@ -1074,7 +1098,9 @@ __global__ __launch_bounds__(256) void k_dir_apply_dot_lds(MGLev L, const double
   const int g = blockIdx.y;
   double s1 = 0.0;
   if (!done[g]) {
-    const double be = cg_beta(g, rzn, rzo, cross);
+    const double2 rz = part_sums(rzp, g, nchunk);
+    if (blockIdx.x == 0 && threadIdx.x == 0) { rzn[g * 2] = rz.x; rzn[g * 2 + 1] = rz.y; }  // for the passes after this one
+    const double be = cg_beta(g, rz.x, rzo, cross);
     auto pn = [&](long e) -> TP {
       if (be == 0.0) return (TP)(double)z[e];
       return (TP)((double)z[e] + be * (double)pp[e]);
@@ -1132,7 +1158,7 @@ __global__ __launch_bounds__(256) void k_dir_apply_dot_lds(MGLev L, const double
 template <typename TP, bool STAGE = false>
 __global__ __launch_bounds__(256) void k_update_apply_dot(MGLev L, const double *__restrict__ lam, long gsize,
                                                           const double *__restrict__ rz,
-                                                          const double *__restrict__ pq, double *__restrict__ x,
+                                                          const double *__restrict__ pqp, double *__restrict__ x,
                                                           const TP *__restrict__ p, double *__restrict__ r,
                                                           float *__restrict__ rf, const float *__restrict__ zf,
                                                           double *__restrict__ part, int nchunk,
@@ -1142,7 +1168,7 @@ __global__ __launch_bounds__(256) void k_update_apply_dot(MGLev L, const double 
   const int g = blockIdx.y;
   double s1 = 0.0, s2 = 0.0;
   if (!done[g]) {
-    const double den = pq[g * 2];
+    const double den = part_sums(pqp, g, nchunk).x;
     // p.Mp > 0 for an SPD operator and p != 0; anything else (p = 0, or a
     // preconditioner output that is not usable) skips the step instead of
     // spreading an overflow or a NaN
@@ -1228,7 +1254,7 @@ __global__ __launch_bounds__(256) void k_update_apply_dot(MGLev L, const double 
 template <typename TP>
 __global__ __launch_bounds__(256) void k_update_apply_dot_lds(MGLev L, const double *__restrict__ lam, long gsize,
                                                               const double *__restrict__ rz,
-                                                              const double *__restrict__ pq, double *__restrict__ x,
+                                                              const double *__restrict__ pqp, double *__restrict__ x,
                                                               const TP *__restrict__ p, double *__restrict__ r,
                                                               float *__restrict__ rf, const float *__restrict__ zf,
                                                               double *__restrict__ part, int nchunk,
@@ -1239,7 +1265,7 @@ __global__ __launch_bounds__(256) void k_update_apply_dot_lds(MGLev L, const dou
   const int g = blockIdx.y;
   double s1 = 0.0, s2 = 0.0;
   if (!done[g]) {
-    const double den = pq[g * 2];
+    const double den = part_sums(pqp, g, nchunk).x;
     // as k_update_apply_dot: an unusable step length skips the step
     double al = den > 0.0 ? rz[g * 2] / den : 0.0;
     if (!(__builtin_fabs(al) < 1e300)) al = 0.0;
@@ -1365,38 +1391,141 @@ __global__ __launch_bounds__(256) void k_sub_mean(MGLev L, T *__restrict__ x, co
   x[idx] -= (T)(sums[g * 2 + 1] / nact[g]);
 }
 
-// one workgroup: updates the done flags, counts the groups left and (list)
-// writes them in increasing order, 256 groups per round (ballot + popcount
-// positions within a wavefront, wavefront totals through LDS)
-__global__ __launch_bounds__(256) void k_flags(int ng, const double *__restrict__ rr, const double *__restrict__ bb,
-                                               double tol2, int *__restrict__ done, int *__restrict__ left,
-                                               int *__restrict__ list, int it) {
-  __shared__ int wsum[4];
-  __shared__ int base;
-  if (threadIdx.x == 0) base = 0;
+// one workgroup: sums the groups' residual norms (part: the update pass's
+// partials, else rr holds them), updates the done flags, counts the groups
+// left and (list) writes them in increasing order, 1024 groups per round
+// (ballot + popcount positions within a wavefront, wavefront totals through
+// LDS).  Latency-bound: each wavefront has the loads of four groups in
+// flight, and the flags pass to the ballot through LDS.
+constexpr int FLAG_NT = 1024, FLAG_W = FLAG_NT / 64;
+__global__ __launch_bounds__(FLAG_NT) void k_flags(int ng, const double *__restrict__ part, int nchunk,
+                                                   double *__restrict__ rr, const double *__restrict__ bb, double tol2,
+                                                   int *__restrict__ done, int *__restrict__ left,
+                                                   int *__restrict__ list, int it) {
+  __shared__ int wsum[FLAG_W], live[FLAG_NT];
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-  for (int g0 = 0; g0 < ng; g0 += 256) {
-    const int g = g0 + threadIdx.x;
-    int act = 0;
-    if (g < ng) {
-      if (!done[g] && rr[g * 2] <= tol2 * bb[g * 2]) done[g] = 1;
-      act = !done[g];
+  int base = 0;
+  for (int g0 = 0; g0 < ng; g0 += FLAG_NT) {
+    const int n = min(ng - g0, FLAG_NT);
+    if (part) {
+      constexpr int U = 4;
+      for (int q0 = wv; q0 < n; q0 += FLAG_W * U) {
+        double a[U], b[U], lim[U];
+        int dn[U];
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+          const int q = q0 + u * FLAG_W;
+          const long g = g0 + min(q, n - 1);
+          a[u] = b[u] = 0.0;
+          dn[u] = done[g];
+          lim[u] = tol2 * bb[g * 2];
+          if (lane < nchunk) {
+            a[u] = part[(g * nchunk + lane) * 2];
+            b[u] = part[(g * nchunk + lane) * 2 + 1];
+          }
+        }
+        for (int c = lane + 64; c < nchunk; c += 64)
+#pragma unroll
+          for (int u = 0; u < U; u++) {
+            const long g = g0 + min(q0 + u * FLAG_W, n - 1);
+            a[u] += part[(g * nchunk + c) * 2];
+            b[u] += part[(g * nchunk + c) * 2 + 1];
+          }
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+          const int q = q0 + u * FLAG_W, g = g0 + q;
+          const double ta = wave_sum(a[u]), tb = wave_sum(b[u]);
+          if (lane != 0 || q >= n) continue;
+          // a group that is done keeps its values
+          if (!dn[u]) { rr[g * 2] = ta; rr[g * 2 + 1] = tb; }
+          const bool now = !dn[u] && ta <= lim[u];
+          if (now) done[g] = 1;
+          live[q] = !dn[u] && !now;
+        }
+      }
+    } else if ((int)threadIdx.x < n) {
+      const int g = g0 + threadIdx.x;
+      const bool was = done[g], now = !was && rr[g * 2] <= tol2 * bb[g * 2];
+      if (now) done[g] = 1;
+      live[threadIdx.x] = !was && !now;
     }
+    __syncthreads();
+    const int act = (int)threadIdx.x < n && live[threadIdx.x];
     const unsigned long long bal = __ballot(act);
     const int pre = __popcll(bal & ((1ull << lane) - 1ull));
     if (lane == 0) wsum[wv] = __popcll(bal);
     __syncthreads();
-    int off = base;
-    for (int k = 0; k < wv; k++) off += wsum[k];
-    const int tot = wsum[0] + wsum[1] + wsum[2] + wsum[3];
-    if (act && list) list[off + pre] = g;
-    __syncthreads();  // base and wsum read by every thread before they change
-    if (threadIdx.x == 0) base += tot;
+    int off = base, tot = 0;
+    for (int k = 0; k < FLAG_W; k++) {
+      if (k < wv) off += wsum[k];
+      tot += wsum[k];
+    }
+    if (act && list) list[off + pre] = g0 + threadIdx.x;
+    base += tot;
+    __syncthreads();  // live and wsum are read before the next round writes them
   }
-  __syncthreads();
   if (threadIdx.x == 0) {
     left[0] = base;
     if (base == 0 && left[1] == 0) left[1] = it + 1;
+  }
+}
+
+// Partial sums of x over the singular groups (glist, one per blockIdx.y):
+// the null-space component that k_dot_rz takes off
+template <typename T>
+__global__ __launch_bounds__(256) void k_null_part(long gsize, const T *__restrict__ x, const int *__restrict__ glist,
+                                                   double *__restrict__ part, int nchunk, const int *__restrict__ done) {
+  __shared__ double sh[4];
+  const int g = glist[blockIdx.y];
+  double s2 = 0.0;
+  if (!(done && done[g])) {
+    const long base = (long)g * gsize;
+    for (long i = (long)blockIdx.x * 256 + threadIdx.x; i < gsize; i += (long)nchunk * 256) s2 += (double)x[base + i];
+  }
+  s2 = wave_sum(s2);
+  if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = s2;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    part[((long)g * nchunk + blockIdx.x) * 2] = 0.0;
+    part[((long)g * nchunk + blockIdx.x) * 2 + 1] = sh[0] + sh[1] + sh[2] + sh[3];
+  }
+}
+
+// Partial sums of r.z per group, z of the singular groups (sing[g]) less its
+// mean over the active cells, which is stored back in the same pass.  Same
+// element order as k_dot.  HBM-bound: r and z read once.
+template <typename T>
+__global__ __launch_bounds__(256) void k_dot_rz(long gsize, const double *__restrict__ r, T *__restrict__ z,
+                                                double *__restrict__ part, int nchunk, const int *__restrict__ done,
+                                                const int *__restrict__ sing, const double *__restrict__ npart,
+                                                const double *__restrict__ nact,
+                                                const unsigned char *__restrict__ act) {
+  __shared__ double sh[4];
+  const int g = blockIdx.y;
+  double s1 = 0.0;
+  if (!(done && done[g])) {
+    const long base = (long)g * gsize;
+    if (sing && sing[g]) {
+      const T mean = (T)(part_sums(npart, g, nchunk).y / nact[g]);
+      for (long i = (long)blockIdx.x * 256 + threadIdx.x; i < gsize; i += (long)nchunk * 256) {
+        T v = z[base + i];
+        if (act[i]) {
+          v -= mean;
+          z[base + i] = v;
+        }
+        s1 += r[base + i] * (double)v;
+      }
+    } else {
+      for (long i = (long)blockIdx.x * 256 + threadIdx.x; i < gsize; i += (long)nchunk * 256)
+        s1 += r[base + i] * (double)z[base + i];
+    }
+  }
+  s1 = wave_sum(s1);
+  if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = s1;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    part[((long)g * nchunk + blockIdx.x) * 2] = sh[0] + sh[1] + sh[2] + sh[3];
+    part[((long)g * nchunk + blockIdx.x) * 2 + 1] = 0.0;
   }
 }
 
@@ -1733,64 +1862,75 @@ void mg_cg_update_dot(hipStream_t st, int ng, long gsize, const double *rz, cons
 }
 
 template <typename TZ, typename TP>
-void mg_dir_apply_dot(hipStream_t st, const MGLev &L, const double *lam, int ng, long gsize, const double *rzn,
-                      const double *rzo, const double *cross, const TZ *z, const TP *p_prev, TP *p, double *part,
-                      int nchunk, double *out, const int *done) {
+void mg_dir_apply_dot(hipStream_t st, const MGLev &L, const double *lam, int ng, long gsize, const double *rzp,
+                      double *rzn, const double *rzo, const double *cross, const TZ *z, const TP *p_prev, TP *p,
+                      double *part, int nchunk, const int *done) {
   // the LDS form where a level's coefficients do not depend on a, its rows
   // divide 256 and a chunk's lines with their two neighbours fit in 64 KB
   const long csz = ((gsize + nchunk - 1) / nchunk + 255) / 256 * 256;
   const size_t lds = L.ns > 0 ? (size_t)(csz / L.ns + 2) * L.ns * sizeof(TP) : 0;
   const size_t ldsg = (size_t)(csz + 2 * L.ns) * sizeof(TP);  // any 2D level: the chunk and a line on each side
   if (g_cg_lds && !L.coupled && L.auni && L.ns > 0 && 256 % L.ns == 0 && lds <= 64 * 1024)
-    hipLaunchKernelGGL((k_dir_apply_dot_lds<TZ, TP>), dim3(nchunk, ng), dim3(256), lds, st, L, lam, gsize, rzn, rzo,
+    hipLaunchKernelGGL((k_dir_apply_dot_lds<TZ, TP>), dim3(nchunk, ng), dim3(256), lds, st, L, lam, gsize, rzp, rzn, rzo,
                        cross, z, p_prev, p, part, nchunk, done);
   else if (g_cg_lds && !L.coupled && ldsg <= 64 * 1024)
-    hipLaunchKernelGGL((k_dir_apply_dot<TZ, TP, true>), dim3(nchunk, ng), dim3(256), ldsg, st, L, lam, gsize, rzn, rzo,
+    hipLaunchKernelGGL((k_dir_apply_dot<TZ, TP, true>), dim3(nchunk, ng), dim3(256), ldsg, st, L, lam, gsize, rzp, rzn, rzo,
                        cross, z, p_prev, p, part, nchunk, done);
   else
-    hipLaunchKernelGGL((k_dir_apply_dot<TZ, TP>), dim3(nchunk, ng), dim3(256), 0, st, L, lam, gsize, rzn, rzo, cross,
+    hipLaunchKernelGGL((k_dir_apply_dot<TZ, TP>), dim3(nchunk, ng), dim3(256), 0, st, L, lam, gsize, rzp, rzn, rzo, cross,
                        z, p_prev, p, part, nchunk, done);
-  SNAC_HIP(hipGetLastError());
-  hipLaunchKernelGGL(k_dot_final, dim3(ng), dim3(64), 0, st, part, nchunk, out, done, nullptr);
   SNAC_HIP(hipGetLastError());
 }
 
 template <typename TP>
 void mg_update_apply_dot(hipStream_t st, const MGLev &L, const double *lam, int ng, long gsize, const double *rz,
-                         const double *pq, double *x, const TP *p, double *r, float *rf, const float *zf,
-                         double *part, int nchunk, double *out, const int *done, bool first) {
+                         const double *pqp, double *x, const TP *p, double *r, float *rf, const float *zf,
+                         double *part, int nchunk, const int *done, bool first) {
   const long csz = ((gsize + nchunk - 1) / nchunk + 255) / 256 * 256;
   const size_t lds = L.ns > 0 ? (size_t)(csz / L.ns + 2) * L.ns * sizeof(TP) : 0;
   const size_t ldsg = (size_t)(csz + 2 * L.ns) * sizeof(TP);
   const int fi = first ? 1 : 0;
   if (g_cg_lds && !L.coupled && L.auni && L.ns > 0 && 256 % L.ns == 0 && lds <= 64 * 1024)
-    hipLaunchKernelGGL(k_update_apply_dot_lds<TP>, dim3(nchunk, ng), dim3(256), lds, st, L, lam, gsize, rz, pq, x, p,
+    hipLaunchKernelGGL(k_update_apply_dot_lds<TP>, dim3(nchunk, ng), dim3(256), lds, st, L, lam, gsize, rz, pqp, x, p,
                        r, rf, zf, part, nchunk, done, fi);
   else if (g_cg_lds && !L.coupled && ldsg <= 64 * 1024)
-    hipLaunchKernelGGL((k_update_apply_dot<TP, true>), dim3(nchunk, ng), dim3(256), ldsg, st, L, lam, gsize, rz, pq, x,
+    hipLaunchKernelGGL((k_update_apply_dot<TP, true>), dim3(nchunk, ng), dim3(256), ldsg, st, L, lam, gsize, rz, pqp, x,
                        p, r, rf, zf, part, nchunk, done, fi);
   else
-    hipLaunchKernelGGL(k_update_apply_dot<TP>, dim3(nchunk, ng), dim3(256), 0, st, L, lam, gsize, rz, pq, x, p, r, rf,
+    hipLaunchKernelGGL(k_update_apply_dot<TP>, dim3(nchunk, ng), dim3(256), 0, st, L, lam, gsize, rz, pqp, x, p, r, rf,
                        zf, part, nchunk, done, fi);
   SNAC_HIP(hipGetLastError());
-  hipLaunchKernelGGL(k_dot_final, dim3(ng), dim3(64), 0, st, part, nchunk, out, done, nullptr);
-  SNAC_HIP(hipGetLastError());
 }
-template void mg_dir_apply_dot<double, double>(hipStream_t, const MGLev &, const double *, int, long, const double *,
-                                               const double *, const double *, const double *, const double *,
-                                               double *, double *, int, double *, const int *);
-template void mg_dir_apply_dot<float, double>(hipStream_t, const MGLev &, const double *, int, long,
-                                              const double *, const double *, const double *, const float *,
-                                              const double *, double *, double *, int, double *, const int *);
-template void mg_dir_apply_dot<float, float>(hipStream_t, const MGLev &, const double *, int, long, const double *,
-                                             const double *, const double *, const float *, const float *, float *,
-                                             double *, int, double *, const int *);
+#define SNAC_INST(TZ, TP)                                                                                             \
+  template void mg_dir_apply_dot<TZ, TP>(hipStream_t, const MGLev &, const double *, int, long, const double *,       \
+                                         double *, const double *, const double *, const TZ *, const TP *, TP *,       \
+                                         double *, int, const int *);
+SNAC_INST(double, double)
+SNAC_INST(float, double)
+SNAC_INST(float, float)
+#undef SNAC_INST
 template void mg_update_apply_dot<double>(hipStream_t, const MGLev &, const double *, int, long, const double *,
                                           const double *, double *, const double *, double *, float *, const float *,
-                                          double *, int, double *, const int *, bool);
+                                          double *, int, const int *, bool);
 template void mg_update_apply_dot<float>(hipStream_t, const MGLev &, const double *, int, long, const double *,
                                          const double *, double *, const float *, double *, float *, const float *,
-                                         double *, int, double *, const int *, bool);
+                                         double *, int, const int *, bool);
+
+template <typename T>
+void mg_dot_rz(hipStream_t st, const MGLev &L, int ng, long gsize, const double *r, T *z, double *part, int nchunk,
+               const int *done, const int *sing, const int *sing_list, int n_sing, double *npart, const double *nact) {
+  if (n_sing > 0) {
+    hipLaunchKernelGGL(k_null_part<T>, dim3(nchunk, n_sing), dim3(256), 0, st, gsize, z, sing_list, npart, nchunk, done);
+    SNAC_HIP(hipGetLastError());
+  }
+  hipLaunchKernelGGL(k_dot_rz<T>, dim3(nchunk, ng), dim3(256), 0, st, gsize, r, z, part, nchunk, done,
+                     n_sing > 0 ? sing : nullptr, npart, nact, L.act);
+  SNAC_HIP(hipGetLastError());
+}
+template void mg_dot_rz<double>(hipStream_t, const MGLev &, int, long, const double *, double *, double *, int,
+                                const int *, const int *, const int *, int, double *, const double *);
+template void mg_dot_rz<float>(hipStream_t, const MGLev &, int, long, const double *, float *, double *, int,
+                               const int *, const int *, const int *, int, double *, const double *);
 
 void mg_set_shift(MGPlan &P, hipStream_t st, double shift) {
   if (P.comp < 0 || !P.lam_base) return;
@@ -1872,9 +2012,9 @@ void mg_sub_mean(hipStream_t st, const MGLev &L, T *x, const double *sums, const
   SNAC_HIP(hipGetLastError());
 }
 
-void mg_flags(hipStream_t st, int ng, const double *rr, const double *bb, double tol2, int *done, int *left,
-              int *list, int it) {
-  hipLaunchKernelGGL(k_flags, dim3(1), dim3(256), 0, st, ng, rr, bb, tol2, done, left, list, it);
+void mg_flags(hipStream_t st, int ng, const double *part, int nchunk, double *rr, const double *bb, double tol2,
+              int *done, int *left, int *list, int it) {
+  hipLaunchKernelGGL(k_flags, dim3(1), dim3(FLAG_NT), 0, st, ng, part, nchunk, rr, bb, tol2, done, left, list, it);
   SNAC_HIP(hipGetLastError());
 }
 

@@ -205,20 +205,28 @@ void mg_warm_residual(hipStream_t st, int ng, long gsize, const double *bb, doub
 void mg_cg_update_dot(hipStream_t st, int ng, long gsize, const double *rz, const double *pq, double *x,
                       const double *p, double *r, const double *q, float *rf, const float *zf, double *part,
                       int nchunk, double *out, const int *done);
+// the preconditioned residual z freed of its null-space component (the
+// singular groups' mean over their active cells, partial sums in npart), and
+// the partial sums of r.z per group
+template <typename T>
+void mg_dot_rz(hipStream_t st, const MGLev &L, int ng, long gsize, const double *r, T *z, double *part, int nchunk,
+               const int *done, const int *sing, const int *sing_list, int n_sing, double *npart, const double *nact);
 // the CG's direction update and operator in one pass: p = z + beta p_prev
-// (beta as mg_cg_dir; p stored as TP, p_prev and p distinct buffers) and
-// out[g*2] = p . (M p) per group
+// (beta as mg_cg_dir; p stored as TP, p_prev and p distinct buffers) and the
+// partial sums of p . (M p) per group.  rzp: mg_dot_rz's partials, whose sums
+// are stored in rzn as well
 template <typename TZ, typename TP>
-void mg_dir_apply_dot(hipStream_t st, const MGLev &L, const double *lam, int ng, long gsize, const double *rzn,
-                      const double *rzo, const double *cross, const TZ *z, const TP *p_prev, TP *p, double *part,
-                      int nchunk, double *out, const int *done);
-// mg_cg_update_dot with q = M p recomputed from p instead of read.  first:
-// the solve's first step from x = 0, x not read (x = alpha p) and set to 0
-// on the groups that are already done
+void mg_dir_apply_dot(hipStream_t st, const MGLev &L, const double *lam, int ng, long gsize, const double *rzp,
+                      double *rzn, const double *rzo, const double *cross, const TZ *z, const TP *p_prev, TP *p,
+                      double *part, int nchunk, const int *done);
+// mg_cg_update_dot with q = M p recomputed from p instead of read, p.q from
+// mg_dir_apply_dot's partials pqp, and its sums left as partials (mg_flags
+// adds them up).  first: the solve's first step from x = 0, x not read (x =
+// alpha p) and set to 0 on the groups that are already done
 template <typename TP>
 void mg_update_apply_dot(hipStream_t st, const MGLev &L, const double *lam, int ng, long gsize, const double *rz,
-                         const double *pq, double *x, const TP *p, double *r, float *rf, const float *zf,
-                         double *part, int nchunk, double *out, const int *done, bool first = false);
+                         const double *pqp, double *x, const TP *p, double *r, float *rf, const float *zf,
+                         double *part, int nchunk, const int *done, bool first = false);
 void mg_izero(hipStream_t st, long n, int *x);
 // dst = (float) src
 void mg_to_float(hipStream_t st, long n, const double *src, float *dst);
@@ -244,13 +252,14 @@ void mg_sub_mean(hipStream_t st, const MGLev &L, T *x, const double *sums, const
                  const double *nact,
                  const int *done);
 // done[g] |= r.r <= tol2 b.b; left[0] = the groups not done; list (when
-// given): those groups in increasing order.  it: the CG iterations done so
-// far; the first call that finds every group done sets left[1] = it + 1
-// (left[1] is cleared at the start of a solve), so a solve whose iterations
-// ran ahead without a host check (captured in a graph) still tells how many
-// it needed
-void mg_flags(hipStream_t st, int ng, const double *rr, const double *bb, double tol2, int *done, int *left,
-              int *list, int it);
+// given): those groups in increasing order.  part: the update pass's partial
+// sums, added up into rr (r.r and the cross term) of the groups not done;
+// null: rr holds the sums.  it: the CG iterations done so far; the first call
+// that finds every group done sets left[1] = it + 1 (left[1] is cleared at the
+// start of a solve), so a solve whose iterations ran ahead without a host
+// check (captured in a graph) still tells how many it needed
+void mg_flags(hipStream_t st, int ng, const double *part, int nchunk, double *rr, const double *bb, double tol2,
+              int *done, int *left, int *list, int it);
 // strided 3D copy (em x ea x es elements) with scaling; `tile` selects an
 // LDS transpose for src stride(a) == 1 -> dst stride(s) == 1 (1) or the
 // reverse (2); 0 = direct with lanes along s
@@ -312,7 +321,8 @@ struct MGPlan {
   // FP64 (p and q) or FP32 (mixed and learned modes)
   double *pd[2] = {nullptr, nullptr};
   float *pf[2] = {nullptr, nullptr};
-  double *part = nullptr, *bb = nullptr, *rr = nullptr, *pq = nullptr, *rz[2] = {nullptr, nullptr}, *sums = nullptr;
+  double *part = nullptr, *part_rz = nullptr, *part_pq = nullptr, *part_null = nullptr;  // per chunk and group
+  double *bb = nullptr, *rr = nullptr, *pq = nullptr, *rz[2] = {nullptr, nullptr}, *sums = nullptr;
   double *nact = nullptr;
   int *done = nullptr, *singular = nullptr, *left = nullptr, *left_host = nullptr;
   int *mlist = nullptr;  // FFT path: the groups not done, in order (left of them)

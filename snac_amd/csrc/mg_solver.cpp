@@ -638,6 +638,9 @@ void mg_plan(MGPlan &P, const Case &cs, int device, int comp) {
   set_tail(P.h32);
   P.nchunk = (int)std::max<long>(1, std::min<long>((P.gsize + 2047) / 2048, std::max(1, 8192 / P.ng)));
   P.part = dev_zeros<double>(P, (size_t)2 * P.ng * P.nchunk);
+  P.part_rz = dev_zeros<double>(P, (size_t)2 * P.ng * P.nchunk);
+  P.part_pq = dev_zeros<double>(P, (size_t)2 * P.ng * P.nchunk);
+  P.part_null = dev_zeros<double>(P, (size_t)2 * P.ng * P.nchunk);
   P.bb = dev_zeros<double>(P, 2 * P.ng);
   P.rr = dev_zeros<double>(P, 2 * P.ng);
   P.pq = dev_zeros<double>(P, 2 * P.ng);
@@ -758,12 +761,12 @@ void project(MGPlan &P, hipStream_t st, T *v) {
 }
 
 // z = V-cycle(r) (or the network's answer, net) with its null-space
-// component removed; rz = r.z.  rr: the per-group r.r of the current
-// residual (the network's input scale)
-void precondition(MGPlan &P, hipStream_t st, double *rz_new, bool net, const double *rr) {
+// component removed, and the partial sums of r.z (part_rz).  rr: the
+// per-group r.r of the current residual (the network's input scale)
+void precondition(MGPlan &P, hipStream_t st, bool net, const double *rr) {
+  const MGLev &L0 = P.h64.lev[0];
   if (P.prec >= 1) {
     if (net) {
-      const MGLev &L0 = P.h64.lev[0];
       launch_net_in(st, P.ng, L0.na, L0.ns, P.nH, P.nW, P.rf, rr, P.nact_plane, P.h64.lam, P.lam_ref,
                     P.net->input());
       P.net->forward(st, P.ng);
@@ -771,12 +774,12 @@ void precondition(MGPlan &P, hipStream_t st, double *rz_new, bool net, const dou
     } else {
       vcycle(P, P.h32, st, 0);
     }
-    project(P, st, P.zf);
-    mg_dot<float, float>(st, P.ng, P.gsize, P.r, P.zf, nullptr, nullptr, P.part, P.nchunk, rz_new, P.done, nullptr);
+    mg_dot_rz<float>(st, L0, P.ng, P.gsize, P.r, P.zf, P.part_rz, P.nchunk, P.done, P.singular, P.sing_list,
+                     P.any_singular ? P.n_sing : 0, P.part_null, P.nact);
   } else {
     vcycle(P, P.h64, st, 0);
-    project(P, st, P.z);
-    mg_dot<double, double>(st, P.ng, P.gsize, P.r, P.z, nullptr, nullptr, P.part, P.nchunk, rz_new, P.done, nullptr);
+    mg_dot_rz<double>(st, L0, P.ng, P.gsize, P.r, P.z, P.part_rz, P.nchunk, P.done, P.singular, P.sing_list,
+                      P.any_singular ? P.n_sing : 0, P.part_null, P.nact);
   }
 }
 
@@ -791,7 +794,7 @@ void mg_iteration(MGPlan &P, hipStream_t st, MGRun &R) {
   const bool mixed = P.prec >= 1;
   const double *rzo = nullptr;
   if (R.it > 0) {
-    precondition(P, st, P.rz[1 - R.cur], R.net, P.rr);
+    precondition(P, st, R.net, P.rr);
     rzo = P.rz[R.cur];
     R.cur = 1 - R.cur;
   }
@@ -805,32 +808,32 @@ void mg_iteration(MGPlan &P, hipStream_t st, MGRun &R) {
   // past the FP32 range), so the learned mode keeps FP64 directions.
   const MGLev &L0 = P.h64.lev[0];
   if (mixed && P.prec == 1) {
-    mg_dir_apply_dot<float, float>(st, L0, P.h64.lam, P.ng, P.gsize, P.rz[R.cur], rzo, rzo ? P.rr : nullptr, P.zf,
-                                   P.pf[R.pc], P.pf[1 - R.pc], P.part, P.nchunk, P.pq, P.done);
+    mg_dir_apply_dot<float, float>(st, L0, P.h64.lam, P.ng, P.gsize, P.part_rz, P.rz[R.cur], rzo, rzo ? P.rr : nullptr, P.zf,
+                                   P.pf[R.pc], P.pf[1 - R.pc], P.part_pq, P.nchunk, P.done);
     R.pc = 1 - R.pc;
     if (P.mark_update) P.mark_update(true);
-    mg_update_apply_dot<float>(st, L0, P.h64.lam, P.ng, P.gsize, P.rz[R.cur], P.pq, P.x, P.pf[R.pc], P.r, P.rf, P.zf,
-                               P.part, P.nchunk, P.rr, P.done, R.x_unset);
+    mg_update_apply_dot<float>(st, L0, P.h64.lam, P.ng, P.gsize, P.rz[R.cur], P.part_pq, P.x, P.pf[R.pc], P.r, P.rf, P.zf,
+                               P.part, P.nchunk, P.done, R.x_unset);
     if (P.mark_update) P.mark_update(false);
   } else if (mixed) {
-    mg_dir_apply_dot<float, double>(st, L0, P.h64.lam, P.ng, P.gsize, P.rz[R.cur], rzo, rzo ? P.rr : nullptr, P.zf,
-                                    P.pd[R.pc], P.pd[1 - R.pc], P.part, P.nchunk, P.pq, P.done);
+    mg_dir_apply_dot<float, double>(st, L0, P.h64.lam, P.ng, P.gsize, P.part_rz, P.rz[R.cur], rzo, rzo ? P.rr : nullptr, P.zf,
+                                    P.pd[R.pc], P.pd[1 - R.pc], P.part_pq, P.nchunk, P.done);
     R.pc = 1 - R.pc;
     if (P.mark_update) P.mark_update(true);
-    mg_update_apply_dot<double>(st, L0, P.h64.lam, P.ng, P.gsize, P.rz[R.cur], P.pq, P.x, P.pd[R.pc], P.r, P.rf,
-                                P.zf, P.part, P.nchunk, P.rr, P.done, R.x_unset);
+    mg_update_apply_dot<double>(st, L0, P.h64.lam, P.ng, P.gsize, P.rz[R.cur], P.part_pq, P.x, P.pd[R.pc], P.r, P.rf,
+                                P.zf, P.part, P.nchunk, P.done, R.x_unset);
     if (P.mark_update) P.mark_update(false);
   } else {
-    mg_dir_apply_dot<double, double>(st, L0, P.h64.lam, P.ng, P.gsize, P.rz[R.cur], rzo, nullptr, P.z, P.pd[R.pc],
-                                     P.pd[1 - R.pc], P.part, P.nchunk, P.pq, P.done);
+    mg_dir_apply_dot<double, double>(st, L0, P.h64.lam, P.ng, P.gsize, P.part_rz, P.rz[R.cur], rzo, nullptr, P.z, P.pd[R.pc],
+                                     P.pd[1 - R.pc], P.part_pq, P.nchunk, P.done);
     R.pc = 1 - R.pc;
     if (P.mark_update) P.mark_update(true);
-    mg_update_apply_dot<double>(st, L0, P.h64.lam, P.ng, P.gsize, P.rz[R.cur], P.pq, P.x, P.pd[R.pc], P.r, nullptr,
-                                nullptr, P.part, P.nchunk, P.rr, P.done, R.x_unset);
+    mg_update_apply_dot<double>(st, L0, P.h64.lam, P.ng, P.gsize, P.rz[R.cur], P.part_pq, P.x, P.pd[R.pc], P.r, nullptr,
+                                nullptr, P.part, P.nchunk, P.done, R.x_unset);
     if (P.mark_update) P.mark_update(false);
   }
   R.x_unset = false;  // written by this iteration's update pass
-  mg_flags(st, P.ng, P.rr, P.bb, P.tol * P.tol, P.done, P.left, P.mlist, R.it + 1);
+  mg_flags(st, P.ng, P.part, P.nchunk, P.rr, P.bb, P.tol * P.tol, P.done, P.left, P.mlist, R.it + 1);
   if (R.net && P.fallback) launch_net_stall(st, P.ng, P.rr, P.rr_prev, P.done, P.stall_ratio * P.stall_ratio, P.stall);
   R.it++;
 }
@@ -870,14 +873,14 @@ MGRun mg_solve(MGPlan &P, hipStream_t st, int fixed) {
   const bool cvt = mixed && !warm;
   if (cvt) mg_dot_self_cvt(st, P.ng, P.gsize, P.r, P.rf, P.part, P.nchunk, P.bb);
   else mg_dot<double, double>(st, P.ng, P.gsize, P.r, P.r, nullptr, nullptr, P.part, P.nchunk, P.bb, P.done, nullptr);
-  mg_flags(st, P.ng, P.bb, P.bb, tol2, P.done, P.left, P.mlist, 0);
+  mg_flags(st, P.ng, nullptr, 0, P.bb, P.bb, tol2, P.done, P.left, P.mlist, 0);
   if (R.record)  // the input half of this solve's training pairs
     launch_net_pair_in(st, P.ng, L0.na, L0.ns, P.nH, P.nW, P.r, P.bb, P.nact_plane, P.h64.lam, P.lam_ref,
                        P.pair_x + (size_t)P.pair_n * pl * 2);
   if (warm) {  // r = b - M x0; groups that x0 already solves stop here
     mg_apply_dot(st, L0, P.h64.lam, P.x, P.q, P.ng, P.gsize, P.part, P.nchunk, P.pq, P.done);
     mg_warm_residual(st, P.ng, P.gsize, P.bb, P.x, P.r, P.q, mixed ? P.rf : nullptr, P.part, P.nchunk, P.rr);
-    mg_flags(st, P.ng, P.rr, P.bb, tol2, P.done, P.left, P.mlist, 0);
+    mg_flags(st, P.ng, nullptr, 0, P.rr, P.bb, tol2, P.done, P.left, P.mlist, 0);
   }
   const double *rr0 = P.bb;  // r.r of the residual the first preconditioning sees
   if (R.net && P.guess) {
@@ -891,14 +894,14 @@ MGRun mg_solve(MGPlan &P, hipStream_t st, int fixed) {
     mg_apply_dot(st, L0, P.h64.lam, P.p, P.q, P.ng, P.gsize, P.part, P.nchunk, P.pq, P.done);
     mg_cg_update_dot(st, P.ng, P.gsize, P.pq, P.pq, P.x, P.p, P.r, P.q, P.rf, nullptr, P.part, P.nchunk, P.rr,
                      P.done);
-    mg_flags(st, P.ng, P.rr, P.bb, tol2, P.done, P.left, P.mlist, 0);
+    mg_flags(st, P.ng, nullptr, 0, P.rr, P.bb, tol2, P.done, P.left, P.mlist, 0);
     rr0 = P.rr;
   }
   if (R.net) {
     mg_izero(st, 1, P.stall);
     SNAC_HIP(hipMemcpyAsync(P.rr_prev, rr0, 2 * P.ng * sizeof(double), hipMemcpyDeviceToDevice, st));
   }
-  precondition(P, st, P.rz[R.cur], R.net, rr0);
+  precondition(P, st, R.net, rr0);
   if (fixed > 0) {  // captured: counted when the host resumes it (mg_continue)
     const int nit = std::min(fixed, P.maxiter);
     while (R.it < nit) mg_iteration(P, st, R);
