@@ -5,6 +5,7 @@
 #include <algorithm>
 #include <stdexcept>
 #include <string>
+#include <vector>
 
 namespace snac {
 
@@ -85,6 +86,45 @@ void launch_rk_mom(hipStream_t s, const Geo &g, const Metrics &m, const double *
                    const double *w, const double *p, double *un, double *vn, double *wn, double *dtu,
                    double *dtv, double *dtw, double f1, double f2, double f12, double visc, double bfx,
                    double bfy, double bfz, const double *s1, const double gb[3], int variant, bool impdiff);
+// One launch over up to GRID_BLOCKS grid blocks: per-block arguments and the
+// first workgroup of each (start[q + 1] == start[q]: no such block).  Small
+// blocks are bound by their launches: the four-block cavity's step took 78 of
+// them (0.26 ms) and takes 33 (0.16 ms).
+constexpr int GRID_BLOCKS = 8;
+template <typename Block>
+struct Blocks {
+  Block b[GRID_BLOCKS];
+  int start[GRID_BLOCKS + 1];
+};
+struct RkBlock {
+  Geo g;
+  Metrics m;
+  const double *u, *v, *w, *p;
+  double *un, *vn, *wn, *dtu, *dtv, *dtw;
+  const double *s1;
+};
+struct FillBlock {
+  Geo g;
+  Metrics m;
+  const double *u, *v, *w;
+  double *pp;
+  const double *r[6];
+};
+struct CorBlock {
+  Geo g;
+  Metrics m;
+  const double *pp, *u, *v, *w;
+  double *un, *vn, *wn, *p;
+};
+using RkBlocks = Blocks<RkBlock>;
+using FillBlocks = Blocks<FillBlock>;
+using CorBlocks = Blocks<CorBlock>;
+// variant 0 of launch_rk_mom, launch_fillps and launch_correc over several
+// blocks at once (the same arithmetic per cell)
+void launch_rk_mom_blocks(hipStream_t s, const std::vector<RkBlock> &blk, double f1, double f2, double f12, double visc,
+                          double bfx, double bfy, double bfz, const double gb[3], bool impdiff);
+void launch_fillps_blocks(hipStream_t s, const std::vector<FillBlock> &blk, int fft_axis, double dtrk);
+void launch_correc_blocks(hipStream_t s, const std::vector<CorBlock> &blk, double dtrk);
 // Mixed precision: the same substage with the right-hand side evaluated in
 // FP32 from FP32 copies of u, v, w staged in LDS and the old tendencies
 // stored in FP32 (same [k][j][component][i] layout, in floats); the RK3
@@ -177,6 +217,16 @@ R2RPlan r2r_plan(int kind, int n, bool rowwise = false);
 int r2r_tile_choices(const R2RPlan &pl);  // number of tile choices of the plan's kernel
 void launch_r2r(hipStream_t s, const R2RPlan &pl, const double *in, long ies, long is1, long is2,
                 double *out, long oes, long os1, long os2, int nb1, int nb2, double scale);
+// several line batches of one plan (one per grid block): one launch where the
+// plan is a matrix product, else one after the other
+struct R2RJob {
+  const double *in;
+  long ies, is1, is2;
+  double *out;
+  long oes, os1, os2;
+  int nb1, nb2;
+};
+void launch_r2r_jobs(hipStream_t s, const R2RPlan &pl, const std::vector<R2RJob> &jobs, double scale);
 // host reference of FFTW's r2r definitions, used to build dense matrices
 double r2r_coef(int kind, int n, int k, int j);
 

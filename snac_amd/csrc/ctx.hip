@@ -541,15 +541,17 @@ void stage_first(snac_ctx *c, const TensorOps &o) {
   const long pst[3] = {1, (long)t.G[0], (long)t.G[0] * t.G[1]};
   int a = t.xaxes[0], b1, b2;
   others(a, b1, b2);
+  std::vector<R2RJob> jobs;
   for (size_t b = 0; b < c->blk.size(); b++) {
     DevBlock &D = c->blk[b];
     const Block &B = c->cs.blocks[b];
     const double *in = D.pp + 1 + D.g.sx + D.g.sx * D.g.sy;
     long off = 0;
     for (int q = 0; q < 3; q++) off += (long)(B.lo_g[q] - t.gmin[q]) * pst[q];
-    launch_r2r(c->stream, o.fwd[0], in, gstride(D, a), gstride(D, b1), gstride(D, b2), t.ph + off, pst[a], pst[b1],
-               pst[b2], bext(D, b1), bext(D, b2), 1.0);
+    jobs.push_back(R2RJob{in, gstride(D, a), gstride(D, b1), gstride(D, b2), t.ph + off, pst[a], pst[b1], pst[b2],
+                          bext(D, b1), bext(D, b2)});
   }
+  launch_r2r_jobs(c->stream, o.fwd[0], jobs, 1.0);
 }
 
 // in-place transform number q on the work array (forward or inverse)
@@ -590,15 +592,17 @@ void stage_last(snac_ctx *c, const TensorOps &o, int comp) {
   const long pst[3] = {1, (long)t.G[0], (long)t.G[0] * t.G[1]};
   int a = t.xaxes[0], b1, b2;
   others(a, b1, b2);
+  std::vector<R2RJob> jobs;
   for (size_t b = 0; b < c->blk.size(); b++) {
     DevBlock &D = c->blk[b];
     const Block &B = c->cs.blocks[b];
     double *out = (comp < 0 ? D.pp : imp_field(c, D, comp)) + 1 + D.g.sx + D.g.sx * D.g.sy;
     long off = 0;
     for (int q = 0; q < 3; q++) off += (long)(B.lo_g[q] - t.gmin[q]) * pst[q];
-    launch_r2r(c->stream, o.bwd[0], t.ph + off, pst[a], pst[b1], pst[b2], out, gstride(D, a), gstride(D, b1),
-               gstride(D, b2), bext(D, b1), bext(D, b2), o.norm[0]);
+    jobs.push_back(R2RJob{t.ph + off, pst[a], pst[b1], pst[b2], out, gstride(D, a), gstride(D, b1), gstride(D, b2),
+                          bext(D, b1), bext(D, b2)});
   }
+  launch_r2r_jobs(c->stream, o.bwd[0], jobs, o.norm[0]);
 }
 
 // the whole tensor-product solve of one operator, pp -> pp (pressure) or
@@ -770,15 +774,17 @@ void mg_stage_in(snac_ctx *c, MGPlan &P) {
   if (P.fa >= 0) {
     int a = P.fa, b1, b2;
     others(a, b1, b2);
+    std::vector<R2RJob> jobs;
     for (size_t b = 0; b < c->blk.size(); b++) {
       DevBlock &D = c->blk[b];
       const Block &B = c->cs.blocks[b];
       const double *in = D.pp + 1 + D.g.sx + D.g.sx * D.g.sy;
       long off = 0;
       for (int q = 0; q < 3; q++) off += (long)(B.lo_g[q] - P.gmin[q]) * pst[q];
-      launch_r2r(c->stream, c->prec == SNAC_PREC_FP64 ? P.fwd : P.fwd_row, in, gstride(D, a), gstride(D, b1), gstride(D, b2), P.ph + off, pst[a], pst[b1],
-                 pst[b2], bext(D, b1), bext(D, b2), 1.0);
+      jobs.push_back(R2RJob{in, gstride(D, a), gstride(D, b1), gstride(D, b2), P.ph + off, pst[a], pst[b1], pst[b2],
+                            bext(D, b1), bext(D, b2)});
     }
+    launch_r2r_jobs(c->stream, c->prec == SNAC_PREC_FP64 ? P.fwd : P.fwd_row, jobs, 1.0);
     mg_copy3(c->stream, P.ph, pst[P.ax_m], pst[P.ax_a], pst[P.ax_s], P.r, na * ns, ns, 1, P.ng, (int)na,
              (int)ns, -1.0, pst[P.ax_a] == 1 ? 1 : 0);
   } else {
@@ -802,15 +808,17 @@ void mg_stage_out(snac_ctx *c, MGPlan &P) {
              (int)ns, 1.0, pst[P.ax_a] == 1 ? 2 : 0);
     int a = P.fa, b1, b2;
     others(a, b1, b2);
+    std::vector<R2RJob> jobs;
     for (size_t b = 0; b < c->blk.size(); b++) {
       DevBlock &D = c->blk[b];
       const Block &B = c->cs.blocks[b];
       double *out = D.pp + 1 + D.g.sx + D.g.sx * D.g.sy;
       long off = 0;
       for (int q = 0; q < 3; q++) off += (long)(B.lo_g[q] - P.gmin[q]) * pst[q];
-      launch_r2r(c->stream, c->prec == SNAC_PREC_FP64 ? P.bwd : P.bwd_row, P.ph + off, pst[a], pst[b1], pst[b2], out, gstride(D, a), gstride(D, b1),
-                 gstride(D, b2), bext(D, b1), bext(D, b2), P.norm);
+      jobs.push_back(R2RJob{P.ph + off, pst[a], pst[b1], pst[b2], out, gstride(D, a), gstride(D, b1), gstride(D, b2),
+                            bext(D, b1), bext(D, b2)});
     }
+    launch_r2r_jobs(c->stream, c->prec == SNAC_PREC_FP64 ? P.bwd : P.bwd_row, jobs, P.norm);
   } else {
     for (size_t b = 0; b < c->blk.size(); b++) {
       DevBlock &D = c->blk[b];
@@ -923,6 +931,16 @@ void rk_mom(snac_ctx *c, int irk, double dt) {
   const double gb[3] = {cs.gacc[0] * cs.beta, cs.gacc[1] * cs.beta, cs.gacc[2] * cs.beta};
   const bool buoy = c->buoyancy && cs.nscal > 0 && (gb[0] != 0.0 || gb[1] != 0.0 || gb[2] != 0.0);
   int nx = 1 - c->cur;
+  if (!c->st32 && c->rk_variant == 0 && c->blk.size() > 1) {
+    std::vector<RkBlock> b;
+    for (auto &D : c->blk)
+      b.push_back(RkBlock{D.g, D.m, D.vel[c->cur][0], D.vel[c->cur][1], D.vel[c->cur][2], D.p, D.vel[nx][0],
+                          D.vel[nx][1], D.vel[nx][2], D.dto[0], D.dto[1], D.dto[2],
+                          buoy ? D.sv[c->scur][0] : nullptr});
+    launch_rk_mom_blocks(c->stream, b, f1, f2, f12, cs.visc, cs.bforce[0], cs.bforce[1], cs.bforce[2], gb, c->impdiff);
+    c->cur = nx;
+    return;
+  }
   for (auto &D : c->blk) {
     if (c->st32)
       launch_rk_mom_f32(c->stream, D.g, D.m, D.vel[c->cur][0], D.vel[c->cur][1], D.vel[c->cur][2], D.p,
@@ -1008,6 +1026,16 @@ void rk_scal(snac_ctx *c, int irk, double dt) {
 }
 
 void fillps(snac_ctx *c, double dtrk) {
+  if (c->blk.size() > 1) {
+    std::vector<FillBlock> b;
+    for (auto &D : c->blk) {
+      FillBlock f{D.g, D.m, D.vel[c->cur][0], D.vel[c->cur][1], D.vel[c->cur][2], D.pp, {}};
+      for (int q = 0; q < 6; q++) f.r[q] = D.rhsp[q];
+      b.push_back(f);
+    }
+    launch_fillps_blocks(c->stream, b, c->cs.fft_axis, dtrk);
+    return;
+  }
   for (auto &D : c->blk)
     launch_fillps(c->stream, D.g, D.m, c->cs.fft_axis, D.vel[c->cur][0], D.vel[c->cur][1], D.vel[c->cur][2], D.pp,
                   dtrk, D.rhsp);
@@ -1015,6 +1043,15 @@ void fillps(snac_ctx *c, double dtrk) {
 
 void correc(snac_ctx *c, double dtrk, bool fuse_pressure) {
   int nx = 1 - c->cur;
+  if (c->blk.size() > 1) {
+    std::vector<CorBlock> b;
+    for (auto &D : c->blk)
+      b.push_back(CorBlock{D.g, D.m, D.pp, D.vel[c->cur][0], D.vel[c->cur][1], D.vel[c->cur][2], D.vel[nx][0],
+                           D.vel[nx][1], D.vel[nx][2], fuse_pressure ? D.p : nullptr});
+    launch_correc_blocks(c->stream, b, dtrk);
+    c->cur = nx;
+    return;
+  }
   for (auto &D : c->blk)
     launch_correc(c->stream, D.g, D.m, D.pp, D.vel[c->cur][0], D.vel[c->cur][1], D.vel[c->cur][2], D.vel[nx][0],
                   D.vel[nx][1], D.vel[nx][2], dtrk, fuse_pressure ? D.p : nullptr);

@@ -599,13 +599,18 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void k_
 // of the lines' bytes); 146 -> 12-17 us for a 180x77x90 channel's, 8.1 -> 3.4
 // us for two-point lines.
 typedef double double4_ __attribute__((ext_vector_type(4)));
-struct MArgs {
+struct MJob {  // one batch of lines and its first workgroup
   const double *in;
   double *out;
   long ies, is1, is2, oes, os1, os2;
+  int nb1, nlines, start;
+};
+struct MArgs {
+  MJob job[GRID_BLOCKS];
+  int njob;
   const double *fs, *fa;  // matrix fragments [tile][k / 4][64] of the two parts
   double scale;
-  int n, nb1, nlines;
+  int n;
   int half;     // samples up to the mirror (MODE 0: n)
   int rows;     // matrix rows of the symmetric part (MODE 2: of both)
   int ks, ka;   // inner lengths of the two parts
@@ -621,14 +626,17 @@ __global__ __launch_bounds__(512) void k_r2r_mfma(MArgs a) {
   double *X = reinterpret_cast<double *>(S);  // [L][ld]: symmetric part, then (at ksp) the antisymmetric one
   long *oin = reinterpret_cast<long *>(X + (size_t)L * a.ld), *oout = oin + L;
   const int ksp = (a.ks + 3) & ~3, kap = (a.ka + 3) & ~3;
-  const int line0 = blockIdx.x * L;
+  int q = 0;
+  while (q + 1 < a.njob && (int)blockIdx.x >= a.job[q + 1].start) q++;
+  const MJob &J = a.job[q];
+  const int line0 = (blockIdx.x - J.start) * L;
   for (int t = threadIdx.x; t < L; t += nthr) {
     const int line = line0 + t;
     long oi = -1, oo = -1;
-    if (line < a.nlines) {
-      const int b1 = line % a.nb1, b2 = line / a.nb1;
-      oi = b1 * a.is1 + b2 * a.is2;
-      oo = b1 * a.os1 + b2 * a.os2;
+    if (line < J.nlines) {
+      const int b1 = line % J.nb1, b2 = line / J.nb1;
+      oi = b1 * J.is1 + b2 * J.is2;
+      oo = b1 * J.os1 + b2 * J.os2;
     }
     oin[t] = oi;
     oout[t] = oo;
@@ -636,23 +644,77 @@ __global__ __launch_bounds__(512) void k_r2r_mfma(MArgs a) {
   __syncthreads();
   // 1. lines into LDS: folded (MODE 1), sorted into the two parts (MODE 2) or
   // as they are; the inner dimension's padding is zero
-  const bool coal = a.ies != 1;  // consecutive threads on consecutive lines
-  const int cols = MODE == 1 ? a.half : n, lsh = __ffs(L) - 1;  // L is a power of two
-  for (int e = threadIdx.x; e < L * cols; e += nthr) {
-    const int l = coal ? e & (L - 1) : e / cols, j = coal ? e >> lsh : e - l * cols;
-    const long o = oin[l];
-    double *row = X + l * a.ld;
-    const double x = o >= 0 ? a.in[j * a.ies + o] : 0.0;
+  const int cols = MODE == 1 ? a.half : n;
+  const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), ln = threadIdx.x & 63;
+  constexpr int U = 4;  // elements (MODE 1: pairs) in flight per thread
+  auto mirror = [&](int j) { return a.hc ? (j == 0 ? 0 : n - j) : n - 1 - j; };
+  auto put = [&](double *row, int j, double x, double y) {
     if (MODE == 1) {
-      const int mir = a.hc ? (j == 0 ? 0 : n - j) : n - 1 - j;
-      const double y = mir != j && o >= 0 ? a.in[mir * a.ies + o] : 0.0;
       row[j] = x + y;
-      if (j < a.ka) row[ksp + j] = mir != j ? x - y : 0.0;
+      if (j < a.ka) row[ksp + j] = mirror(j) != j ? x - y : 0.0;
     } else if (MODE == 2) {
       if (a.hc) row[j < a.ks ? j : ksp + n - 1 - j] = x;
       else row[(j & 1) ? ksp + (j >> 1) : j >> 1] = x;
     } else {
       row[j] = x;
+    }
+  };
+  if (J.ies != 1) {  // strided lines: consecutive threads on consecutive lines, one line per thread
+    const int lsh = __ffs(L) - 1, l = threadIdx.x & (L - 1), js = nthr >> lsh;  // L is a power of two dividing nthr
+    const long o = oin[l];
+    double *row = X + l * a.ld;
+    const double *p = J.in + (o >= 0 ? o : 0);
+    for (int j0 = threadIdx.x >> lsh; j0 < cols; j0 += js * U) {
+      double x[U], y[U];
+#pragma unroll
+      for (int u = 0; u < U; u++) {
+        const int j = j0 + u * js;
+        const bool ok = o >= 0 && j < cols;
+        x[u] = ok ? p[j * J.ies] : 0.0;
+        y[u] = MODE == 1 && ok && mirror(j) != j ? p[mirror(j) * J.ies] : 0.0;
+      }
+#pragma unroll
+      for (int u = 0; u < U; u++)
+        if (j0 + u * js < cols) put(row, j0 + u * js, x[u], y[u]);
+    }
+  } else if (cols < 48) {  // short contiguous lines: samples of several lines per wavefront
+    for (int e0 = threadIdx.x; e0 < L * cols; e0 += nthr * U) {
+      double x[U], y[U];
+      int l[U], j[U];
+#pragma unroll
+      for (int u = 0; u < U; u++) {
+        const int e = e0 + u * nthr;
+        l[u] = min(e / cols, L - 1);
+        j[u] = e - l[u] * cols;
+        const long o = oin[l[u]];
+        const bool ok = o >= 0 && j[u] < cols;
+        const double *p = J.in + o;
+        x[u] = ok ? p[j[u]] : 0.0;
+        y[u] = MODE == 1 && ok && mirror(j[u]) != j[u] ? p[mirror(j[u])] : 0.0;
+      }
+#pragma unroll
+      for (int u = 0; u < U; u++)
+        if (j[u] < cols) put(X + l[u] * a.ld, j[u], x[u], y[u]);
+    }
+  } else {  // contiguous lines: a wavefront on 64 samples of a line
+    const int nch = (cols + 63) >> 6, nw = a.tw * a.lg, tot = (L / nw + (wv < L % nw ? 1 : 0)) * nch;
+    for (int t0 = 0; t0 < tot; t0 += U) {
+      double x[U], y[U];
+      int l[U], j[U];
+#pragma unroll
+      for (int u = 0; u < U; u++) {
+        const int t = t0 + u, q = t / nch;
+        l[u] = min(wv + q * nw, L - 1);
+        j[u] = t < tot ? ((t - q * nch) << 6) + ln : cols;
+        const long o = oin[l[u]];
+        const bool ok = o >= 0 && j[u] < cols;
+        const double *p = J.in + o;
+        x[u] = ok ? p[j[u]] : 0.0;
+        y[u] = MODE == 1 && ok && mirror(j[u]) != j[u] ? p[mirror(j[u])] : 0.0;
+      }
+#pragma unroll
+      for (int u = 0; u < U; u++)
+        if (j[u] < cols) put(X + l[u] * a.ld, j[u], x[u], y[u]);
     }
   }
   for (int l = threadIdx.x; l < L; l += nthr) {
@@ -661,7 +723,6 @@ __global__ __launch_bounds__(512) void k_r2r_mfma(MArgs a) {
     for (int k = a.ka; k < kap; k++) row[ksp + k] = 0.0;
   }
   __syncthreads();
-  const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), ln = threadIdx.x & 63;
   const int lq = ln & 15, kq = ln >> 4, l0 = (wv / a.tw) * 16 * NTL;
   for (int tile = wv % a.tw; tile < a.ntile; tile += a.tw) {
     double4_ es[NTL], ea[NTL];
@@ -669,29 +730,51 @@ __global__ __launch_bounds__(512) void k_r2r_mfma(MArgs a) {
     for (int t = 0; t < NTL; t++) { es[t] = double4_{0, 0, 0, 0}; ea[t] = double4_{0, 0, 0, 0}; }
     // 2. the two products; operand layout: lane -> (row or column ln & 15, inner ln >> 4)
     const double *xs = X + (l0 + lq) * a.ld + kq;
-    auto product = [&](const double *f, const double *x, int nk, double4_ (&acc)[NTL]) {
-      auto step = [&](double m, int k) {
+    auto step = [&](double m, const double *x, int k, double4_ (&acc)[NTL]) {
 #pragma unroll
-        for (int t = 0; t < NTL; t++) {
-          const double b = x[t * 16 * a.ld + 4 * k];
-          acc[t] = SWAP ? __builtin_amdgcn_mfma_f64_16x16x4f64(b, m, acc[t], 0, 0, 0)
-                        : __builtin_amdgcn_mfma_f64_16x16x4f64(m, b, acc[t], 0, 0, 0);
-        }
-      };
-      f += ln;
-      int k = 0;
-      for (; k + 4 <= nk; k += 4, f += 256) {  // four matrix loads in flight
-        const double m0 = f[0], m1 = f[64], m2 = f[128], m3 = f[192];
-        step(m0, k);
-        step(m1, k + 1);
-        step(m2, k + 2);
-        step(m3, k + 3);
+      for (int t = 0; t < NTL; t++) {
+        const double b = x[t * 16 * a.ld + 4 * k];
+        acc[t] = SWAP ? __builtin_amdgcn_mfma_f64_16x16x4f64(b, m, acc[t], 0, 0, 0)
+                      : __builtin_amdgcn_mfma_f64_16x16x4f64(m, b, acc[t], 0, 0, 0);
       }
-      for (; k < nk; k++, f += 64) step(f[0], k);
     };
-    product(a.fs + (size_t)tile * (ksp / 4) * 64, xs, ksp / 4, es);
-    if (MODE != 0) product(a.fa + (size_t)tile * (kap / 4) * 64, xs + ksp, kap / 4, ea);
+    // both parts side by side, the matrix values of the next W inner blocks
+    // loaded before this one's products (W of either part in flight)
+    constexpr int W = 4;
+    const int nks = ksp / 4, nka = MODE != 0 ? kap / 4 : 0;
+    const double *fs = a.fs + (size_t)tile * nks * 64 + ln, *fa = a.fa + (size_t)tile * nka * 64 + ln;
+    const int nk = MODE != 0 ? min(nks, nka) : nks, nw = nk / W * W;
+    double ms[W], ma[W];
+    if (nw > 0) {
+#pragma unroll
+      for (int u = 0; u < W; u++) {
+        ms[u] = fs[u * 64];
+        if (MODE != 0) ma[u] = fa[u * 64];
+      }
+    }
+    for (int k = 0; k < nw; k += W) {
+      double ns[W], na[W];
+      const bool more = k + W < nw;
+#pragma unroll
+      for (int u = 0; u < W; u++) {
+        ns[u] = more ? fs[(size_t)(k + W + u) * 64] : 0.0;
+        if (MODE != 0) na[u] = more ? fa[(size_t)(k + W + u) * 64] : 0.0;
+      }
+#pragma unroll
+      for (int u = 0; u < W; u++) {
+        step(ms[u], xs, k + u, es);
+        if (MODE != 0) step(ma[u], xs + ksp, k + u, ea);
+      }
+#pragma unroll
+      for (int u = 0; u < W; u++) {
+        ms[u] = ns[u];
+        if (MODE != 0) ma[u] = na[u];
+      }
+    }
+    for (int k = nw; k < nks; k++) step(fs[(size_t)k * 64], xs, k, es);
+    for (int k = nw; k < nka; k++) step(fa[(size_t)k * 64], xs + ksp, k, ea);
     // 3. results: register v of a lane is row 4 v + (ln >> 4), column ln & 15
+    const long oes = SWAP ? 1 : J.oes;
 #pragma unroll
     for (int t = 0; t < NTL; t++)
 #pragma unroll
@@ -699,16 +782,16 @@ __global__ __launch_bounds__(512) void k_r2r_mfma(MArgs a) {
         const int l = l0 + 16 * t + (SWAP ? 4 * v + kq : lq), r = 16 * tile + (SWAP ? lq : 4 * v + kq);
         const long o = oout[l];
         if (o < 0 || r >= a.rows) continue;
-        double *y = a.out + o;
+        double *y = J.out + o;
         if (MODE == 0) {
-          y[r * a.oes] = es[t][v] * a.scale;
+          y[r * oes] = es[t][v] * a.scale;
         } else if (MODE == 1) {
-          y[(a.hc ? r : 2 * r) * a.oes] = es[t][v] * a.scale;
-          if (r < a.na) y[(a.hc ? n - 1 - r : 2 * r + 1) * a.oes] = ea[t][v] * a.scale;
+          y[(a.hc ? r : 2 * r) * oes] = es[t][v] * a.scale;
+          if (r < a.na) y[(a.hc ? n - 1 - r : 2 * r + 1) * oes] = ea[t][v] * a.scale;
         } else {
-          const int mir = a.hc ? (r == 0 ? 0 : n - r) : n - 1 - r;
-          y[r * a.oes] = (es[t][v] + ea[t][v]) * a.scale;
-          if (mir != r) y[mir * a.oes] = (es[t][v] - ea[t][v]) * a.scale;
+          const int mir = mirror(r);
+          y[r * oes] = (es[t][v] + ea[t][v]) * a.scale;
+          if (mir != r) y[mir * oes] = (es[t][v] - ea[t][v]) * a.scale;
         }
       }
   }
@@ -946,13 +1029,11 @@ std::vector<double> mfma_fragments(int kind, int n) {
   return f;
 }
 
-void launch_mfma(hipStream_t s, const Args &b, int kind, double scale, const double *frag) {
-  const MSplit m = mfma_split(kind, b.n);
-  MArgs a;
-  a.in = b.in; a.out = b.out;
-  a.ies = b.ies; a.is1 = b.is1; a.is2 = b.is2; a.oes = b.oes; a.os1 = b.os1; a.os2 = b.os2;
+void launch_mfma(hipStream_t s, int kind, int n, const R2RJob *jobs, int njob, double scale, const double *frag) {
+  const MSplit m = mfma_split(kind, n);
+  MArgs a{};
   a.scale = scale;
-  a.n = b.n; a.nb1 = b.nb1; a.nlines = b.nlines;
+  a.n = n;
   a.half = m.half; a.rows = m.rows; a.ks = m.ks; a.ka = m.ka; a.na = m.na; a.hc = m.hc;
   a.ld = mfma_ld(m);
   a.ntile = (m.rows + 15) / 16;
@@ -962,14 +1043,25 @@ void launch_mfma(hipStream_t s, const Args &b, int kind, double scale, const dou
   // groups per workgroup instead (at least four wavefronts)
   a.tw = std::min(a.ntile, 8);
   a.lg = a.tw == 1 ? 4 : (a.tw == 2 ? 2 : 1);
+  long total = 0;
+  for (int q = 0; q < njob; q++) total += (long)jobs[q].nb1 * jobs[q].nb2;
   // two tiles of lines per wavefront (each matrix load used twice) where two
   // workgroups still fit a CU's LDS and the launch has two workgroups per CU
-  const int ntl = mfma_lds(a.ld, 32 * a.lg) <= LDS_MAX / 2 && a.nlines >= 32 * a.lg * 512 ? 2 : 1;
+  const int ntl = mfma_lds(a.ld, 32 * a.lg) <= LDS_MAX / 2 && total >= 32L * a.lg * 512 ? 2 : 1;
   while (a.lg > 1 && mfma_lds(a.ld, 16 * ntl * a.lg) > LDS_MAX) a.lg >>= 1;
   const int L = 16 * ntl * a.lg;
-  const dim3 grid((unsigned)((a.nlines + L - 1) / L)), blk(64 * a.tw * a.lg);
+  int wg = 0;
+  for (int q = 0; q < njob; q++) {
+    const R2RJob &b = jobs[q];
+    const int nlines = b.nb1 * b.nb2;
+    if (nlines <= 0) continue;
+    a.job[a.njob++] = MJob{b.in, b.out, b.ies, b.is1, b.is2, b.oes, b.os1, b.os2, b.nb1, nlines, wg};
+    wg += (nlines + L - 1) / L;
+  }
+  if (wg == 0) return;
+  const dim3 grid((unsigned)wg), blk(64 * a.tw * a.lg);
   const size_t lds = mfma_lds(a.ld, L);
-  const bool sw = a.oes == 1;
+  const bool sw = jobs[0].oes == 1;  // the same axis, so the same for every job
 #define SNAC_MF(M, W, T) hipLaunchKernelGGL((k_r2r_mfma<M, W, T>), grid, blk, lds, s, a)
 #define SNAC_MFM(M)                                                                  \
   do {                                                                               \
@@ -1099,7 +1191,8 @@ void launch_r2r(hipStream_t s, const R2RPlan &pl, const double *in, long ies, lo
     size_t lds = (size_t)L * pl.n * sizeof(double2);
     launch_fft_kind(pl.kind, pl.n, ls, grid, lds, s, a);
   } else if (pl.mfma) {
-    launch_mfma(s, a, pl.kind, scale, pl.tab);
+    const R2RJob j{in, ies, is1, is2, out, oes, os1, os2, nb1, nb2};
+    launch_mfma(s, pl.kind, pl.n, &j, 1, scale, pl.tab);
   } else {
     int L = std::max(1, std::min(2 * LDS_COMPLEX / pl.n, a.nlines));
     a.L = L;
@@ -1110,6 +1203,18 @@ void launch_r2r(hipStream_t s, const R2RPlan &pl, const double *in, long ies, lo
     hipLaunchKernelGGL(k_r2r_dense, grid, dim3(NT), lds, s, a);
   }
   SNAC_HIP(hipGetLastError());
+}
+
+void launch_r2r_jobs(hipStream_t s, const R2RPlan &pl, const std::vector<R2RJob> &jobs, double scale) {
+  if (pl.mfma) {
+    for (size_t q = 0; q < jobs.size(); q += GRID_BLOCKS) {
+      launch_mfma(s, pl.kind, pl.n, &jobs[q], (int)std::min<size_t>(GRID_BLOCKS, jobs.size() - q), scale, pl.tab);
+      SNAC_HIP(hipGetLastError());
+    }
+    return;
+  }
+  for (const R2RJob &j : jobs)
+    launch_r2r(s, pl, j.in, j.ies, j.is1, j.is2, j.out, j.oes, j.os1, j.os2, j.nb1, j.nb2, scale);
 }
 
 }  // namespace snac

@@ -13,19 +13,33 @@ constexpr int TX = 64, TY = 4;
 
 __device__ __forceinline__ long gidx(long i, long j, long k, long sx, long sy) { return i + sx * (j + sy * k); }
 
-// Tile coordinates of this workgroup in a (gx, gy, *) tile grid launched as a
-// 1D grid.  Workgroups are dispatched round-robin over the 8 XCDs; remapping
+// Tile coordinates of workgroup bid of nblk in a (gx, gy, *) tile grid launched
+// as a 1D grid.  Workgroups are dispatched round-robin over the 8 XCDs; remapping
 // gives each XCD one contiguous run of tiles (a k-slab), so the i/j/k
 // neighbours a stencil re-reads sit in the same XCD's L2.  A bijection for
 // any grid size.
-__device__ __forceinline__ void tile_of(int gx, int gy, int &bx, int &by, int &bz) {
-  const int nblk = gridDim.x, bid = blockIdx.x;
+__device__ __forceinline__ void tile_of(int nblk, int bid, int gx, int gy, int &bx, int &by, int &bz) {
   const int xcd = bid & 7, q = bid >> 3, per = nblk >> 3, rem = nblk & 7;
   const int lid = (xcd < rem ? xcd * (per + 1) : rem * (per + 1) + (xcd - rem) * per) + q;
   bx = lid % gx;
   const int t = lid / gx;
   by = t % gy;
   bz = t / gy;
+}
+__device__ __forceinline__ void tile_of(int gx, int gy, int &bx, int &by, int &bz) {
+  tile_of(gridDim.x, blockIdx.x, gx, gy, bx, by, bz);
+}
+// Which grid block a workgroup of a launch over several works on: start[q] is
+// the first workgroup of block q (the last entries repeat the total).  Cases
+// of several small grid blocks are bound by their launches, about 4 us each.
+template <typename Args>
+__device__ __forceinline__ int block_of(const Args &A, int &bid, int &nblk) {
+  int q = 0;
+#pragma unroll
+  for (int e = 1; e < GRID_BLOCKS; e++) q += (int)blockIdx.x >= A.start[e];
+  bid = blockIdx.x - A.start[q];
+  nblk = A.start[q + 1] - A.start[q];
+  return q;
 }
 
 // The old tendencies dudtrko, dvdtrko, dwdtrko share one array, row by row:
@@ -39,17 +53,9 @@ __device__ __forceinline__ long dto_index(const Geo &g, int i, int j, int k) {
 // BUOY: Boussinesq buoyancy of scalar 1, -f12*gacc*beta*(face average of s)
 // (rk.f90:104-108), gb = gacc*beta
 template <bool BUOY, bool IMP>
-__global__ __launch_bounds__(TX *TY) void k_rk_mom(Geo g, Metrics m, const double *__restrict__ u,
-                                                    const double *__restrict__ v, const double *__restrict__ w,
-                                                    const double *__restrict__ p, double *__restrict__ un,
-                                                    double *__restrict__ vn, double *__restrict__ wn,
-                                                    double *__restrict__ dtu, double *__restrict__ dtv,
-                                                    double *__restrict__ dtw, double f1, double f2, double f12,
-                                                    double visc, double bfx, double bfy, double bfz,
-                                                    const double *__restrict__ s1, double gbx, double gby,
-                                                    double gbz) {
+__device__ __forceinline__ void rk_mom_cell(int nblk, int bid, Geo g, Metrics m, const double *__restrict__ u, const double *__restrict__ v, const double *__restrict__ w, const double *__restrict__ p, double *__restrict__ un, double *__restrict__ vn, double *__restrict__ wn, double *__restrict__ dtu, double *__restrict__ dtv, double *__restrict__ dtw, double f1, double f2, double f12, double visc, double bfx, double bfy, double bfz, const double *__restrict__ s1, double gbx, double gby, double gbz) {
   int bx, by, bz;
-  tile_of((g.nx + TX - 1) / TX, (g.ny + TY - 1) / TY, bx, by, bz);
+  tile_of(nblk, bid, (g.nx + TX - 1) / TX, (g.ny + TY - 1) / TY, bx, by, bz);
   const int i = bx * TX + threadIdx.x + 1;
   const int j = by * TY + threadIdx.y + 1;
   const int k = bz + 1;
@@ -134,6 +140,28 @@ __global__ __launch_bounds__(TX *TY) void k_rk_mom(Geo g, Metrics m, const doubl
   un[c] = un_;
   vn[c] = vn_;
   wn[c] = wn_;
+}
+template <bool BUOY, bool IMP>
+__global__ __launch_bounds__(TX *TY) void k_rk_mom(Geo g, Metrics m, const double *__restrict__ u,
+                                                    const double *__restrict__ v, const double *__restrict__ w,
+                                                    const double *__restrict__ p, double *__restrict__ un,
+                                                    double *__restrict__ vn, double *__restrict__ wn,
+                                                    double *__restrict__ dtu, double *__restrict__ dtv,
+                                                    double *__restrict__ dtw, double f1, double f2, double f12,
+                                                    double visc, double bfx, double bfy, double bfz,
+                                                    const double *__restrict__ s1, double gbx, double gby,
+                                                    double gbz) {
+  rk_mom_cell<BUOY, IMP>(gridDim.x, blockIdx.x, g, m, u, v, w, p, un, vn, wn, dtu, dtv, dtw, f1, f2, f12, visc, bfx, bfy, bfz, s1, gbx, gby, gbz);
+}
+
+template <bool BUOY, bool IMP>
+__global__ __launch_bounds__(TX *TY) void k_rk_mom_blocks(RkBlocks A, double f1, double f2, double f12, double visc,
+                                                          double bfx, double bfy, double bfz, double gbx, double gby,
+                                                          double gbz) {
+  int bid, nblk;
+  const RkBlock &b = A.b[block_of(A, bid, nblk)];
+  rk_mom_cell<BUOY, IMP>(nblk, bid, b.g, b.m, b.u, b.v, b.w, b.p, b.un, b.vn, b.wn, b.dtu, b.dtv, b.dtw, f1, f2, f12,
+                         visc, bfx, bfy, bfz, b.s1, gbx, gby, gbz);
 }
 
 // The same substage with each thread marching along k over a chunk of KB
@@ -548,13 +576,9 @@ __global__ __launch_bounds__(TX *TY) void k_rk_scal(Geo g, Metrics m, const doub
   dso[q] = d;
 }
 
-__global__ __launch_bounds__(TX *TY) void k_fillps(Geo g, Metrics m, int fa, const double *__restrict__ u,
-                                                    const double *__restrict__ v, const double *__restrict__ w,
-                                                    double *__restrict__ pp, double idtrk, const double *rx0,
-                                                    const double *rx1, const double *ry0, const double *ry1,
-                                                    const double *rz0, const double *rz1) {
+__device__ __forceinline__ void fillps_cell(int nblk, int bid, Geo g, Metrics m, int fa, const double *__restrict__ u, const double *__restrict__ v, const double *__restrict__ w, double *__restrict__ pp, double idtrk, const double *rx0, const double *rx1, const double *ry0, const double *ry1, const double *rz0, const double *rz1) {
   int bx, by, bz;
-  tile_of((g.nx + TX - 1) / TX, (g.ny + TY - 1) / TY, bx, by, bz);
+  tile_of(nblk, bid, (g.nx + TX - 1) / TX, (g.ny + TY - 1) / TY, bx, by, bz);
   const int i = bx * TX + threadIdx.x + 1;
   const int j = by * TY + threadIdx.y + 1;
   const int k = bz + 1;
@@ -580,16 +604,19 @@ __global__ __launch_bounds__(TX *TY) void k_fillps(Geo g, Metrics m, int fa, con
   if (rz1 && k == g.nz) r += rz1[(i - 1) + (long)g.nx * (j - 1)];
   st_nt<true>(pp + c, r);  // written once, read by the next kernel
 }
+__global__ __launch_bounds__(TX *TY) void k_fillps(Geo g, Metrics m, int fa, const double *__restrict__ u,
+                                                    const double *__restrict__ v, const double *__restrict__ w,
+                                                    double *__restrict__ pp, double idtrk, const double *rx0,
+                                                    const double *rx1, const double *ry0, const double *ry1,
+                                                    const double *rz0, const double *rz1) {
+  fillps_cell(gridDim.x, blockIdx.x, g, m, fa, u, v, w, pp, idtrk, rx0, rx1, ry0, ry1, rz0, rz1);
+}
 
 // correc over the whole ghosted box; cells outside the reference's loop
 // ranges (i <= nx for u, j <= ny for v, k <= nz for w) are copied
-__global__ __launch_bounds__(TX *TY) void k_correc(Geo g, Metrics m, const double *__restrict__ pp,
-                                                    const double *__restrict__ u, const double *__restrict__ v,
-                                                    const double *__restrict__ w, double *__restrict__ un,
-                                                    double *__restrict__ vn, double *__restrict__ wn, double dtrk,
-                                                    double *__restrict__ p) {
+__device__ __forceinline__ void correc_cell(int nblk, int bid, Geo g, Metrics m, const double *__restrict__ pp, const double *__restrict__ u, const double *__restrict__ v, const double *__restrict__ w, double *__restrict__ un, double *__restrict__ vn, double *__restrict__ wn, double dtrk, double *__restrict__ p) {
   int bx, by, bz;
-  tile_of((g.nx + 2 + TX - 1) / TX, (g.ny + 2 + TY - 1) / TY, bx, by, bz);
+  tile_of(nblk, bid, (g.nx + 2 + TX - 1) / TX, (g.ny + 2 + TY - 1) / TY, bx, by, bz);
   const int i = bx * TX + threadIdx.x;
   const int j = by * TY + threadIdx.y;
   const int k = bz;
@@ -605,6 +632,25 @@ __global__ __launch_bounds__(TX *TY) void k_correc(Geo g, Metrics m, const doubl
   vn[c] = vv;
   wn[c] = ww;
   if (p && i >= 1 && i <= g.nx && j >= 1 && j <= g.ny && k >= 1 && k <= g.nz) p[c] = p[c] + pc;
+}
+__global__ __launch_bounds__(TX *TY) void k_correc(Geo g, Metrics m, const double *__restrict__ pp,
+                                                    const double *__restrict__ u, const double *__restrict__ v,
+                                                    const double *__restrict__ w, double *__restrict__ un,
+                                                    double *__restrict__ vn, double *__restrict__ wn, double dtrk,
+                                                    double *__restrict__ p) {
+  correc_cell(gridDim.x, blockIdx.x, g, m, pp, u, v, w, un, vn, wn, dtrk, p);
+}
+
+__global__ __launch_bounds__(TX *TY) void k_fillps_blocks(FillBlocks A, int fa, double idtrk) {
+  int bid, nblk;
+  const FillBlock &b = A.b[block_of(A, bid, nblk)];
+  fillps_cell(nblk, bid, b.g, b.m, fa, b.u, b.v, b.w, b.pp, idtrk, b.r[0], b.r[1], b.r[2], b.r[3], b.r[4], b.r[5]);
+}
+
+__global__ __launch_bounds__(TX *TY) void k_correc_blocks(CorBlocks A, double dtrk) {
+  int bid, nblk;
+  const CorBlock &b = A.b[block_of(A, bid, nblk)];
+  correc_cell(nblk, bid, b.g, b.m, b.pp, b.u, b.v, b.w, b.un, b.vn, b.wn, dtrk, b.p);
 }
 
 __global__ __launch_bounds__(TX *TY) void k_updt_pressure(Geo g, const double *__restrict__ pp,
@@ -812,6 +858,26 @@ void launch_rk_mom_f32(hipStream_t s, const Geo &g, const Metrics &m, const doub
                            variant, impdiff);
 }
 
+namespace {
+// launches go(args, workgroups) over the blocks, GRID_BLOCKS at a time
+template <typename Args, typename Block, typename Size, typename Go>
+void in_batches(const std::vector<Block> &blk, Size &&size, Go &&go) {
+  for (size_t q0 = 0; q0 < blk.size(); q0 += GRID_BLOCKS) {
+    Args A{};
+    int n = 0;
+    for (int q = 0; q < GRID_BLOCKS; q++) {
+      A.start[q] = n;
+      if (q0 + q >= blk.size()) continue;
+      A.b[q] = blk[q0 + q];
+      n += (int)size(A.b[q]);
+    }
+    A.start[GRID_BLOCKS] = n;
+    go(A, (unsigned)n);
+    SNAC_HIP(hipGetLastError());
+  }
+}
+}  // namespace
+
 void launch_rk_mom(hipStream_t s, const Geo &g, const Metrics &m, const double *u, const double *v, const double *w,
                    const double *p, double *un, double *vn, double *wn, double *dtu, double *dtv, double *dtw,
                    double f1, double f2, double f12, double visc, double bfx, double bfy, double bfz,
@@ -895,6 +961,34 @@ void launch_bulk_force(hipStream_t s, const Geo &g, double *f, const double *red
   SNAC_HIP(hipGetLastError());
 }
 
+void launch_rk_mom_blocks(hipStream_t s, const std::vector<RkBlock> &blk, double f1, double f2, double f12, double visc,
+                          double bfx, double bfy, double bfz, const double gb[3], bool impdiff) {
+  in_batches<RkBlocks>(blk, [](const RkBlock &b) { return interior_tiles(b.g).x; }, [&](const RkBlocks &A, unsigned n) {
+#define SNAC_KB(B, I)                                                                                               \
+  hipLaunchKernelGGL((k_rk_mom_blocks<B, I>), dim3(n), dim3(TX, TY), 0, s, A, f1, f2, f12, visc, bfx, bfy, bfz, gb[0], \
+                     gb[1], gb[2])
+    if (blk[0].s1) {
+      if (impdiff) SNAC_KB(true, true);
+      else SNAC_KB(true, false);
+    } else {
+      if (impdiff) SNAC_KB(false, true);
+      else SNAC_KB(false, false);
+    }
+#undef SNAC_KB
+  });
+}
+void launch_fillps_blocks(hipStream_t s, const std::vector<FillBlock> &blk, int fa, double dtrk) {
+  in_batches<FillBlocks>(blk, [](const FillBlock &b) { return interior_tiles(b.g).x; },
+                         [&](const FillBlocks &A, unsigned n) {
+                           hipLaunchKernelGGL(k_fillps_blocks, dim3(n), dim3(TX, TY), 0, s, A, fa, 1.0 / dtrk);
+                         });
+}
+void launch_correc_blocks(hipStream_t s, const std::vector<CorBlock> &blk, double dtrk) {
+  in_batches<CorBlocks>(blk, [](const CorBlock &b) { return ghosted_tiles(b.g).x; },
+                        [&](const CorBlocks &A, unsigned n) {
+                          hipLaunchKernelGGL(k_correc_blocks, dim3(n), dim3(TX, TY), 0, s, A, dtrk);
+                        });
+}
 void launch_fillps(hipStream_t s, const Geo &g, const Metrics &m, int fa, const double *u, const double *v,
                    const double *w, double *pp, double dtrk, const double *const r[6]) {
   hipLaunchKernelGGL(k_fillps, interior_tiles(g), dim3(TX, TY), 0, s, g, m, fa, u, v, w, pp, 1.0 / dtrk, r[0], r[1], r[2],
