@@ -202,7 +202,8 @@ void launch_face_ops(hipStream_t s, const FaceOp *dev_ops, int nops, int max_pla
 // from r2r_table(); mat: dense n x n matrix (row = output) or null.
 struct R2RPlan {
   int n = 0, kind = 0;
-  bool fft = false;        // LDS FFT path (n a power of two >= 4, supported kind)
+  bool fft = false;        // LDS FFT path (n a power of two >= 4, supported kind; or mixed)
+  bool mixed = false;      // R2HC/HC2R of a length 2 N1 N2 with factors 3 and 5 (tiles 0, 1)
   bool mfma = false;       // matrix product on the matrix cores (tab: its fragments)
   int lshift = 0;          // FFT tile (autotuned): 0..2 lines per workgroup = max >> lshift;
                            // 3, 4 (R2HC/HC2R): full tiles, 2 / 4 per workgroup, pipelined

@@ -100,6 +100,91 @@ __device__ __forceinline__ void fft_reg(double2 (&v)[N], const double2 *__restri
   }
 }
 
+// R-point DFT in registers for the odd factors of the mixed-radix lengths
+// (y_q = sum_r x_r e^{-2 pi i r q/R}, conjugated when inv)
+template <int R>
+__device__ __forceinline__ void dft_prime(double2 (&x)[R], bool inv) {
+  const double sg = inv ? -1.0 : 1.0;
+  if constexpr (R == 2) {
+    const double2 a = x[0], b = x[1];
+    x[0] = make_double2(a.x + b.x, a.y + b.y);
+    x[1] = make_double2(a.x - b.x, a.y - b.y);
+  } else if constexpr (R == 3) {
+    const double s3 = sg * 0.86602540378443864676;  // sin(2 pi/3)
+    const double2 t = make_double2(x[1].x + x[2].x, x[1].y + x[2].y);
+    const double2 d = make_double2(s3 * (x[1].x - x[2].x), s3 * (x[1].y - x[2].y));
+    const double2 m = make_double2(x[0].x - 0.5 * t.x, x[0].y - 0.5 * t.y);
+    x[0] = make_double2(x[0].x + t.x, x[0].y + t.y);
+    x[1] = make_double2(m.x + d.y, m.y - d.x);
+    x[2] = make_double2(m.x - d.y, m.y + d.x);
+  } else {
+    static_assert(R == 5, "factors 2, 3 and 5");
+    const double c1 = 0.30901699437494742410, c2 = -0.80901699437494742410;        // cos(2 pi/5), cos(4 pi/5)
+    const double s1 = sg * 0.95105651629515357212, s2 = sg * 0.58778525229247312917;  // sin(2 pi/5), sin(4 pi/5)
+    const double2 p1 = make_double2(x[1].x + x[4].x, x[1].y + x[4].y), q1 = make_double2(x[1].x - x[4].x, x[1].y - x[4].y);
+    const double2 p2 = make_double2(x[2].x + x[3].x, x[2].y + x[3].y), q2 = make_double2(x[2].x - x[3].x, x[2].y - x[3].y);
+    const double2 m1 = make_double2(x[0].x + c1 * p1.x + c2 * p2.x, x[0].y + c1 * p1.y + c2 * p2.y);
+    const double2 m2 = make_double2(x[0].x + c2 * p1.x + c1 * p2.x, x[0].y + c2 * p1.y + c1 * p2.y);
+    const double2 d1 = make_double2(s1 * q1.x + s2 * q2.x, s1 * q1.y + s2 * q2.y);
+    const double2 d2 = make_double2(s2 * q1.x - s1 * q2.x, s2 * q1.y - s1 * q2.y);
+    x[0] = make_double2(x[0].x + p1.x + p2.x, x[0].y + p1.y + p2.y);
+    x[1] = make_double2(m1.x + d1.y, m1.y - d1.x);
+    x[4] = make_double2(m1.x - d1.y, m1.y + d1.x);
+    x[2] = make_double2(m2.x + d2.y, m2.y - d2.x);
+    x[3] = make_double2(m2.x - d2.y, m2.y + d2.x);
+  }
+}
+// N points of v, S apart from element O on, transformed into out (natural
+// order): N = R M, M-point transforms of every R-th point, twiddles, R-point
+// transforms across them.  Everything unrolls to registers; tw as in fft_reg.
+template <int N, int O, int S, int NV>
+__device__ __forceinline__ void dft_mixed(const double2 (&v)[NV], double2 (&out)[N], const double2 *__restrict__ tw,
+                                          int stride, bool inv) {
+  if constexpr (N == 1) {
+    out[0] = v[O];
+  } else {
+    constexpr int R = N % 5 == 0 ? 5 : (N % 3 == 0 ? 3 : 2), M = N / R;
+    double2 part[R][M];
+    if constexpr (R >= 2) {
+      dft_mixed<M, O, S * R, NV>(v, part[0], tw, stride * R, inv);
+      dft_mixed<M, O + S, S * R, NV>(v, part[1], tw, stride * R, inv);
+    }
+    if constexpr (R >= 3) dft_mixed<M, O + 2 * S, S * R, NV>(v, part[2], tw, stride * R, inv);
+    if constexpr (R >= 5) {
+      dft_mixed<M, O + 3 * S, S * R, NV>(v, part[3], tw, stride * R, inv);
+      dft_mixed<M, O + 4 * S, S * R, NV>(v, part[4], tw, stride * R, inv);
+    }
+#pragma unroll
+    for (int k = 0; k < M; k++) {
+      double2 x[R];
+#pragma unroll
+      for (int r = 0; r < R; r++) {
+        x[r] = part[r][k];
+        if (r * k != 0) {
+          double2 w = tw[r * k * stride];
+          if (inv) w.y = -w.y;
+          x[r] = make_double2(part[r][k].x * w.x - part[r][k].y * w.y, part[r][k].x * w.y + part[r][k].y * w.x);
+        }
+      }
+      dft_prime<R>(x, inv);
+#pragma unroll
+      for (int q = 0; q < R; q++) out[k + M * q] = x[q];
+    }
+  }
+}
+// the register DFT of either kind of length, in place
+template <int N>
+__device__ __forceinline__ void fft_any(double2 (&v)[N], const double2 *__restrict__ tw, int stride, bool inv) {
+  if constexpr ((N & (N - 1)) == 0) {
+    fft_reg<N>(v, tw, stride, inv);
+  } else {
+    double2 out[N];
+    dft_mixed<N, 0, 1, N>(v, out, tw, stride, inv);
+#pragma unroll
+    for (int i = 0; i < N; i++) v[i] = out[i];
+  }
+}
+
 // complex input slot s of the n-point sequence for KIND, from the raw line r
 // (raw index n maps to zero where the kind needs x_n).  tk[k] = (cos, sin)(pi k / 2n).
 template <int KIND>
@@ -406,10 +491,10 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(N1 < N2 ? 4 
           v[j1] = make_double2(xk.x + xc.x - by, xk.y + xc.y + bx);        // A + i B
         }
       }
-      fft_reg<N1>(v, tw, 2 * N2, INV);
+      fft_any<N1>(v, tw, 2 * N2, INV);
 #pragma unroll
       for (int k1 = 1; k1 < N1; k1++) {
-        double2 w = tw[(2 * j2 * k1) & (n - 1)];
+        double2 w = tw[2 * j2 * k1];  // 2 j2 k1 < n
         if (INV) w.y = -w.y;
         double2 y = v[k1];
         v[k1] = make_double2(y.x * w.x - y.y * w.y, y.x * w.y + y.y * w.x);
@@ -453,7 +538,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(N1 < N2 ? 4 
       double y;
       if (!INV) {
         const int k = q <= h ? q : n - q;
-        const double2 zk = Z[k & (h - 1)], zc = Z[(h - k) & (h - 1)];  // Z[k], Z[h-k] (mod h)
+        const double2 zk = Z[k < h ? k : 0], zc = Z[k > 0 ? h - k : 0];  // Z[k], Z[h-k] (mod h)
         const double ex = 0.5 * (zk.x + zc.x), ey = 0.5 * (zk.y - zc.y);
         const double ox = 0.5 * (zk.y + zc.y), oy = -0.5 * (zk.x - zc.x);
         const double2 w = tw[k];
@@ -595,9 +680,9 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void k_
 // TFLOP/s measured on a large product) against 16 bytes per point; at n = 192
 // the folded product takes about as long as the memory does.  The form it
 // replaces walked a matrix row per thread (8-byte loads a row apart): 347 us
-// on average over the transforms of a 192x96x96 box, 17-22 us now (1.6 TB/s
-// of the lines' bytes); 146 -> 12-17 us for a 180x77x90 channel's, 8.1 -> 3.4
-// us for two-point lines.
+// on average over the transforms of a 192x96x96 box, 16-26 us this way; 146 ->
+// 12-18 us for a 180x77x90 channel's (0.8 TB/s of the lines' bytes), 8.1 ->
+// 3.4 us for two-point lines.
 typedef double double4_ __attribute__((ext_vector_type(4)));
 struct MJob {  // one batch of lines and its first workgroup
   const double *in;
@@ -910,6 +995,44 @@ void launch_rfft_swapped(bool inv, bool wave, dim3 grid, size_t lds, hipStream_t
   }
 }
 
+// Mixed-radix lengths n = 2 N1 N2 (N1 with factors 3 and 5, N2 a power of two):
+// the same kernel; the split of each length, or false.  From n = 72 on: there
+// the matrix product's 2 n^2 operations a line take longer than its memory
+// traffic (a 192x96x96 box: 96-point lines 16 -> 12-14 us, 192-point lines
+// 23-26 -> 12-15 us); at 48 points both take 8 us, and the product takes
+// several grid blocks in one launch.
+bool rfft_mixed_split(int n, int &n1, int &n2) {
+  static const int t[][3] = {{72, 9, 4},   {80, 5, 8},   {96, 6, 8},    {120, 15, 4},  {144, 9, 8},  {160, 10, 8},
+                             {192, 12, 8}, {240, 15, 8}, {288, 9, 16}, {320, 10, 16}, {384, 12, 16}, {480, 15, 16}};
+  for (auto &e : t)
+    if (e[0] == n) {
+      n1 = e[1];
+      n2 = e[2];
+      return true;
+    }
+  return false;
+}
+template <int N1, int N2>
+void launch_rfft_mixed_sized(bool inv, int ls, dim3 grid, size_t lds, hipStream_t s, const Args &a) {
+  if (ls == 0) {
+    if (inv) hipLaunchKernelGGL((k_rfft<N1, N2, true, 0, 1>), grid, dim3(NT), lds, s, a);
+    else hipLaunchKernelGGL((k_rfft<N1, N2, false, 0, 1>), grid, dim3(NT), lds, s, a);
+  } else {
+    if (inv) hipLaunchKernelGGL((k_rfft<N1, N2, true, 1, 1>), grid, dim3(NT), lds, s, a);
+    else hipLaunchKernelGGL((k_rfft<N1, N2, false, 1, 1>), grid, dim3(NT), lds, s, a);
+  }
+}
+void launch_rfft_mixed(bool inv, int n, int ls, dim3 grid, size_t lds, hipStream_t s, const Args &a) {
+#define SNAC_MX(N, A, B) case N: launch_rfft_mixed_sized<A, B>(inv, ls, grid, lds, s, a); break;
+  switch (n) {
+    SNAC_MX(72, 9, 4) SNAC_MX(80, 5, 8)
+    SNAC_MX(96, 6, 8) SNAC_MX(120, 15, 4) SNAC_MX(144, 9, 8) SNAC_MX(160, 10, 8) SNAC_MX(192, 12, 8)
+    SNAC_MX(240, 15, 8) SNAC_MX(288, 9, 16) SNAC_MX(320, 10, 16) SNAC_MX(384, 12, 16) SNAC_MX(480, 15, 16)
+    default: throw std::runtime_error("r2r: no mixed-radix path for length " + std::to_string(n));
+  }
+#undef SNAC_MX
+}
+
 // h-point split of an n = 2h point real transform
 void launch_rfft(bool inv, int n, int ls, dim3 grid, size_t lds, hipStream_t s, const Args &a) {
   const bool sw = ls == 6 || ls == 7, wv = ls == 7;
@@ -1110,6 +1233,7 @@ double r2r_coef(int kind, int n, int k, int j) {
 
 int r2r_tile_choices(const R2RPlan &pl) {
   if (!pl.fft) return 1;
+  if (pl.mixed) return 2;
   return (pl.kind == K_R2HC || pl.kind == K_HC2R) && pl.n >= 8 ? 8 : 3;
 }
 
@@ -1123,6 +1247,8 @@ R2RPlan r2r_plan(int kind, int n, bool rowwise) {
   pl.n = n;
   pl.kind = kind;
   pl.fft = fft_kind(kind) && n >= 4 && (n & (n - 1)) == 0 && n <= 1024;
+  int m1, m2;
+  if (!rowwise && (kind == K_R2HC || kind == K_HC2R) && rfft_mixed_split(n, m1, m2)) pl.fft = pl.mixed = true;
   std::vector<double> h;
   const double pi = std::acos(-1.0);
   if (pl.fft) {
@@ -1167,7 +1293,16 @@ void launch_r2r(hipStream_t s, const R2RPlan &pl, const double *in, long ies, lo
   a.nlines = nb1 * nb2;
   a.coal = (ies != 1) ? 1 : 0;
   if (a.nlines <= 0) return;
-  if (pl.fft && (pl.kind == K_R2HC || pl.kind == K_HC2R) && pl.n >= 8) {
+  if (pl.mixed) {
+    int n1 = 0, n2 = 0;
+    rfft_mixed_split(pl.n, n1, n2);
+    const int ls = pl.lshift == 1 ? 1 : 0, L = std::max(1, rfft_lines(n1, n2) >> ls);
+    a.L = L;
+    a.scale = scale;
+    a.tab = pl.tab;
+    launch_rfft_mixed(pl.kind == K_HC2R, pl.n, ls, dim3((unsigned)((a.nlines + L - 1) / L)),
+                      (size_t)L * (pl.n + RPAD) * sizeof(double), s, a);
+  } else if (pl.fft && (pl.kind == K_R2HC || pl.kind == K_HC2R) && pl.n >= 8) {
     int n1 = 0, n2 = 0;
     fft_split(pl.n / 2, n1, n2);
     const int ls = pl.lshift <= 2 ? pl.lshift : 0, tpb = rfft_tpb(pl.lshift);

@@ -40,7 +40,7 @@ def matrix(kind, n):
     return 2 * sin((j + 1) * (k + 1), n + 1)
 
 
-def check(ctx, kind, n, howmany):
+def check(ctx, kind, n, howmany, tile=0):
     M = matrix(kind, n)
     x = np.random.default_rng(n + howmany).uniform(-1, 1, (howmany, n))
     x[howmany // 2] = 0.0
@@ -52,7 +52,7 @@ def check(ctx, kind, n, howmany):
     tol = (n + 4) * u * (np.abs(x) @ np.abs(M).astype(np.float64).T) + 16 * u * np.abs(x).sum(1)[:, None]
     tol *= 1 if howmany < 1000 else 2
     for strided in (False, True):
-        y = ctx.r2r_lines(kind, x, strided=strided)
+        y = ctx.r2r_lines(kind, x, strided=strided, tile=tile)
         assert (np.abs(y - ref) <= tol).all(), (kind, n, strided, float(np.abs(y - ref).max()))
         assert not y[howmany // 2].any()
 
@@ -71,7 +71,15 @@ def test_matrix_lines(ctx, kind, n):
     check(ctx, kind, n, 37)
 
 
+@pytest.mark.parametrize("kind", ["R2HC", "HC2R"])
+@pytest.mark.parametrize("n", [48, 72, 80, 96, 120, 144, 160, 192, 240, 288, 320, 384, 480])
+def test_mixed_radix_lines(ctx, kind, n):
+    """The lengths with factors 3 and 5 that have an FFT, both tiles."""
+    for tile in (0, 1):
+        check(ctx, kind, n, 75, tile)
+
+
 @pytest.mark.parametrize("kind", ["R2HC", "HC2R", "REDFT11"])
-@pytest.mark.parametrize("n", [48, 2])
+@pytest.mark.parametrize("n", [42, 2])
 def test_many_lines(ctx, kind, n):
     check(ctx, kind, n, 16384 * 4 + 21)
