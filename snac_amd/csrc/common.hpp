@@ -184,6 +184,9 @@ struct ImpRhs {
 // out (ghosted, same layout as phi) = phi*alphai*w0*w1*w2 + BC planes over
 // the unknowns, 0 past them
 void launch_imp_rhs(hipStream_t s, const Geo &g, const ImpRhs &r, const double *phi, double *out, double alphai);
+// the same of the three velocity components in one launch
+void launch_imp_rhs3(hipStream_t s, const Geo &g, const ImpRhs *const r[3], const double *const phi[3],
+                     double *const out[3], double alphai);
 // dst = src over the unknowns (indices 1..ext of each axis) of a block
 void launch_copy_unknowns(hipStream_t s, const Geo &g, const int ext[3], const double *src, double *dst);
 // updt_pressure of the _IMPDIFF build: p += pp + alpha * Laplacian(pp)
@@ -218,8 +221,10 @@ R2RPlan r2r_plan(int kind, int n, bool rowwise = false);
 int r2r_tile_choices(const R2RPlan &pl);  // number of tile choices of the plan's kernel
 void launch_r2r(hipStream_t s, const R2RPlan &pl, const double *in, long ies, long is1, long is2,
                 double *out, long oes, long os1, long os2, int nb1, int nb2, double scale);
-// several line batches of one plan (one per grid block): one launch where the
-// plan is a matrix product, else one after the other
+// several line batches of one plan (one per grid block or field): one launch
+// for up to GRID_BLOCKS where the plan is a matrix product, for up to
+// R2R_FIELDS of the same extents and strides where it is an FFT
+constexpr int R2R_FIELDS = 4;
 struct R2RJob {
   const double *in;
   long ies, is1, is2;
@@ -253,6 +258,10 @@ struct TridiagLine {
 // dscratch (d') and cscratch (c', used only for lines longer than the LDS
 // budget) have the size and layout of x
 void launch_tridiag(hipStream_t st, const TridiagLine &t, double *x, double *dscratch, double *cscratch);
+// the line solves of up to TRIDIAG_FIELDS operators of one grid (the same G, s
+// and variant 2 or 3) in one launch, operator q on x[q]
+constexpr int TRIDIAG_FIELDS = 3;
+void launch_tridiag_fields(hipStream_t st, const TridiagLine *t, double *const *x, int n);
 // chunks per line of variant 2 (fine: variant 3) for lines of length m
 // (0: not available)
 int tridiag_chunks(int m, bool fine = false);

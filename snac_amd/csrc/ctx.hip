@@ -564,7 +564,7 @@ void stage_inplace(snac_ctx *c, const TensorOps &o, size_t q, bool fwd) {
              t.G[b1], t.G[b2], fwd ? 1.0 : o.norm[q]);
 }
 
-void stage_tridiag(snac_ctx *c, const TensorOps &o, double shift) {
+TridiagLine tridiag_line(snac_ctx *c, const TensorOps &o, double shift) {
   TensorPlan &t = c->tp;
   TridiagLine tl;
   for (int q = 0; q < 3; q++) tl.G[q] = t.G[q];
@@ -576,7 +576,12 @@ void stage_tridiag(snac_ctx *c, const TensorOps &o, double shift) {
   tl.lamB = o.lam[o2];
   tl.pin_when_zero = o.pin;
   tl.shift = shift;
-  launch_tridiag(c->stream, tl, t.ph, t.scratch, t.scratch2);
+  return tl;
+}
+
+void stage_tridiag(snac_ctx *c, const TensorOps &o, double shift) {
+  TensorPlan &t = c->tp;
+  launch_tridiag(c->stream, tridiag_line(c, o, shift), t.ph, t.scratch, t.scratch2);
 }
 
 // the current buffer of field comp of a Helmholtz solve (velocity
@@ -714,6 +719,90 @@ void plan_impdiff(snac_ctx *c) {
   if (forced)
     for (auto &D : c->blk)
       if (!D.sdd) D.sdd = dalloc<double>(c, D.nin);
+}
+
+// The Helmholtz problems of u, v and w on the tensor-product plan side by
+// side: the three right-hand sides (in the other velocity buffers, free until
+// correc writes them), transforms and line solves each in one launch per
+// stage.  At a million cells a stage of one component is bound by its launch
+// and its first loads.  Needs the components to share their transforms (a
+// channel's do; a component staggered along a bounded transformed axis has
+// n - 1 points there), the chunked line solve, whose scratch arrays are then
+// free to hold the second and third component, and a grid whose planes the
+// launch can count three times.
+bool impdiff_together(snac_ctx *c) {
+  const TensorPlan &t = c->tp;
+  if (use_mg(c) || !t.ok || t.tvariant < 2 || c->imp.size() < 3) return false;
+  if (tridiag_chunks(t.G[t.s], t.tvariant == 3) == 0) return false;
+  for (auto &D : c->blk)
+    if (D.g.nz > 65535 / 3) return false;
+  const TensorOps &a = c->imp[0].ops;
+  for (int comp = 1; comp < 3; comp++) {
+    const TensorOps &b = c->imp[comp].ops;
+    for (size_t q = 0; q < t.xaxes.size(); q++)
+      if (a.fwd[q].kind != b.fwd[q].kind || a.fwd[q].n != b.fwd[q].n || a.bwd[q].kind != b.bwd[q].kind ||
+          a.bwd[q].n != b.bwd[q].n)
+        return false;
+  }
+  return true;
+}
+
+void solve_impdiff_uvw(snac_ctx *c, double alpha) {
+  TensorPlan &t = c->tp;
+  const double alphai = 1.0 / alpha;
+  Phase tp(c, SNAC_PH_HELMHOLTZ);
+  double *ph[3] = {t.ph, t.scratch, t.scratch2};
+  const int nx = 1 - c->cur;
+  for (size_t b = 0; b < c->blk.size(); b++) {
+    DevBlock &D = c->blk[b];
+    const ImpRhs *r[3] = {&c->imp[0].rhs[b], &c->imp[1].rhs[b], &c->imp[2].rhs[b]};
+    const double *phi[3] = {D.vel[c->cur][0], D.vel[c->cur][1], D.vel[c->cur][2]};
+    launch_imp_rhs3(c->stream, D.g, r, phi, D.vel[nx], alphai);
+  }
+  const long pst[3] = {1, (long)t.G[0], (long)t.G[0] * t.G[1]};
+  auto axis = [&](size_t q, int &a, int &b1, int &b2) {
+    a = t.xaxes[q];
+    others(a, b1, b2);
+  };
+  // the first (last) transform runs block by block from (into) the fields
+  auto ends = [&](bool fwd) {
+    int a, b1, b2;
+    axis(0, a, b1, b2);
+    for (size_t b = 0; b < c->blk.size(); b++) {
+      DevBlock &D = c->blk[b];
+      const Block &B = c->cs.blocks[b];
+      long off = 0;
+      for (int q = 0; q < 3; q++) off += (long)(B.lo_g[q] - t.gmin[q]) * pst[q];
+      std::vector<R2RJob> jobs;
+      for (int q = 0; q < 3; q++) {
+        double *f = D.vel[fwd ? nx : c->cur][q] + 1 + D.g.sx + D.g.sx * D.g.sy;
+        if (fwd)
+          jobs.push_back(R2RJob{f, gstride(D, a), gstride(D, b1), gstride(D, b2), ph[q] + off, pst[a], pst[b1],
+                                pst[b2], bext(D, b1), bext(D, b2)});
+        else
+          jobs.push_back(R2RJob{ph[q] + off, pst[a], pst[b1], pst[b2], f, gstride(D, a), gstride(D, b1),
+                                gstride(D, b2), bext(D, b1), bext(D, b2)});
+      }
+      const TensorOps &o = c->imp[0].ops;
+      launch_r2r_jobs(c->stream, fwd ? o.fwd[0] : o.bwd[0], jobs, fwd ? 1.0 : o.norm[0]);
+    }
+  };
+  auto inner = [&](size_t q, bool fwd) {
+    int a, b1, b2;
+    axis(q, a, b1, b2);
+    std::vector<R2RJob> jobs;
+    for (int f = 0; f < 3; f++)
+      jobs.push_back(R2RJob{ph[f], pst[a], pst[b1], pst[b2], ph[f], pst[a], pst[b1], pst[b2], t.G[b1], t.G[b2]});
+    const TensorOps &o = c->imp[0].ops;
+    launch_r2r_jobs(c->stream, fwd ? o.fwd[q] : o.bwd[q], jobs, fwd ? 1.0 : o.norm[q]);
+  };
+  ends(true);
+  for (size_t q = 1; q < t.xaxes.size(); q++) inner(q, true);
+  TridiagLine tl[3];
+  for (int f = 0; f < 3; f++) tl[f] = tridiag_line(c, c->imp[f].ops, alphai);
+  launch_tridiag_fields(c->stream, tl, ph, 3);
+  for (size_t q = t.xaxes.size() - 1; q >= 1; q--) inner(q, false);
+  ends(false);
 }
 
 void mg_stage_in(snac_ctx *c, MGPlan &P);
@@ -1068,8 +1157,11 @@ void substage(snac_ctx *c, int irk, double dt) {
   }
   { Phase t(c, SNAC_PH_RK_MOM); rk_mom(c, irk, dt); }
   const double alpha = -c->cs.visc * dtrk / 2.0;  // main.f90:935
-  if (c->impdiff)  // main.f90:947-997
-    for (int comp = 0; comp < 3; comp++) solve_impdiff(c, comp, alpha);
+  if (c->impdiff) {  // main.f90:947-997
+    if (impdiff_together(c)) solve_impdiff_uvw(c, alpha);
+    else
+      for (int comp = 0; comp < 3; comp++) solve_impdiff(c, comp, alpha);
+  }
   { Phase t(c, SNAC_PH_BOUND); run_program(c, c->prog_uvw[c->cur][0]); }  // bounduvw + inflow
   { Phase t(c, SNAC_PH_FILLPS); fillps(c, dtrk); }
   solve_pressure(c);

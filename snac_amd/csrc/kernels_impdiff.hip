@@ -14,11 +14,10 @@ constexpr int TX = 64, TY = 4;
 // planes of the bounded faces in updt_rhs's order (x lo, x hi, y lo, ...);
 // 0 at the cells past the unknowns (the bounded upper face of a staggered
 // component), which the solve keeps decoupled
-__global__ __launch_bounds__(TX *TY) void k_imp_rhs(Geo g, ImpRhs r, const double *__restrict__ phi,
-                                                    double *__restrict__ out, double alphai) {
+__device__ __forceinline__ void imp_rhs_cell(const Geo &g, const ImpRhs &r, const double *__restrict__ phi,
+                                             double *__restrict__ out, double alphai, int k) {
   const int i = blockIdx.x * TX + threadIdx.x + 1;
   const int j = blockIdx.y * TY + threadIdx.y + 1;
-  const int k = blockIdx.z + 1;
   if (i > g.nx || j > g.ny) return;
   const long c = i + g.sx * (j + g.sy * (long)k);
   if (i > r.ext[0] || j > r.ext[1] || k > r.ext[2]) {
@@ -37,6 +36,21 @@ __global__ __launch_bounds__(TX *TY) void k_imp_rhs(Geo g, ImpRhs r, const doubl
   if (k == 1 && r.plane[2][0]) v = v + r.plane[2][0][(i - 1) + (long)e0 * (j - 1)];
   if (k == r.ext[2] && r.plane[2][1]) v = v + r.plane[2][1][(i - 1) + (long)e0 * (j - 1)];
   out[c] = v;
+}
+__global__ __launch_bounds__(TX *TY) void k_imp_rhs(Geo g, ImpRhs r, const double *__restrict__ phi,
+                                                    double *__restrict__ out, double alphai) {
+  imp_rhs_cell(g, r, phi, out, alphai, blockIdx.z + 1);
+}
+
+// the three velocity components, nz planes each
+struct ImpRhs3 {
+  ImpRhs r[3];
+  const double *phi[3];
+  double *out[3];
+};
+__global__ __launch_bounds__(TX *TY) void k_imp_rhs3(Geo g, ImpRhs3 a, double alphai) {
+  const int c = blockIdx.z / g.nz;
+  imp_rhs_cell(g, a.r[c], a.phi[c], a.out[c], alphai, blockIdx.z - c * g.nz + 1);
 }
 
 // p += pp, then p += alpha * (Laplacian of pp) (the reference's two loops)
@@ -73,6 +87,20 @@ dim3 interior_grid(const Geo &g) { return dim3((g.nx + TX - 1) / TX, (g.ny + TY 
 
 void launch_imp_rhs(hipStream_t s, const Geo &g, const ImpRhs &r, const double *phi, double *out, double alphai) {
   hipLaunchKernelGGL(k_imp_rhs, interior_grid(g), dim3(TX, TY), 0, s, g, r, phi, out, alphai);
+  SNAC_HIP(hipGetLastError());
+}
+
+void launch_imp_rhs3(hipStream_t s, const Geo &g, const ImpRhs *const r[3], const double *const phi[3],
+                     double *const out[3], double alphai) {
+  ImpRhs3 a;
+  for (int c = 0; c < 3; c++) {
+    a.r[c] = *r[c];
+    a.phi[c] = phi[c];
+    a.out[c] = out[c];
+  }
+  dim3 grid = interior_grid(g);
+  grid.z *= 3;
+  hipLaunchKernelGGL(k_imp_rhs3, grid, dim3(TX, TY), 0, s, g, a, alphai);
   SNAC_HIP(hipGetLastError());
 }
 

@@ -37,7 +37,23 @@ struct Args {
   int coal;  // 1: consecutive threads walk the batch index (line stride != 1)
   double scale;
   const double *tab;
+  // lines of several fields in one launch (nlines counts them all): nf lines
+  // each, field f at element offsets fin[f] / fout[f] from in / out
+  int nf;
+  long fin[R2R_FIELDS], fout[R2R_FIELDS];
 };
+
+// input and output offsets of a line (-1: past the last)
+__device__ __forceinline__ void line_offset(const Args &a, int line, long &oi, long &oo) {
+  oi = oo = -1;
+  if (line >= a.nlines) return;
+  int f = 0;
+#pragma unroll
+  for (int e = 1; e < R2R_FIELDS; e++) f += line >= e * a.nf;
+  const int q = line - f * a.nf, b1 = q % a.nb1, b2 = q / a.nb1;
+  oi = a.fin[f] + b1 * a.is1 + b2 * a.is2;
+  oo = a.fout[f] + b1 * a.os1 + b2 * a.os2;
+}
 
 // lines per workgroup for an N1 x N2 FFT: one task per thread in each pass
 // and at most LDS_COMPLEX complex values of LDS
@@ -53,12 +69,8 @@ template <int L>
 __device__ __forceinline__ void line_offsets(const Args &a, int line0, long (&oin)[L], long (&oout)[L]) {
   for (int t = threadIdx.x; t < L; t += NT) {
     const int line = line0 + t;
-    long oi = -1, oo = -1;
-    if (line < a.nlines) {
-      const int b1 = line % a.nb1, b2 = line / a.nb1;
-      oi = b1 * a.is1 + b2 * a.is2;
-      oo = b1 * a.os1 + b2 * a.os2;
-    }
+    long oi, oo;
+    line_offset(a, line, oi, oo);
     oin[t] = oi;
     oout[t] = oo;
   }
@@ -429,12 +441,8 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(N1 < N2 ? 4 
   auto offsets = [&](int slot, int tile) {
     for (int t = threadIdx.x; t < L; t += NT) {
       const int line = tile * L + t;
-      long oi = -1, oo = -1;
-      if (line < a.nlines) {
-        const int b1 = line % a.nb1, b2 = line / a.nb1;
-        oi = b1 * a.is1 + b2 * a.is2;
-        oo = b1 * a.os1 + b2 * a.os2;
-      }
+      long oi, oo;
+      line_offset(a, line, oi, oo);
       oin[slot][t] = oi;
       oout[slot][t] = oo;
     }
@@ -587,12 +595,8 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void k_
   const int wv = threadIdx.x >> 6, ln = threadIdx.x & 63;
   for (int t = threadIdx.x; t < L; t += NT) {
     const int line = blockIdx.x * L + t;
-    long oi = -1, oo = -1;
-    if (line < a.nlines) {
-      const int b1 = line % a.nb1, b2 = line / a.nb1;
-      oi = b1 * a.is1 + b2 * a.is2;
-      oo = b1 * a.os1 + b2 * a.os2;
-    }
+    long oi, oo;
+    line_offset(a, line, oi, oo);
     oin[t] = oi;
     oout[t] = oo;
   }
@@ -1281,17 +1285,34 @@ R2RPlan r2r_plan(int kind, int n, bool rowwise) {
   return pl;
 }
 
-void launch_r2r(hipStream_t s, const R2RPlan &pl, const double *in, long ies, long is1, long is2, double *out,
-                long oes, long os1, long os2, int nb1, int nb2, double scale) {
+namespace {
+// the jobs of one plan in one launch (matrix products: any, up to
+// GRID_BLOCKS; else the same extents and strides, up to R2R_FIELDS)
+void launch_jobs(hipStream_t s, const R2RPlan &pl, const R2RJob *jobs, int njob, double scale) {
+  if (pl.mfma) {
+    launch_mfma(s, pl.kind, pl.n, jobs, njob, scale, pl.tab);
+    SNAC_HIP(hipGetLastError());
+    return;
+  }
+  const R2RJob &j0 = jobs[0];
   Args a;
-  a.in = in; a.out = out;
-  a.ies = ies; a.is1 = is1; a.is2 = is2; a.oes = oes; a.os1 = os1; a.os2 = os2;
+  a.in = j0.in; a.out = j0.out;
+  for (int f = 0; f < njob; f++) {
+    a.in = std::min(a.in, jobs[f].in);
+    a.out = std::min(a.out, jobs[f].out);
+  }
+  for (int f = 0; f < R2R_FIELDS; f++) {
+    a.fin[f] = f < njob ? jobs[f].in - a.in : 0;
+    a.fout[f] = f < njob ? jobs[f].out - a.out : 0;
+  }
+  a.ies = j0.ies; a.is1 = j0.is1; a.is2 = j0.is2; a.oes = j0.oes; a.os1 = j0.os1; a.os2 = j0.os2;
   a.n = pl.n;
   a.logn = 0;
   while ((1 << a.logn) < pl.n) a.logn++;
-  a.nb1 = nb1;
-  a.nlines = nb1 * nb2;
-  a.coal = (ies != 1) ? 1 : 0;
+  a.nb1 = j0.nb1;
+  a.nf = j0.nb1 * j0.nb2;
+  a.nlines = a.nf * njob;
+  a.coal = (a.ies != 1) ? 1 : 0;
   if (a.nlines <= 0) return;
   if (pl.mixed) {
     int n1 = 0, n2 = 0;
@@ -1325,9 +1346,6 @@ void launch_r2r(hipStream_t s, const R2RPlan &pl, const double *in, long ies, lo
     dim3 grid((unsigned)((a.nlines + L - 1) / L));
     size_t lds = (size_t)L * pl.n * sizeof(double2);
     launch_fft_kind(pl.kind, pl.n, ls, grid, lds, s, a);
-  } else if (pl.mfma) {
-    const R2RJob j{in, ies, is1, is2, out, oes, os1, os2, nb1, nb2};
-    launch_mfma(s, pl.kind, pl.n, &j, 1, scale, pl.tab);
   } else {
     int L = std::max(1, std::min(2 * LDS_COMPLEX / pl.n, a.nlines));
     a.L = L;
@@ -1340,16 +1358,27 @@ void launch_r2r(hipStream_t s, const R2RPlan &pl, const double *in, long ies, lo
   SNAC_HIP(hipGetLastError());
 }
 
+}  // namespace
+
+void launch_r2r(hipStream_t s, const R2RPlan &pl, const double *in, long ies, long is1, long is2, double *out,
+                long oes, long os1, long os2, int nb1, int nb2, double scale) {
+  const R2RJob j{in, ies, is1, is2, out, oes, os1, os2, nb1, nb2};
+  launch_jobs(s, pl, &j, 1, scale);
+}
+
 void launch_r2r_jobs(hipStream_t s, const R2RPlan &pl, const std::vector<R2RJob> &jobs, double scale) {
-  if (pl.mfma) {
-    for (size_t q = 0; q < jobs.size(); q += GRID_BLOCKS) {
-      launch_mfma(s, pl.kind, pl.n, &jobs[q], (int)std::min<size_t>(GRID_BLOCKS, jobs.size() - q), scale, pl.tab);
-      SNAC_HIP(hipGetLastError());
-    }
-    return;
+  auto alike = [](const R2RJob &x, const R2RJob &y) {
+    return x.ies == y.ies && x.is1 == y.is1 && x.is2 == y.is2 && x.oes == y.oes && x.os1 == y.os1 && x.os2 == y.os2 &&
+           x.nb1 == y.nb1 && x.nb2 == y.nb2;
+  };
+  // the dense kernel keeps its launch per batch of lines
+  const size_t most = pl.mfma ? GRID_BLOCKS : (pl.fft ? R2R_FIELDS : 1);
+  for (size_t q = 0; q < jobs.size();) {
+    size_t e = q + 1;
+    while (e < jobs.size() && e - q < most && (pl.mfma || alike(jobs[q], jobs[e]))) e++;
+    launch_jobs(s, pl, &jobs[q], (int)(e - q), scale);
+    q = e;
   }
-  for (const R2RJob &j : jobs)
-    launch_r2r(s, pl, j.in, j.ies, j.is1, j.is2, j.out, j.oes, j.os1, j.os2, j.nb1, j.nb2, scale);
 }
 
 }  // namespace snac

@@ -109,7 +109,7 @@ __global__ __launch_bounds__(WG) void k_tridiag(TridiagLine t, double *__restric
 // pin_when_zero take x = 0 on their last row; a zero pivot (the
 // all-periodic zero mode) gives 0.
 template <int NC, int K>
-__global__ __launch_bounds__(64 * NC) void k_tridiag_chunk(TridiagLine t, double *__restrict__ x, int base, int extra) {
+__device__ __forceinline__ void tridiag_chunk(const TridiagLine &t, double *__restrict__ x, int base, int extra) {
   constexpr int NR = 2 * NC;
   __shared__ double red[4 * NR * 64];  // [comp][row][lane]: a, b, c (then c'), d (then d', then x)
   // the chunk index is wave-uniform: scalar registers, scalar coefficient loads
@@ -209,6 +209,21 @@ __global__ __launch_bounds__(64 * NC) void k_tridiag_chunk(TridiagLine t, double
     if (j <= cnt - 2) xl[(p0 + j) * ss] = D[j] - A[j] * xp - C[j] * xq;
 }
 
+template <int NC, int K>
+__global__ __launch_bounds__(64 * NC) void k_tridiag_chunk(TridiagLine t, double *__restrict__ x, int base, int extra) {
+  tridiag_chunk<NC, K>(t, x, base, extra);
+}
+
+// blockIdx.y = operator: the three velocity components' Helmholtz lines
+struct TridiagFields {
+  TridiagLine t[TRIDIAG_FIELDS];
+  double *x[TRIDIAG_FIELDS];
+};
+template <int NC, int K>
+__global__ __launch_bounds__(64 * NC) void k_tridiag_fields(TridiagFields f, int base, int extra) {
+  tridiag_chunk<NC, K>(f.t[blockIdx.y], f.x[blockIdx.y], base, extra);
+}
+
 }  // namespace
 
 // chunk count for the chunked variant (0: not applicable to this length):
@@ -246,6 +261,32 @@ void launch_tridiag(hipStream_t st, const TridiagLine &t, double *x, double *dsc
     hipLaunchKernelGGL(k_tridiag<true>, grid, dim3(WG), 0, st, t, x, dscratch, cscratch);
   else
     hipLaunchKernelGGL(k_tridiag<false>, grid, dim3(WG), 0, st, t, x, dscratch, cscratch);
+  SNAC_HIP(hipGetLastError());
+}
+
+void launch_tridiag_fields(hipStream_t st, const TridiagLine *t, double *const *x, int n) {
+  const int s = t[0].s, m = t[0].G[s];
+  const int nc = tridiag_chunks(m, t[0].variant == 3);
+  if (nc == 0 || n < 1 || n > TRIDIAG_FIELDS) throw std::runtime_error("internal: no chunked line solve");
+  TridiagFields f{};
+  for (int q = 0; q < n; q++) {
+    f.t[q] = t[q];
+    f.x[q] = x[q];
+  }
+  const int o1 = s == 0 ? 1 : 0, o2 = s == 2 ? 1 : 2;
+  const long nlines = (long)t[0].G[o1] * t[0].G[o2];
+  const dim3 grid((unsigned)((nlines + 63) / 64), (unsigned)n);
+  const int base = m / nc, extra = m % nc;
+  const bool small = base + (extra ? 1 : 0) <= 9;
+#define SNAC_TF(NC)                                                                                             \
+  do {                                                                                                          \
+    if (small) hipLaunchKernelGGL((k_tridiag_fields<NC, 9>), grid, dim3(64 * NC), 0, st, f, base, extra);        \
+    else hipLaunchKernelGGL((k_tridiag_fields<NC, 17>), grid, dim3(64 * NC), 0, st, f, base, extra);             \
+  } while (0)
+  if (nc == 4) SNAC_TF(4);
+  else if (nc == 8) SNAC_TF(8);
+  else SNAC_TF(16);
+#undef SNAC_TF
   SNAC_HIP(hipGetLastError());
 }
 
