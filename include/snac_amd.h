@@ -299,7 +299,9 @@ enum {
   SNAC_PH_RK_SCAL = 7,  /* rk_scal + bulk forcing of the scalars            */
   SNAC_PH_HELMHOLTZ = 8, /* implicit diffusion: the three Helmholtz solves  */
   SNAC_PH_MG_LINE0 = 9, /* MG-PCG: each finest-level zebra colour sweep that
-                           reads its neighbour lines (inside SNAC_PH_TRIDIAG) */
+                           reads its neighbour lines, or each descent of both
+                           colours in one launch: either moves 1.5 vectors of
+                           the level (inside SNAC_PH_TRIDIAG)                 */
   SNAC_PH_MG_TAIL = 10, /* MG-PCG: each launch of the fused coarse end of the
                            V-cycle (inside SNAC_PH_TRIDIAG)                  */
   SNAC_PH_MG_UPDATE = 11, /* MG-PCG: each CG update pass (x += alpha p,

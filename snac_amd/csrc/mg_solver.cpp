@@ -711,6 +711,17 @@ void vcycle(MGPlan &P, MGHier<T> &H, hipStream_t st, size_t l) {
   // factored lines, unless a line kernel is forced
   const MGFacT<T> &F = H.fac[l];
   const bool fac = fac_in_use(F) && !L.coupled && mg_line_variant() < 0;
+  if constexpr (sizeof(T) == 8) {
+    if (fac && nc == 2 && !(l == 0 && P.smooth_only) && mg_pair_fits(L, F)) {
+      const bool mk = l == 0 && P.mark_line0;
+      if (mk) P.mark_line0(true);
+      mg_pair_down(st, L, F, b, H.bl[l + 1], P.done);
+      if (mk) P.mark_line0(false);
+      vcycle(P, H, st, l + 1);
+      mg_pair_up(st, L, F, x, b, H.xl[l + 1], P.done);
+      return;
+    }
+  }
   if (zero_first) mg_zero(st, (long)L.nm * L.na * L.ns, x);
   for (int k = 0; k < nc; k++) {
     const int znb = (!zero_first && k == 0) ? 1 : 0;
