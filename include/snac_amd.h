@@ -301,7 +301,8 @@ enum {
   SNAC_PH_MG_LINE0 = 9, /* MG-PCG: each finest-level zebra colour sweep that
                            reads its neighbour lines, or each descent of both
                            colours in one launch: either moves 1.5 vectors of
-                           the level (inside SNAC_PH_TRIDIAG)                 */
+                           the level, the FP32 descent 2 (inside
+                           SNAC_PH_TRIDIAG)                                   */
   SNAC_PH_MG_TAIL = 10, /* MG-PCG: each launch of the fused coarse end of the
                            V-cycle (inside SNAC_PH_TRIDIAG)                  */
   SNAC_PH_MG_UPDATE = 11, /* MG-PCG: each CG update pass (x += alpha p,
@@ -330,7 +331,8 @@ int snac_get_timing(snac_ctx *ctx, double *ms, int *count);
  * counterpart in the reference (its FFTW plans use FFTW_ESTIMATE).          */
 int snac_get_autotune(snac_ctx *ctx, int *choices, double *ms, int n);
 /* the MG-PCG line relaxation kernel each level runs (SNAC_KV_MG_LINE
- * numbering, chosen by timing when the MG-PCG plan is set up), for levels
+ * numbering, chosen by timing when the MG-PCG plan is set up; 5: lines from
+ * precomputed factors, FP64 levels with few kinds of columns), for levels
  * 0..n-1 of the FP64 and of the FP32 V-cycle; -1 for levels in the fused
  * coarse-end kernel, past the last level, or before the MG-PCG path is
  * planned (either pointer may be null).  No counterpart in the reference. */

@@ -1,5 +1,5 @@
 // Both colours of a multigrid level's zebra sweep in one launch (FFT path,
-// FP64, factored lines), for the descent and for the ascent of the V-cycle.
+// factored lines), for the descent and for the ascent of the V-cycle.
 //
 // A lane segment marches over the level's line pairs (2I, 2I + 1): the
 // colour-0 lines ahead of it, with their neighbours at zero, need nothing but
@@ -17,6 +17,10 @@
 // 512 columns, 128 rows: the finest level 19 us down, 27 us up (the memory's
 // share is 8 and 13), the last launched one (64 columns) 7 and 8; five
 // launches a level before, 8.9 us on average; a step 7.4 -> 6.0 ms.
+// FP32 (64 modes, 256 x 256): the descent stores both colours for the
+// restriction's own kernel, whose bits count, three launches a level: 12 us
+// down, 18 up on the finest, 5 and 8 on the last launched (6.2 per colour
+// before); a step 8.06 -> 7.67 ms.
 // A segment solves the lines at its ends that its neighbours also solve, so
 // no segment reads what another writes.
 #include "mgline_device.hpp"
@@ -26,10 +30,10 @@ namespace {
 
 // line_apply for N lines of one class at once: the steps of a line's solve
 // depend on each other, those of different lines overlap
-template <int N, int K, int LPL, bool FULL>
-__device__ __forceinline__ void lines_apply(const LineFac<K, LPL, double> &f, const double (&r)[N][K], int cnt,
-                                            int lane, int seg0, double (&x)[N][K]) {
-  double d[N][K], e0[N], e1[N];
+template <int N, int K, int LPL, typename T, bool FULL, int MODE>
+__device__ __forceinline__ void lines_apply(const LineFac<K, LPL, T> &f, const T (&r)[N][K], int cnt, int lane, int seg0,
+                                            T (&x)[N][K]) {
+  T d[N][K], e0[N], e1[N];
 #pragma unroll
   for (int n = 0; n < N; n++) {
     d[n][0] = r[n][0];
@@ -38,7 +42,9 @@ __device__ __forceinline__ void lines_apply(const LineFac<K, LPL, double> &f, co
 #pragma unroll
   for (int j = 2; j < K; j++)
 #pragma unroll
-    for (int n = 0; n < N; n++) d[n][j] = f.g[j - 1] * r[n][j] - f.h[j - 1] * d[n][j - 1];
+    for (int n = 0; n < N; n++)
+      d[n][j] = MODE == 0 ? f.g[j - 1] * r[n][j] - f.h[j - 1] * d[n][j - 1]
+                          : (r[n][j] - f.h[j - 1] * d[n][j - 1]) * f.g[j - 1];
 #pragma unroll
   for (int n = 0; n < N; n++) {
     e1[n] = d[n][K - 1];
@@ -52,7 +58,7 @@ __device__ __forceinline__ void lines_apply(const LineFac<K, LPL, double> &f, co
   for (int n = 0; n < N; n++) e0[n] = r[n][0] - f.u0 * d[n][1];
   {
     const int sm = seg0 + (lane > 0 ? lane - 1 : lane), sp = seg0 + (lane < LPL - 1 ? lane + 1 : lane);
-    double lo[N], hi[N];
+    T lo[N], hi[N];
 #pragma unroll
     for (int n = 0; n < N; n++) {
       lo[n] = shf(e1[n], sm);
@@ -60,8 +66,8 @@ __device__ __forceinline__ void lines_apply(const LineFac<K, LPL, double> &f, co
     }
 #pragma unroll
     for (int n = 0; n < N; n++) {
-      const double n0 = e0[n] - f.k[0] * lo[n] - f.k[1] * e1[n];
-      const double n1 = e1[n] - f.k[2] * e0[n] - f.k[3] * hi[n];
+      const T n0 = e0[n] - f.k[0] * lo[n] - f.k[1] * e1[n];
+      const T n1 = e1[n] - f.k[2] * e0[n] - f.k[3] * hi[n];
       e0[n] = n0;
       e1[n] = n1;
     }
@@ -69,7 +75,7 @@ __device__ __forceinline__ void lines_apply(const LineFac<K, LPL, double> &f, co
 #pragma unroll
   for (int q = 1, h = 1; h < LPL; q++, h <<= 1) {
     const int sm = seg0 + (lane >= h ? lane - h : lane), sp = seg0 + (lane + h < LPL ? lane + h : lane);
-    double a0[N], b0[N], a1[N], b1[N];
+    T a0[N], b0[N], a1[N], b1[N];
 #pragma unroll
     for (int n = 0; n < N; n++) {
       a0[n] = shf(e0[n], sm);
@@ -85,7 +91,7 @@ __device__ __forceinline__ void lines_apply(const LineFac<K, LPL, double> &f, co
   }
 #pragma unroll
   for (int n = 0; n < N; n++) {
-    const double xp = e0[n] * f.i0, xl = e1[n] * f.i1;
+    const T xp = MODE == 2 ? e0[n] / f.i0 : e0[n] * f.i0, xl = MODE == 2 ? e1[n] / f.i1 : e1[n] * f.i1;
     x[n][0] = xp;
 #pragma unroll
     for (int j = 1; j < K - 1; j++) x[n][j] = d[n][j] - f.a[j - 1] * xp - f.xq[j - 1] * xl;
@@ -96,15 +102,15 @@ __device__ __forceinline__ void lines_apply(const LineFac<K, LPL, double> &f, co
 }
 
 // A segment's lines: positions u = 2 i0 - 2 ... 2 i1 of a periodic level.
-template <int K, int LPL, bool FULL>
+template <int K, int LPL, typename T, bool FULL, int MODE>
 struct March {
-  LineFac<K, LPL, double> f;
-  double cap[K], cam[K];
-  const double *b;
+  LineFac<K, LPL, T> f;
+  T cap[K], cam[K];
+  const T *b;
   int m, i0, i1, lane, seg0, cnt, p0, na, ns;
 
   // false: no line for the calling thread's segment
-  __device__ __forceinline__ bool init(const MGLev &L, const MGFacT<double> &F, const double *b_, const int *done,
+  __device__ __forceinline__ bool init(const MGLevT<T> &L, const MGFacT<T> &F, const T *b_, const int *done,
                                        int nc, int r, int ngrp) {
     const int sid = (int)(((long)blockIdx.x * 256 + threadIdx.x) / LPL);
     const int slot = sid / ngrp, grp = sid - slot * ngrp;
@@ -121,74 +127,88 @@ struct March {
     na = L.na;
     ns = L.ns;
     b = b_ + (long)m * na * ns + p0;
-    f.load(F.tab + (long)m * LineFac<K, LPL, double>::NE * LPL + lane);
-    coup_load<K, LPL, double>(F.cc + lane, cap, cam);
+    f.load(F.tab + (long)m * LineFac<K, LPL, T>::NE * LPL + lane);
+    coup_load<K, LPL, T>(F.cc + lane, cap, cam);
     return i0 < i1;
   }
   __device__ __forceinline__ int line(int u) const { return u < 0 ? u + na : u < na ? u : u - na; }
   // this lane's rows of b at u (on: else zeros)
-  __device__ __forceinline__ void rows(int u, double (&v)[K], bool on = true) const {
-    if (on) rows_get<K, double, FULL>(b + (long)line(u) * ns, cnt, v);
+  __device__ __forceinline__ void rows(int u, T (&v)[K], bool on = true) const {
+    if (on) rows_get<K, T, FULL>(b + (long)line(u) * ns, cnt, v);
     else {
 #pragma unroll
       for (int j = 0; j < K; j++) v[j] = 0;
     }
   }
-  // adds the prolongation onto the colour-0 line at u
-  __device__ __forceinline__ void prolong(const double *c, int u, double (&v)[K]) const {
-    double w[K];
-    rows_get<K, double, FULL>(c + (long)(line(u) >> 1) * ns, cnt, w);
+  // adds the prolongation onto the colour-0 line at u (to the rounded value,
+  // as if v came from memory: not fused with the product that v ends with)
+  __device__ __forceinline__ void prolong(const T *c, int u, T (&v)[K]) const {
+#pragma clang fp contract(off)
+    T w[K];
+    rows_get<K, T, FULL>(c + (long)(line(u) >> 1) * ns, cnt, w);
 #pragma unroll
     for (int j = 0; j < K; j++) v[j] += w[j];
   }
   // x of N lines: right-hand sides b, plus the couplings to the lines below
   // (lo) and above (hi) unless bit n of Z says that there are none
   template <int Z, int N>
-  __device__ __forceinline__ void solve(const double (&bb)[N][K], const double (&lo)[N][K], const double (&hi)[N][K],
-                                        double (&x)[N][K]) const {
-    double r[N][K];
+  __device__ __forceinline__ void solve(const T (&bb)[N][K], const T (&lo)[N][K], const T (&hi)[N][K],
+                                        T (&x)[N][K]) const {
+    T r[N][K];
 #pragma unroll
     for (int n = 0; n < N; n++)
 #pragma unroll
       for (int j = 0; j < K; j++)
         r[n][j] = (Z >> n) & 1 ? bb[n][j] : bb[n][j] + fma_(cam[j], lo[n][j], cap[j] * hi[n][j]);
-    lines_apply<N, K, LPL, FULL>(f, r, cnt, lane, seg0, x);
+    lines_apply<N, K, LPL, T, FULL, MODE>(f, r, cnt, lane, seg0, x);
   }
 };
 
-template <int K>
-__device__ __forceinline__ void set(double (&d)[K], const double (&s)[K]) {
+template <int K, typename T>
+__device__ __forceinline__ void set(T (&d)[K], const T (&s)[K]) {
 #pragma unroll
   for (int j = 0; j < K; j++) d[j] = s[j];
 }
 
-// The descent: bc = the restricted residual after colour 0 (neighbours at
-// zero) and colour 1.
-template <int K, int LPL, bool FULL>
-__global__ __launch_bounds__(256) void k_pair_down(MGLev L, MGFacT<double> F, const double *__restrict__ b,
-                                                   double *__restrict__ bc, const int *__restrict__ done, int nc, int r,
+// The descent, colour 0 (neighbours at zero) and colour 1.  FP64: out = the
+// restricted residual.  FP32: out = both colours, for a restriction of its
+// own: the bits of the residual are those of the unfactored form.
+template <int K, int LPL, typename T, bool FULL, int MODE>
+__global__ __launch_bounds__(256) void k_pair_down(MGLevT<T> L, MGFacT<T> F, const T *__restrict__ b,
+                                                   T *__restrict__ out, const int *__restrict__ done, int nc, int r,
                                                    int ngrp) {
-  March<K, LPL, FULL> M;
+  March<K, LPL, T, FULL, MODE> M;
   if (!M.init(L, F, b, done, nc, r, ngrp)) return;
   const int i0 = M.i0, i1 = M.i1, cnt = M.cnt;
-  bc += (long)M.m * nc * M.ns + M.p0;
-  double lo[2][K], hi[2][K], bb[2][K], nb[2][K], x[2][K], c[K], n[K], xm[K];
-  M.rows(2 * i0 - 2, bb[0]);
-  M.rows(2 * i0, bb[1]);
-  M.rows(2 * i0 - 1, nb[0]);
-  M.rows(2 * i0 + 2, nb[1]);
-  M.template solve<3>(bb, lo, hi, x);
-  set(lo[0], x[0]);
-  set(hi[0], x[1]);
-  set(c, x[1]);
+  out += (long)M.m * (MODE == 0 ? nc : M.na) * M.ns + M.p0;
+  T lo[2][K], hi[2][K], bb[2][K], nb[2][K], x[2][K], c[K], n[K], xm[K];
+  if constexpr (MODE == 0) {
+    M.rows(2 * i0 - 2, bb[0]);
+    M.rows(2 * i0, bb[1]);
+    M.rows(2 * i0 - 1, nb[0]);
+    M.rows(2 * i0 + 2, nb[1]);
+    M.template solve<3>(bb, lo, hi, x);
+    set(lo[0], x[0]);
+    set(hi[0], x[1]);
+    set(c, x[1]);
+  } else {
+    M.rows(2 * i0, nb[0]);
+    M.rows(2 * i0 + 2, nb[1]);
+  }
   M.rows(2 * i0 + 1, bb[0]);
   M.rows(2 * i0 + 4, bb[1], i0 + 1 < i1);
-  M.template solve<2>(nb, lo, hi, x);
-  set(xm, x[0]);
+  if constexpr (MODE == 0) {
+    M.template solve<2>(nb, lo, hi, x);
+    set(xm, x[0]);
+  } else {
+    M.template solve<3>(nb, lo, hi, x);
+    set(c, x[0]);
+  }
   set(n, x[1]);
   for (int I = i0; I < i1; I++) {
     const int u = 2 * I;
-    double xp[K];
+    T xp[K];
+    if constexpr (MODE != 0) rows_put<K, T, FULL>(out + (long)u * M.ns, cnt, c);
     if (I + 1 < i1) {
       set(lo[0], c);
       set(hi[0], n);
@@ -201,33 +221,37 @@ __global__ __launch_bounds__(256) void k_pair_down(MGLev L, MGFacT<double> F, co
       set(bb[0], nb[0]);
       set(bb[1], nb[1]);
     } else {
-      double l1[1][K], h1[1][K], b1[1][K], y[1][K];
+      T l1[1][K], h1[1][K], b1[1][K], y[1][K];
       set(l1[0], c);
       set(h1[0], n);
       set(b1[0], bb[0]);
       M.template solve<0>(b1, l1, h1, y);
       set(xp, y[0]);
     }
-    double v[K];
+    if constexpr (MODE == 0) {
+      T v[K];
 #pragma unroll
-    for (int j = 0; j < K; j++) v[j] = M.cap[j] * xp[j] + M.cam[j] * xm[j];
-    rows_put<K, double, FULL>(bc + (long)I * M.ns, cnt, v);
-    set(xm, xp);
+      for (int j = 0; j < K; j++) v[j] = M.cap[j] * xp[j] + M.cam[j] * xm[j];
+      rows_put<K, T, FULL>(out + (long)I * M.ns, cnt, v);
+      set(xm, xp);
+    } else {
+      rows_put<K, T, FULL>(out + (long)(u + 1) * M.ns, cnt, xp);
+    }
   }
 }
 
 // The ascent: colour 1 against the colour-0 lines of the descent with xc
 // added, then colour 0; x = both.
-template <int K, int LPL, bool FULL>
-__global__ __launch_bounds__(256) void k_pair_up(MGLev L, MGFacT<double> F, double *__restrict__ x,
-                                                 const double *__restrict__ b, const double *__restrict__ xc,
+template <int K, int LPL, typename T, bool FULL, int MODE>
+__global__ __launch_bounds__(256) void k_pair_up(MGLevT<T> L, MGFacT<T> F, T *__restrict__ x,
+                                                 const T *__restrict__ b, const T *__restrict__ xc,
                                                  const int *__restrict__ done, int nc, int r, int ngrp) {
-  March<K, LPL, FULL> M;
+  March<K, LPL, T, FULL, MODE> M;
   if (!M.init(L, F, b, done, nc, r, ngrp)) return;
   const int i0 = M.i0, i1 = M.i1, cnt = M.cnt, ns = M.ns;
   x += (long)M.m * M.na * ns + M.p0;
   xc += (long)M.m * nc * ns + M.p0;
-  double lo[3][K], hi[3][K], bb[3][K], nb[3][K], y[3][K], xm[K], xp[K], z1[K], z2[K];
+  T lo[3][K], hi[3][K], bb[3][K], nb[3][K], y[3][K], xm[K], xp[K], z1[K], z2[K];
   {
     const int u = 2 * i0;
     M.rows(u - 2, bb[0]);
@@ -267,8 +291,8 @@ __global__ __launch_bounds__(256) void k_pair_up(MGLev L, MGFacT<double> F, doub
       M.rows(u + 8, nb[2], I + 3 < i1);
       M.template solve<4>(bb, lo, hi, y);  // lines u, u + 3 and u + 6
       if (two) M.prolong(xc, u + 6, y[2]);
-      rows_put<K, double, FULL>(x + (long)u * ns, cnt, y[0]);
-      rows_put<K, double, FULL>(x + (long)(u + 1) * ns, cnt, xp);
+      rows_put<K, T, FULL>(x + (long)u * ns, cnt, y[0]);
+      rows_put<K, T, FULL>(x + (long)(u + 1) * ns, cnt, xp);
       set(xm, xp);
       set(xp, y[1]);
       set(z1, z2);
@@ -276,23 +300,33 @@ __global__ __launch_bounds__(256) void k_pair_up(MGLev L, MGFacT<double> F, doub
 #pragma unroll
       for (int n = 0; n < 3; n++) set(bb[n], nb[n]);
     } else {
-      double l1[1][K], h1[1][K], b1[1][K], y1[1][K];
+      T l1[1][K], h1[1][K], b1[1][K], y1[1][K];
       set(l1[0], xm);
       set(h1[0], xp);
       set(b1[0], bb[0]);
       M.template solve<0>(b1, l1, h1, y1);
-      rows_put<K, double, FULL>(x + (long)u * ns, cnt, y1[0]);
-      rows_put<K, double, FULL>(x + (long)(u + 1) * ns, cnt, xp);
+      rows_put<K, T, FULL>(x + (long)u * ns, cnt, y1[0]);
+      rows_put<K, T, FULL>(x + (long)(u + 1) * ns, cnt, xp);
     }
   }
 }
 
-template <typename G>
-void fp64_shape(const MGFacT<double> &F, G &&go) {
+// calls go(K, LPL, FULL, MODE) as integral constants for a level's instance
+template <typename T, typename G>
+void pair_shape(const MGLevT<T> &L, const MGFacT<T> &F, G &&go) {
   with_shape(F.K, F.lpl, [&](auto kk, auto ll) {
     constexpr int K = decltype(kk)::value, LPL = decltype(ll)::value;
-    if constexpr (LPL == 32 && K <= 6) go(kk, ll);
-    else throw std::runtime_error("internal: no line-pair instance");
+    if constexpr (LPL == 32 && (sizeof(T) == 4 || K <= 6)) {
+      auto mode = [&](auto full) {
+        if constexpr (sizeof(T) == 8) go(kk, ll, full, std::integral_constant<int, 0>{});
+        else if (F.mode == 1) go(kk, ll, full, std::integral_constant<int, 1>{});
+        else go(kk, ll, full, std::integral_constant<int, 2>{});
+      };
+      if (L.ns == F.lpl * F.K) mode(std::true_type{});
+      else mode(std::false_type{});
+    } else {
+      throw std::runtime_error("internal: no line-pair instance");
+    }
   });
 }
 
@@ -300,7 +334,8 @@ void fp64_shape(const MGFacT<double> &F, G &&go) {
 // registers allow).  A segment solves 2 r + 3 lines going down and 3 r + 3
 // going up for its r pairs; a step of 64 modes, 512 columns, 128 rows with
 // 512 / 1024 / 2048 / 4096 wavefronts: 6.3 / 6.0 / 6.1 / 6.2 ms.
-int pairs_per_segment(const MGLev &L, const MGFacT<double> &F, int nc) {
+template <typename T>
+int pairs_per_segment(const MGLevT<T> &L, const MGFacT<T> &F, int nc) {
   return (int)std::max<long>(1, (long)nc * L.nm / (1024L * (64 / F.lpl)));
 }
 
@@ -311,34 +346,45 @@ int pairs_per_segment(const MGLev &L, const MGFacT<double> &F, int nc) {
 // step) a segment reloads its factors at each class' end, and the launch
 // waits for those segments: a step of 48 modes, 512 columns, 80 rows 10.4 ms
 // against 9.3 with one colour per launch.
-bool mg_pair_fits(const MGLev &L, const MGFacT<double> &F) {
-  return F.tab && F.ncls == 1 && F.lpl == 32 && F.K <= 6 && !L.coupled && L.per_a && L.na >= 8 && L.na % 2 == 0;
+template <typename T>
+bool mg_pair_fits(const MGLevT<T> &L, const MGFacT<T> &F) {
+  return F.tab && F.ncls == 1 && F.lpl == 32 && (sizeof(T) == 4 || F.K <= 6) && !L.coupled && L.per_a && L.na >= 8 &&
+         L.na % 2 == 0;
 }
+template bool mg_pair_fits<double>(const MGLev &, const MGFacT<double> &);
+template bool mg_pair_fits<float>(const MGLevT<float> &, const MGFacT<float> &);
 
-void mg_pair_down(hipStream_t st, const MGLev &L, const MGFacT<double> &F, const double *b, double *bc,
-                  const int *done) {
+template <typename T>
+void mg_pair_down(hipStream_t st, const MGLevT<T> &L, const MGFacT<T> &F, const T *b, T *out, const int *done) {
   const int nc = L.na / 2, r = pairs_per_segment(L, F, nc), ngrp = (nc + r - 1) / r;
   const dim3 grid((unsigned)(((long)ngrp * L.nm * F.lpl + 255) / 256));
-  const bool full = L.ns == F.lpl * F.K;
-  fp64_shape(F, [&](auto kk, auto ll) {
-    constexpr int K = decltype(kk)::value, LPL = decltype(ll)::value;
-    if (full) hipLaunchKernelGGL((k_pair_down<K, LPL, true>), grid, dim3(256), 0, st, L, F, b, bc, done, nc, r, ngrp);
-    else hipLaunchKernelGGL((k_pair_down<K, LPL, false>), grid, dim3(256), 0, st, L, F, b, bc, done, nc, r, ngrp);
+  pair_shape(L, F, [&](auto kk, auto ll, auto fu, auto mo) {
+    hipLaunchKernelGGL((k_pair_down<decltype(kk)::value, decltype(ll)::value, T, decltype(fu)::value,
+                                    decltype(mo)::value>),
+                       grid, dim3(256), 0, st, L, F, b, out, done, nc, r, ngrp);
   });
   SNAC_HIP(hipGetLastError());
 }
+template void mg_pair_down<double>(hipStream_t, const MGLev &, const MGFacT<double> &, const double *, double *,
+                                   const int *);
+template void mg_pair_down<float>(hipStream_t, const MGLevT<float> &, const MGFacT<float> &, const float *, float *,
+                                  const int *);
 
-void mg_pair_up(hipStream_t st, const MGLev &L, const MGFacT<double> &F, double *x, const double *b, const double *xc,
+template <typename T>
+void mg_pair_up(hipStream_t st, const MGLevT<T> &L, const MGFacT<T> &F, T *x, const T *b, const T *xc,
                 const int *done) {
   const int nc = L.na / 2, r = pairs_per_segment(L, F, nc), ngrp = (nc + r - 1) / r;
   const dim3 grid((unsigned)(((long)ngrp * L.nm * F.lpl + 255) / 256));
-  const bool full = L.ns == F.lpl * F.K;
-  fp64_shape(F, [&](auto kk, auto ll) {
-    constexpr int K = decltype(kk)::value, LPL = decltype(ll)::value;
-    if (full) hipLaunchKernelGGL((k_pair_up<K, LPL, true>), grid, dim3(256), 0, st, L, F, x, b, xc, done, nc, r, ngrp);
-    else hipLaunchKernelGGL((k_pair_up<K, LPL, false>), grid, dim3(256), 0, st, L, F, x, b, xc, done, nc, r, ngrp);
+  pair_shape(L, F, [&](auto kk, auto ll, auto fu, auto mo) {
+    hipLaunchKernelGGL((k_pair_up<decltype(kk)::value, decltype(ll)::value, T, decltype(fu)::value,
+                                  decltype(mo)::value>),
+                       grid, dim3(256), 0, st, L, F, x, b, xc, done, nc, r, ngrp);
   });
   SNAC_HIP(hipGetLastError());
 }
+template void mg_pair_up<double>(hipStream_t, const MGLev &, const MGFacT<double> &, double *, const double *,
+                                 const double *, const int *);
+template void mg_pair_up<float>(hipStream_t, const MGLevT<float> &, const MGFacT<float> &, float *, const float *,
+                                const float *, const int *);
 
 }  // namespace snac

@@ -180,14 +180,16 @@ void mg_line_fac(hipStream_t st, const MGLevT<T> &L, const MGFacT<T> &F, T *x, c
 // mg_tail with the levels' factors; false (nothing launched) where a level has none
 template <typename T>
 bool mg_tail_fac(hipStream_t st, const MGTailT<T> &t, int nm, const T *lam, const int *done);
-// both colours of a level in one launch (FP64, kernels_mgpair.hip): whether
-// the level has that form; the restricted residual bc after a pre-smoothing
-// from zero (x is not written); x after the post-smoothing with the coarse
-// correction xc
-bool mg_pair_fits(const MGLev &L, const MGFacT<double> &F);
-void mg_pair_down(hipStream_t st, const MGLev &L, const MGFacT<double> &F, const double *b, double *bc,
-                  const int *done);
-void mg_pair_up(hipStream_t st, const MGLev &L, const MGFacT<double> &F, double *x, const double *b, const double *xc,
+// both colours of a level in one launch (kernels_mgpair.hip): whether the
+// level has that form; the pre-smoothing from zero, of which out is the
+// restricted residual (FP64; x is not written) or x (FP32); x after the
+// post-smoothing with the coarse correction xc
+template <typename T>
+bool mg_pair_fits(const MGLevT<T> &L, const MGFacT<T> &F);
+template <typename T>
+void mg_pair_down(hipStream_t st, const MGLevT<T> &L, const MGFacT<T> &F, const T *b, T *out, const int *done);
+template <typename T>
+void mg_pair_up(hipStream_t st, const MGLevT<T> &L, const MGFacT<T> &F, T *x, const T *b, const T *xc,
                 const int *done);
 // the restricted residual after a two-colour pre-smoothing from zero (FP64)
 void mg_restrict_zebra(hipStream_t st, const MGLev &F, const MGLev &C, const double *x, double *bc, const int *done);

@@ -711,16 +711,15 @@ void vcycle(MGPlan &P, MGHier<T> &H, hipStream_t st, size_t l) {
   // factored lines, unless a line kernel is forced
   const MGFacT<T> &F = H.fac[l];
   const bool fac = fac_in_use(F) && !L.coupled && mg_line_variant() < 0;
-  if constexpr (sizeof(T) == 8) {
-    if (fac && nc == 2 && !(l == 0 && P.smooth_only) && mg_pair_fits(L, F)) {
-      const bool mk = l == 0 && P.mark_line0;
-      if (mk) P.mark_line0(true);
-      mg_pair_down(st, L, F, b, H.bl[l + 1], P.done);
-      if (mk) P.mark_line0(false);
-      vcycle(P, H, st, l + 1);
-      mg_pair_up(st, L, F, x, b, H.xl[l + 1], P.done);
-      return;
-    }
+  if (fac && nc == 2 && !(l == 0 && P.smooth_only) && mg_pair_fits(L, F)) {
+    const bool mk = l == 0 && P.mark_line0;
+    if (mk) P.mark_line0(true);
+    mg_pair_down<T>(st, L, F, b, sizeof(T) == 8 ? H.bl[l + 1] : x, P.done);
+    if (mk) P.mark_line0(false);
+    if (sizeof(T) == 4) mg_restrict_residual(st, L, H.lev[l + 1], H.lam, x, b, H.bl[l + 1], P.done);
+    vcycle(P, H, st, l + 1);
+    mg_pair_up<T>(st, L, F, x, b, H.xl[l + 1], P.done);
+    return;
   }
   if (zero_first) mg_zero(st, (long)L.nm * L.na * L.ns, x);
   for (int k = 0; k < nc; k++) {
