@@ -318,13 +318,16 @@ def run_form(name, d, b, args, cells, dt_ref):
             if l0_n > 0:
                 esz = 4 if f32 else 8
                 avg = l0_ms / l0_n
-                bytes_ = 1.5 * unk * esz
+                # one launch per CG iteration: the descent of both colours,
+                # else the three sweeps that read their neighbour lines
+                pair = l0_n <= up_n
+                bytes_ = (2 if pair and f32 else 1.5) * unk * esz
                 out["roofline_line0"] = {
                     "bound": "hbm", "achieved": round(bytes_ / (avg * 1e-3) / 1e9, 1), "peak": HBM_PEAK_GBS,
                     "unit": "GB/s", "frac": round(bytes_ / (avg * 1e-3) / 1e9 / HBM_PEAK_GBS, 4),
-                    "traffic": traffic_for("k_line", args.workload, args.size, name),
-                    "kernel": f"k_line, finest level, one zebra colour ({'FP32' if f32 else 'FP64'}; "
-                              f"1.5 x {esz} B per unknown)", "avg_launch_ms": round(avg, 4),
+                    "traffic": None if pair else traffic_for("k_line", args.workload, args.size, name),
+                    "kernel": f"{'k_pair_down, finest level, both zebra colours' if pair else 'k_line, finest level, one zebra colour'} "
+                              f"({'FP32' if f32 else 'FP64'}; {2 if pair and f32 else 1.5} x {esz} B per unknown)", "avg_launch_ms": round(avg, 4),
                     "launches": l0_n, "ms_per_step": round(l0_ms / ne, 4)}
             # the dominant MG kernel: the one with more time per step
             cand = [k for k in ("roofline_update", "roofline_line0") if k in out]

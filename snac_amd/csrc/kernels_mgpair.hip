@@ -311,12 +311,19 @@ __global__ __launch_bounds__(256) void k_pair_up(MGLevT<T> L, MGFacT<T> F, T *__
   }
 }
 
+// shapes whose factors and lines in flight fit the registers of a wavefront
+// or two per SIMD
+template <typename T>
+constexpr bool pair_instance(int K, int lpl) {
+  return lpl == 32 ? (sizeof(T) == 4 || K <= 6) : (sizeof(T) == 8 && K <= 4);
+}
+
 // calls go(K, LPL, FULL, MODE) as integral constants for a level's instance
 template <typename T, typename G>
 void pair_shape(const MGLevT<T> &L, const MGFacT<T> &F, G &&go) {
   with_shape(F.K, F.lpl, [&](auto kk, auto ll) {
     constexpr int K = decltype(kk)::value, LPL = decltype(ll)::value;
-    if constexpr (LPL == 32 && (sizeof(T) == 4 || K <= 6)) {
+    if constexpr (pair_instance<T>(K, LPL)) {
       auto mode = [&](auto full) {
         if constexpr (sizeof(T) == 8) go(kk, ll, full, std::integral_constant<int, 0>{});
         else if (F.mode == 1) go(kk, ll, full, std::integral_constant<int, 1>{});
@@ -341,15 +348,15 @@ int pairs_per_segment(const MGLevT<T> &L, const MGFacT<T> &F, int nc) {
 
 }  // namespace
 
-// Levels whose columns are all alike (a uniform periodic axis of even length)
-// with 32 lanes per line.  Where the columns fall into classes (a wall, a
-// step) a segment reloads its factors at each class' end, and the launch
+// Levels whose columns are all alike (a uniform periodic axis of even
+// length): 64 modes of 512 x 128 above; 256 modes of 512 x 256 in FP64 (64
+// lanes) 36.5 -> 30.5 ms a step.  Where the columns fall into classes (a wall,
+// a step) a segment reloads its factors at each class' end, and the launch
 // waits for those segments: a step of 48 modes, 512 columns, 80 rows 10.4 ms
 // against 9.3 with one colour per launch.
 template <typename T>
 bool mg_pair_fits(const MGLevT<T> &L, const MGFacT<T> &F) {
-  return F.tab && F.ncls == 1 && F.lpl == 32 && (sizeof(T) == 4 || F.K <= 6) && !L.coupled && L.per_a && L.na >= 8 &&
-         L.na % 2 == 0;
+  return F.tab && F.ncls == 1 && pair_instance<T>(F.K, F.lpl) && !L.coupled && L.per_a && L.na >= 8 && L.na % 2 == 0;
 }
 template bool mg_pair_fits<double>(const MGLev &, const MGFacT<double> &);
 template bool mg_pair_fits<float>(const MGLevT<float> &, const MGFacT<float> &);

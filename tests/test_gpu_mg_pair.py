@@ -1,6 +1,6 @@
 """Both colours of a periodic multigrid level in one launch, over several line
 pairs per lane segment: a last segment that is full, short or of one pair,
-lines of 2..6 rows per lane in whole and ragged chunks, against the direct
+lines of 2..6 rows on 32 lanes and 4 on 64 in whole and ragged chunks, against the direct
 solver and the unfactored kernels.  (One pair per segment and the edges of
 the lane splits: the factored lines' test.)"""
 import numpy as np
@@ -12,7 +12,8 @@ from test_gpu_mg_factored import solve
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("n", [(512, 64, 32), (500, 12, 64), (258, 33, 128), (480, 130, 36), (136, 192, 128), (66, 20, 256)])
+@pytest.mark.parametrize("n", [(512, 64, 32), (500, 12, 64), (258, 33, 128), (480, 130, 36), (136, 192, 128), (66, 20, 256),
+                               (260, 256, 64), (264, 200, 36)])
 def test_line_pairs(tmp_path, n):
     blk = cases.channel_block(n)
     ref, _, _ = solve(tmp_path, "t", blk, "fp64", "tensor")
