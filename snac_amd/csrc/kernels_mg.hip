@@ -199,17 +199,28 @@ __device__ __forceinline__ void line_elim(int ns, int nch, int cnt, bool act, RO
 // one row of line (m, a): diagonal, couplings below and above and the
 // right-hand side with the neighbour lines' contribution (zero_nb: read as
 // zero; xc: with the prolongation of xc added), or the identity row of the
-// pinned row of a singular group
+// pinned row of a singular group.  wa, wm: the line's entries of MGEnds, or null
 template <typename T>
 __device__ __forceinline__ void line_row(const MGLevT<T> &L, T lmv, const T *__restrict__ x, const T *__restrict__ b,
                                          int m, int a, int s, long e, long q, int zero_nb, int pin_s, bool pin,
-                                         const T *__restrict__ xc, int cna, T &l, T &d, T &u, T &r) {
+                                         const T *__restrict__ xc, int cna, const T *wa, const T *wm, T &l, T &d, T &u,
+                                         T &r) {
   d = L.dg[q] - lmv * L.w[q];
   l = s > 0 ? -L.cs[q - 1] : T(0);
   u = s < L.ns - 1 ? -L.cs[q] : T(0);
   r = b[e];
-  if (!zero_nb) r += xc ? nb_sum_pro(L, x, m, a, s, e, q, xc, cna) : nb_sum(L, x, m, a, e, q);
+  if (!zero_nb) {
+    if (xc) r += nb_sum_pro(L, x, m, a, s, e, q, xc, cna);
+    else r += nb_sum(L, x, m, a, e, q, wa ? wa + s : nullptr, wm ? wm + s : nullptr);
+  }
   if (pin && s == pin_s) { d = 1; l = 0; u = 0; r = 0; }
+}
+
+// the two end lines of an odd periodic axis at position i of the other axis
+// (MGEnds; null: none)
+template <typename T>
+__device__ __forceinline__ const T *ends_at(const T *w, const MGLevT<T> &L, int i) {
+  return w ? w + (long)i * 2 * L.ns : nullptr;
 }
 
 // relaxes line (m, a) with the calling lane segment, rows read from and x
@@ -222,7 +233,7 @@ __device__ __forceinline__ void line_row(const MGLevT<T> &L, T lmv, const T *__r
 template <int K, int LPL, typename T, bool FR = false, bool FULL = false>
 __device__ __forceinline__ void line_solve(const MGLevT<T> &L, T lmv, T *__restrict__ x, const T *__restrict__ b,
                                            int m, int a, int zero_nb, int pin_s, bool pin, bool act,
-                                           const T *__restrict__ xc = nullptr, int cna = 0) {
+                                           const T *__restrict__ xc, int cna, const T *wa, const T *wm) {
   if (FULL && !act) return;
   const int wl = threadIdx.x & 63, lane = wl & (LPL - 1);
   const long e0 = vidx(L, m, a, 0), q0 = cidx(L, m, a, 0);
@@ -234,7 +245,7 @@ __device__ __forceinline__ void line_solve(const MGLevT<T> &L, T lmv, T *__restr
     lo[j] = 0; dg[j] = 1; up[j] = 0; rh[j] = 0;
     if (j < cnt) {
       const int s = p0 + j;
-      line_row(L, lmv, x, b, m, a, s, e0 + s, q0 + s, zero_nb, pin_s, pin, xc, cna, lo[j], dg[j], up[j], rh[j]);
+      line_row(L, lmv, x, b, m, a, s, e0 + s, q0 + s, zero_nb, pin_s, pin, xc, cna, wa, wm, lo[j], dg[j], up[j], rh[j]);
     }
   }
   line_elim<K, LPL, T, FR, FULL>(
@@ -242,11 +253,15 @@ __device__ __forceinline__ void line_solve(const MGLevT<T> &L, T lmv, T *__restr
       [&](int j, T v) { x[e0 + p0 + j] = v; });
 }
 
-template <int K, int LPL, typename T>
+// ENDS: the level has an odd periodic axis (E); levels without are spared the
+// checks (1-2 % of a solve of the 3D path; k_line_modes: 2.5 % of a step of
+// 256 modes, 512 x 256, mixed)
+template <int K, int LPL, typename T, bool ENDS>
 __global__ __launch_bounds__(256) void k_line(MGLevT<T> L, const T *__restrict__ lam, T *__restrict__ x,
                                               const T *__restrict__ b, int col_a, int col_m, int nla, int nlm,
                                               int zero_nb, int pin_s, const int *__restrict__ singular,
-                                              const int *__restrict__ done, const T *__restrict__ xc, int cna) {
+                                              const int *__restrict__ done, const T *__restrict__ xc, int cna,
+                                              MGEnds<T> E) {
   const long line = ((long)blockIdx.x * 256 + threadIdx.x) / LPL;
   if (line >= (long)nla * nlm) return;  // a whole lane segment leaves together
   const int a = 2 * (int)(line % nla) + col_a;
@@ -256,7 +271,8 @@ __global__ __launch_bounds__(256) void k_line(MGLevT<T> L, const T *__restrict__
   if (done && done[g]) return;
   const T lmv = lam ? lam[m] : T(0);
   const bool pin = pin_s >= 0 && singular && singular[g];
-  line_solve<K, LPL, T>(L, lmv, x, b, m, a, zero_nb, pin_s, pin, true, xc, cna);
+  line_solve<K, LPL, T>(L, lmv, x, b, m, a, zero_nb, pin_s, pin, true, xc, cna,
+                        ENDS ? ends_at(E.wa, L, m) : nullptr, ENDS ? ends_at(E.wm, L, a) : nullptr);
 }
 
 // The same relaxation with the right-hand sides staged through LDS: the
@@ -267,11 +283,12 @@ __global__ __launch_bounds__(256) void k_line(MGLevT<T> L, const T *__restrict__
 // as line_solve does (the same arithmetic, so the same values), and x goes
 // back through LDS to coalesced stores.  The coefficients (mode-independent
 // on the FFT path, so cache-resident) are still read per lane.
-template <int K, int LPL, typename T>
+template <int K, int LPL, typename T, bool ENDS>
 __global__ __launch_bounds__(256) void k_line_lds(MGLevT<T> L, const T *__restrict__ lam, T *__restrict__ x,
                                                   const T *__restrict__ b, int col_a, int col_m, int nla, int nlm,
                                                   int zero_nb, int pin_s, const int *__restrict__ singular,
-                                                  const int *__restrict__ done, const T *__restrict__ xc, int cna) {
+                                                  const int *__restrict__ done, const T *__restrict__ xc, int cna,
+                                                  MGEnds<T> E) {
   constexpr int NLW = 256 / LPL;  // lines per workgroup
   extern __shared__ unsigned char smem_[];
   T *sh = reinterpret_cast<T *>(smem_);  // [NLW][nsp]: right-hand sides, then x (rows at lpad)
@@ -291,7 +308,8 @@ __global__ __launch_bounds__(256) void k_line_lds(MGLevT<T> L, const T *__restri
     const long e0 = vidx(L, m, a, 0), q0 = cidx(L, m, a, 0);
     for (int s = threadIdx.x; s < ns; s += 256) {
       T l, d, u, r;
-      line_row(L, lmv, x, b, m, a, s, e0 + s, q0 + s, zero_nb, pin_s, pin, xc, cna, l, d, u, r);
+      line_row(L, lmv, x, b, m, a, s, e0 + s, q0 + s, zero_nb, pin_s, pin, xc, cna,
+               ENDS ? ends_at(E.wa, L, m) : nullptr, ENDS ? ends_at(E.wm, L, a) : nullptr, l, d, u, r);
       sh[li * nsp + lpad(s)] = r;
     }
   }
@@ -362,12 +380,12 @@ __global__ __launch_bounds__(256) void k_line_lds(MGLevT<T> L, const T *__restri
 // count the arithmetic is line_solve's, so the values are the same; with
 // fewer lanes per line (longer chunks, a shorter interface system) the
 // same line is solved with another elimination order.
-template <int K, int LPL, typename T, bool FR, bool FULL = false>
+template <int K, int LPL, typename T, bool FR, bool FULL, bool ENDS>
 __global__ __launch_bounds__(256) void k_line_modes(MGLevT<T> L, const T *__restrict__ lam, T *__restrict__ x,
                                                     const T *__restrict__ b, int col_a, int nla, int zero_nb,
                                                     int pin_s, const int *__restrict__ singular,
                                                     const int *__restrict__ done, const T *__restrict__ xc,
-                                                    int cna) {
+                                                    int cna, MGEnds<T> E) {
   constexpr int NLW = 256 / LPL;            // modes per workgroup
   constexpr int MB = NLW < 4 ? NLW : 4;     // modes whose loads are issued together
   extern __shared__ unsigned char smem_[];
@@ -420,6 +438,9 @@ __global__ __launch_bounds__(256) void k_line_modes(MGLevT<T> L, const T *__rest
   // 64-bit address arithmetic
   const long mst = (long)L.na * ns, cmst = (long)cna * sa;  // elements per mode, fine and coarse
   const T *b0 = b + vidx(L, 0, a, 0), *x0 = x + vidx(L, 0, a, 0);
+  // across an odd periodic axis, the ends' values from before the sweep
+  const bool ep = ENDS && a == L.na - 1, em = ENDS && a == 0;
+  const T *xp0 = ep ? E.wa : x0 + dp, *xm0 = em ? E.wa + ns : x0 + dm;
   for (int g0 = 0; g0 < NLW; g0 += MB) {
     bool live[MB];
     int pinrow[MB];
@@ -437,8 +458,8 @@ __global__ __launch_bounds__(256) void k_line_modes(MGLevT<T> L, const T *__rest
         const long m = smode[g0 + k];
         const long mo = m * mst, co = m * cmst;
         bv[k] = live[k] ? (b0 + mo)[us] : T(0);
-        xp[k] = live[k] && !zero_nb && hp ? (x0 + mo + dp)[us] : T(0);
-        xm[k] = live[k] && !zero_nb && hm ? (x0 + mo + dm)[us] : T(0);
+        xp[k] = live[k] && !zero_nb && hp ? (xp0 + (ep ? m * 2 * ns : mo))[us] : T(0);
+        xm[k] = live[k] && !zero_nb && hm ? (xm0 + (em ? m * 2 * ns : mo))[us] : T(0);
         cp[k] = live[k] && !zero_nb && actp ? (xc + co + (long)cnp * sa)[us] : T(0);
         cm[k] = live[k] && !zero_nb && actm ? (xc + co + (long)cnm * sa)[us] : T(0);
       }
@@ -507,7 +528,7 @@ __global__ __launch_bounds__(256) void k_line_modes(MGLevT<T> L, const T *__rest
 // level arrays then addressed as mode 0 (the coefficients do not depend on
 // the mode); the arithmetic is the same, so the values are.
 template <int K, int LPL, typename T, bool FR, bool LX, bool FULL = false>
-__global__ __launch_bounds__(1024) void k_tail(MGTailT<T> t, const T *__restrict__ lam, int pin_s,
+__global__ __launch_bounds__(1024) void k_tail(MGTailT<T> t, MGTailEnds<T> E, const T *__restrict__ lam, int pin_s,
                                                const int *__restrict__ singular, const int *__restrict__ done) {
   extern __shared__ unsigned char smem_[];
   const int m = blockIdx.x;
@@ -534,7 +555,8 @@ __global__ __launch_bounds__(1024) void k_tail(MGTailT<T> t, const T *__restrict
       const int nlc = (L.na - c + 1) / 2;  // lines a = 2 j + c of this colour
       for (int j0 = SPW * wv; j0 < nlc; j0 += SPW * nw) {
         const int j = j0 + hs;
-        line_solve<K, LPL, T, FR, FULL>(L, lmv, X(l), B(l), mi, 2 * j + c, c == 0, -1, false, j < nlc);
+        line_solve<K, LPL, T, FR, FULL>(L, lmv, X(l), B(l), mi, 2 * j + c, c == 0, -1, false, j < nlc, nullptr, 0,
+                                        nullptr, nullptr);
       }
       __syncthreads();
     }
@@ -555,7 +577,9 @@ __global__ __launch_bounds__(1024) void k_tail(MGTailT<T> t, const T *__restrict
   // coarsest: one line, solved exactly
   {
     const int l = t.nl - 1;
-    if (wv == 0) line_solve<K, LPL, T, FR, FULL>(t.lev[l], lmv, X(l), B(l), mi, 0, 1, pin_s, pin, hs == 0);
+    if (wv == 0)
+      line_solve<K, LPL, T, FR, FULL>(t.lev[l], lmv, X(l), B(l), mi, 0, 1, pin_s, pin, hs == 0, nullptr, 0, nullptr,
+                                      nullptr);
     __syncthreads();
   }
   // up: post-smooth (colour 1, then colour 0); the colour-1 sweep reads its
@@ -566,10 +590,23 @@ __global__ __launch_bounds__(1024) void k_tail(MGTailT<T> t, const T *__restrict
     const MGLevT<T> &L = t.lev[l], &Cl = t.lev[l + 1];
     for (int c = 1; c >= 0; c--) {
       const int nlc = (L.na - c + 1) / 2;
+      // the ends of an odd periodic axis, neighbours of colour 0, take each
+      // other's value from before the sweep (with the coarse correction)
+      const bool ends = c == 0 && E.wa[l];
+      T *w = E.wa[l] + (long)m * 2 * L.ns;
+      if (ends) {
+        for (int e = threadIdx.x; e < 2 * L.ns; e += blockDim.x) {
+          const int s = e < L.ns ? e : e - L.ns, a = e < L.ns ? 0 : L.na - 1;
+          T v = X(l)[vidx(L, mi, a, s)];
+          if (L.act[cidx(L, mi, a, s)]) v += X(l + 1)[vidx(Cl, mi, a >> 1, s)];
+          w[e] = v;
+        }
+        __syncthreads();
+      }
       for (int j0 = SPW * wv; j0 < nlc; j0 += SPW * nw) {
         const int j = j0 + hs;
         line_solve<K, LPL, T, FR, FULL>(L, lmv, X(l), B(l), mi, 2 * j + c, 0, -1, false, j < nlc,
-                                  c == 1 ? X(l + 1) : nullptr, Cl.na);
+                                        c == 1 ? X(l + 1) : nullptr, Cl.na, ends ? w : nullptr, nullptr);
       }
       __syncthreads();
     }
@@ -712,6 +749,24 @@ __global__ __launch_bounds__(256) void k_restrict_modes(MGLevT<T> F, MGLevT<T> C
         if (live[k]) bc[vidx(Cl, smode[g0 + k], I, s)] = sum[k];
     }
   }
+}
+
+// the two end lines of the odd periodic axes, with the coarse correction xc
+// that they still lack (null: none)
+template <typename T>
+__global__ __launch_bounds__(256) void k_save_ends(MGLevT<T> L, MGEnds<T> E, const T *__restrict__ x,
+                                                   const T *__restrict__ xc, int cna, const int *__restrict__ done) {
+  const long na2 = E.wa ? (long)L.nm * 2 * L.ns : 0, nm2 = E.wm ? (long)L.na * 2 * L.ns : 0;
+  const long idx = (long)blockIdx.x * 256 + threadIdx.x;
+  if (idx >= na2 + nm2) return;
+  const bool along_a = idx < na2;
+  const long t = along_a ? idx : idx - na2;
+  const int s = (int)(t % L.ns), e = (int)(t / L.ns & 1), o = (int)(t / L.ns >> 1);
+  const int m = along_a ? o : (e ? L.nm - 1 : 0), a = along_a ? (e ? L.na - 1 : 0) : o;
+  if (done && done[group_of(L, m)]) return;
+  T v = x[vidx(L, m, a, s)];
+  if (xc && L.act[cidx(L, m, a, s)]) v += xc[((long)m * cna + (cna != L.na ? a >> 1 : a)) * L.ns + s];
+  (along_a ? E.wa : E.wm)[t] = v;
 }
 
 template <typename T>
@@ -1607,32 +1662,33 @@ int line_modes_rows(const MGLevT<T> &L) {
 
 template <int LP, typename T>
 bool launch_line_modes(hipStream_t st, const MGLevT<T> &L, const T *lam, T *x, const T *b, int col_a, int nla,
-                       int zero_nb, int pin_s, const int *singular, const int *done, const T *xc, int cna) {
+                       int zero_nb, int pin_s, const int *singular, const int *done, const T *xc, int cna,
+                       const MGEnds<T> &E) {
   const int rows = line_modes_rows<LP>(L);
   if (!rows) return false;
   constexpr int NLW = 256 / LP;
   const size_t shm = (size_t)(NLW + 5) * lpad_len(L.ns) * sizeof(T);
   dim3 gm((unsigned)((long)nla * ((L.nm + NLW - 1) / NLW)));
-  auto go = [&](auto kk) {
+  auto launch = [&](auto kk, auto fu, auto en) {
     constexpr int KK = decltype(kk)::value;
+    constexpr bool FU = decltype(fu)::value, EN = decltype(en)::value;
     if (g_fast_rcp)
-      hipLaunchKernelGGL((k_line_modes<KK, LP, T, true>), gm, dim3(256), shm, st, L, lam, x, b, col_a, nla, zero_nb,
-                         pin_s, singular, done, xc, cna);
+      hipLaunchKernelGGL((k_line_modes<KK, LP, T, true, FU, EN>), gm, dim3(256), shm, st, L, lam, x, b, col_a, nla,
+                         zero_nb, pin_s, singular, done, xc, cna, E);
     else
-      hipLaunchKernelGGL((k_line_modes<KK, LP, T, false>), gm, dim3(256), shm, st, L, lam, x, b, col_a, nla, zero_nb,
-                         pin_s, singular, done, xc, cna);
+      hipLaunchKernelGGL((k_line_modes<KK, LP, T, false, FU, EN>), gm, dim3(256), shm, st, L, lam, x, b, col_a, nla,
+                         zero_nb, pin_s, singular, done, xc, cna, E);
+    SNAC_HIP(hipGetLastError());
   };
+  auto with_ends = [&](auto kk, auto fu) {
+    if (E.wa) launch(kk, fu, std::true_type{});
+    else launch(kk, fu, std::false_type{});
+  };
+  auto go = [&](auto kk) { with_ends(kk, std::false_type{}); };
   // lines of exactly LP * K rows: the instance with compile-time chunks
   auto full = [&](auto kk) {
-    constexpr int KK = decltype(kk)::value;
-    if (L.ns != LP * KK) return false;
-    if (g_fast_rcp)
-      hipLaunchKernelGGL((k_line_modes<KK, LP, T, true, true>), gm, dim3(256), shm, st, L, lam, x, b, col_a, nla,
-                         zero_nb, pin_s, singular, done, xc, cna);
-    else
-      hipLaunchKernelGGL((k_line_modes<KK, LP, T, false, true>), gm, dim3(256), shm, st, L, lam, x, b, col_a, nla,
-                         zero_nb, pin_s, singular, done, xc, cna);
-    SNAC_HIP(hipGetLastError());
+    if (L.ns != LP * decltype(kk)::value) return false;
+    with_ends(kk, std::true_type{});
     return true;
   };
   if constexpr (LP == 32) {
@@ -1660,13 +1716,13 @@ bool launch_line_modes(hipStream_t st, const MGLevT<T> &L, const T *lam, T *x, c
     if (rows <= 17) go(std::integral_constant<int, 17>{});
     else go(std::integral_constant<int, 33>{});
   }
-  SNAC_HIP(hipGetLastError());
   return true;
 }
 
 template <int LPL, typename T>
 void mg_line_k(hipStream_t st, const MGLevT<T> &L, const T *lam, T *x, const T *b, int col_a, int col_m, int nla,
-               int nlm, int zero_nb, int pin_s, const int *singular, const int *done, const T *xc, int cna) {
+               int nlm, int zero_nb, int pin_s, const int *singular, const int *done, const T *xc, int cna,
+               const MGEnds<T> &E) {
   const long lines = (long)nla * nlm;
   dim3 grid((unsigned)((lines * LPL + 255) / 256));
   const int rows = L.base + (L.extra ? 1 : 0);
@@ -1674,43 +1730,32 @@ void mg_line_k(hipStream_t st, const MGLevT<T> &L, const T *lam, T *x, const T *
   const size_t shb = (size_t)(256 / LPL) * nsp * sizeof(T);
   const int lv = g_line_variant >= 0 ? g_line_variant : (L.lvar >= 0 ? L.lvar : 2);
   // a variant the level does not allow falls back to the next lower one
-  if (lv >= 4 && launch_line_modes<8>(st, L, lam, x, b, col_a, nla, zero_nb, pin_s, singular, done, xc, cna)) return;
-  if (lv >= 3 && launch_line_modes<16>(st, L, lam, x, b, col_a, nla, zero_nb, pin_s, singular, done, xc, cna))
+  if (lv >= 4 && launch_line_modes<8>(st, L, lam, x, b, col_a, nla, zero_nb, pin_s, singular, done, xc, cna, E))
     return;
-  if (lv >= 2 && launch_line_modes<LPL>(st, L, lam, x, b, col_a, nla, zero_nb, pin_s, singular, done, xc, cna))
+  if (lv >= 3 && launch_line_modes<16>(st, L, lam, x, b, col_a, nla, zero_nb, pin_s, singular, done, xc, cna, E))
     return;
-  if (lv >= 1 && L.ns >= 2 && shb <= 64 * 1024) {
-    if (rows <= 3)
-      hipLaunchKernelGGL((k_line_lds<3, LPL, T>), grid, dim3(256), shb, st, L, lam, x, b, col_a, col_m, nla, nlm,
-                         zero_nb, pin_s, singular, done, xc, cna);
-    else if (rows <= 5)
-      hipLaunchKernelGGL((k_line_lds<5, LPL, T>), grid, dim3(256), shb, st, L, lam, x, b, col_a, col_m, nla, nlm,
-                         zero_nb, pin_s, singular, done, xc, cna);
-    else if (rows <= 9)
-      hipLaunchKernelGGL((k_line_lds<9, LPL, T>), grid, dim3(256), shb, st, L, lam, x, b, col_a, col_m, nla, nlm,
-                         zero_nb, pin_s, singular, done, xc, cna);
-    else if (rows <= 17)
-      hipLaunchKernelGGL((k_line_lds<17, LPL, T>), grid, dim3(256), shb, st, L, lam, x, b, col_a, col_m, nla, nlm,
-                         zero_nb, pin_s, singular, done, xc, cna);
+  if (lv >= 2 && launch_line_modes<LPL>(st, L, lam, x, b, col_a, nla, zero_nb, pin_s, singular, done, xc, cna, E))
+    return;
+  const bool lds = lv >= 1 && L.ns >= 2 && shb <= 64 * 1024;
+  auto go = [&](auto kk, auto ends) {
+    constexpr int KK = decltype(kk)::value;
+    constexpr bool EN = decltype(ends)::value;
+    if (lds)
+      hipLaunchKernelGGL((k_line_lds<KK, LPL, T, EN>), grid, dim3(256), shb, st, L, lam, x, b, col_a, col_m, nla, nlm,
+                         zero_nb, pin_s, singular, done, xc, cna, E);
     else
-      throw std::runtime_error("multigrid line relaxation: lines longer than 1088 cells are not supported");
-    SNAC_HIP(hipGetLastError());
-    return;
-  }
-  if (rows <= 3)
-    hipLaunchKernelGGL((k_line<3, LPL, T>), grid, dim3(256), 0, st, L, lam, x, b, col_a, col_m, nla, nlm, zero_nb,
-                       pin_s, singular, done, xc, cna);
-  else if (rows <= 5)
-    hipLaunchKernelGGL((k_line<5, LPL, T>), grid, dim3(256), 0, st, L, lam, x, b, col_a, col_m, nla, nlm, zero_nb,
-                       pin_s, singular, done, xc, cna);
-  else if (rows <= 9)
-    hipLaunchKernelGGL((k_line<9, LPL, T>), grid, dim3(256), 0, st, L, lam, x, b, col_a, col_m, nla, nlm, zero_nb,
-                       pin_s, singular, done, xc, cna);
-  else if (rows <= 17)
-    hipLaunchKernelGGL((k_line<17, LPL, T>), grid, dim3(256), 0, st, L, lam, x, b, col_a, col_m, nla, nlm, zero_nb,
-                       pin_s, singular, done, xc, cna);
-  else
-    throw std::runtime_error("multigrid line relaxation: lines longer than 1088 cells are not supported");
+      hipLaunchKernelGGL((k_line<KK, LPL, T, EN>), grid, dim3(256), 0, st, L, lam, x, b, col_a, col_m, nla, nlm,
+                         zero_nb, pin_s, singular, done, xc, cna, E);
+  };
+  auto rows_of = [&](auto kk) {
+    if (E.wa || E.wm) go(kk, std::true_type{});
+    else go(kk, std::false_type{});
+  };
+  if (rows <= 3) rows_of(std::integral_constant<int, 3>{});
+  else if (rows <= 5) rows_of(std::integral_constant<int, 5>{});
+  else if (rows <= 9) rows_of(std::integral_constant<int, 9>{});
+  else if (rows <= 17) rows_of(std::integral_constant<int, 17>{});
+  else throw std::runtime_error("multigrid line relaxation: lines longer than 1088 cells are not supported");
   SNAC_HIP(hipGetLastError());
 }
 
@@ -1738,18 +1783,31 @@ int mg_line_variant() { return g_line_variant; }
 
 template <typename T>
 void mg_line(hipStream_t st, const MGLevT<T> &L, const T *lam, T *x, const T *b, int col_a, int col_m, int zero_nb,
-             int pin_s, const int *singular, const int *done, const T *xc, int cna) {
+             int pin_s, const int *singular, const int *done, const T *xc, int cna, const MGEnds<T> &E) {
   const int nla = (L.na - col_a + 1) / 2;
   const int nlm = L.coupled ? (L.nm - col_m + 1) / 2 : L.nm;
   if (nla <= 0 || nlm <= 0) return;
   if (xc && (L.coupled || zero_nb)) throw std::runtime_error("internal: fused prolongation needs an FFT-path sweep");
-  if (L.lpl == 32) mg_line_k<32>(st, L, lam, x, b, col_a, col_m, nla, nlm, zero_nb, pin_s, singular, done, xc, cna);
-  else mg_line_k<64>(st, L, lam, x, b, col_a, col_m, nla, nlm, zero_nb, pin_s, singular, done, xc, cna);
+  if (L.lpl == 32) mg_line_k<32>(st, L, lam, x, b, col_a, col_m, nla, nlm, zero_nb, pin_s, singular, done, xc, cna, E);
+  else mg_line_k<64>(st, L, lam, x, b, col_a, col_m, nla, nlm, zero_nb, pin_s, singular, done, xc, cna, E);
 }
 
+template <typename T>
+void mg_save_ends(hipStream_t st, const MGLevT<T> &L, const MGEnds<T> &E, const T *x, const T *xc, int cna,
+                  const int *done) {
+  const long n = 2L * L.ns * ((E.wa ? L.nm : 0) + (E.wm ? L.na : 0));
+  if (n == 0) return;
+  hipLaunchKernelGGL(k_save_ends<T>, dim3(blocks_for(n)), dim3(256), 0, st, L, E, x, xc, cna, done);
+  SNAC_HIP(hipGetLastError());
+}
+template void mg_save_ends<double>(hipStream_t, const MGLev &, const MGEnds<double> &, const double *, const double *,
+                                   int, const int *);
+template void mg_save_ends<float>(hipStream_t, const MGLevT<float> &, const MGEnds<float> &, const float *,
+                                  const float *, int, const int *);
+
 template <int LPL, typename T>
-void mg_tail_k(hipStream_t st, const MGTailT<T> &t, int nm, const T *lam, int pin_s, const int *singular,
-               const int *done) {
+void mg_tail_k(hipStream_t st, const MGTailT<T> &t, int nm, const MGTailEnds<T> &E, const T *lam, int pin_s,
+               const int *singular, const int *done) {
   const MGLevT<T> &L = t.lev[0];
   const int rows = L.base + (L.extra ? 1 : 0);
   const size_t shm = (size_t)t.lds_elems * sizeof(T);
@@ -1759,11 +1817,11 @@ void mg_tail_k(hipStream_t st, const MGTailT<T> &t, int nm, const T *lam, int pi
 #define LAUNCH_TAIL(KK)                                                                                             \
   do {                                                                                                              \
     if (lx)                                                                                                         \
-      hipLaunchKernelGGL((k_tail<KK, LPL, T, false, true>), dim3(nm), dim3(1024), shm, st, t, lam, pin_s, singular,  \
-                         done);                                                                                     \
+      hipLaunchKernelGGL((k_tail<KK, LPL, T, false, true>), dim3(nm), dim3(1024), shm, st, t, E, lam, pin_s,        \
+                         singular, done);                                                                           \
     else                                                                                                            \
-      hipLaunchKernelGGL((k_tail<KK, LPL, T, false, false>), dim3(nm), dim3(1024), 0, st, t, lam, pin_s, singular,   \
-                         done);                                                                                     \
+      hipLaunchKernelGGL((k_tail<KK, LPL, T, false, false>), dim3(nm), dim3(1024), 0, st, t, E, lam, pin_s,         \
+                         singular, done);                                                                           \
   } while (0)
   // lines of exactly LPL * K rows (IEEE divisions): the instance with
   // compile-time chunks
@@ -1773,10 +1831,10 @@ void mg_tail_k(hipStream_t st, const MGTailT<T> &t, int nm, const T *lam, int pi
       constexpr int KK = decltype(kk)::value;
       if (L.ns != LPL * KK) return false;
       if (lx)
-        hipLaunchKernelGGL((k_tail<KK, LPL, T, false, true, true>), dim3(nm), dim3(1024), shm, st, t, lam, pin_s,
+        hipLaunchKernelGGL((k_tail<KK, LPL, T, false, true, true>), dim3(nm), dim3(1024), shm, st, t, E, lam, pin_s,
                            singular, done);
       else
-        hipLaunchKernelGGL((k_tail<KK, LPL, T, false, false, true>), dim3(nm), dim3(1024), 0, st, t, lam, pin_s,
+        hipLaunchKernelGGL((k_tail<KK, LPL, T, false, false, true>), dim3(nm), dim3(1024), 0, st, t, E, lam, pin_s,
                            singular, done);
       return true;
     };
@@ -1793,10 +1851,10 @@ void mg_tail_k(hipStream_t st, const MGTailT<T> &t, int nm, const T *lam, int pi
 }
 
 template <typename T>
-void mg_tail(hipStream_t st, const MGTailT<T> &t, int nm, const T *lam, int pin_s, const int *singular,
-             const int *done) {
-  if (t.lev[0].lpl == 32) mg_tail_k<32>(st, t, nm, lam, pin_s, singular, done);
-  else mg_tail_k<64>(st, t, nm, lam, pin_s, singular, done);
+void mg_tail(hipStream_t st, const MGTailT<T> &t, int nm, const MGTailEnds<T> &E, const T *lam, int pin_s,
+             const int *singular, const int *done) {
+  if (t.lev[0].lpl == 32) mg_tail_k<32>(st, t, nm, E, lam, pin_s, singular, done);
+  else mg_tail_k<64>(st, t, nm, E, lam, pin_s, singular, done);
 }
 
 template <typename T>
@@ -2036,8 +2094,9 @@ void mg_copy3(hipStream_t st, const double *src, long sm, long sa, long ss, doub
 
 #define SNAC_MG_INST(T)                                                                                               \
   template void mg_line<T>(hipStream_t, const MGLevT<T> &, const T *, T *, const T *, int, int, int, int, const int *, \
-                           const int *, const T *, int);                                                              \
-  template void mg_tail<T>(hipStream_t, const MGTailT<T> &, int, const T *, int, const int *, const int *);           \
+                           const int *, const T *, int, const MGEnds<T> &);                                           \
+  template void mg_tail<T>(hipStream_t, const MGTailT<T> &, int, const MGTailEnds<T> &, const T *, int, const int *,   \
+                           const int *);                                                                              \
   template void mg_restrict_residual<T>(hipStream_t, const MGLevT<T> &, const MGLevT<T> &, const T *, const T *,       \
                                         const T *, T *, const int *);                                                 \
   template void mg_prolong<T>(hipStream_t, const MGLevT<T> &, const MGLevT<T> &, const T *, T *, const int *);        \

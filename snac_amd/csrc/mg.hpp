@@ -56,6 +56,16 @@ struct MGLevT {
 };
 using MGLev = MGLevT<double>;
 
+// A level's odd periodic axes: the two end lines of such an axis are
+// neighbours of one colour, and the unfactored sweeps of that colour read
+// them here, as they were before the sweep (mg_save_ends): wa[m][2][s] of the
+// lines a = 0 and na - 1, wm[a][2][s] of m = 0 and nm - 1 (3D path); null
+// where the axis is even or not periodic
+template <typename T>
+struct MGEnds {
+  T *wa = nullptr, *wm = nullptr;
+};
+
 // A level's factored lines (FFT path, kernels_mgline.hip).  Columns with the
 // same coefficients form a class; each (mode, class) has one table of the
 // constants of a line's partitioned elimination, [entry][lane].  Absent (tab
@@ -98,6 +108,11 @@ struct MGTailT {
   int ox[MG_TAIL_MAX], ob[MG_TAIL_MAX];
   int lds_elems;
 };
+// the odd periodic levels' end lines (MGEnds::wa of each tail level)
+template <typename T>
+struct MGTailEnds {
+  T *wa[MG_TAIL_MAX] = {};
+};
 
 // the V-cycle hierarchy in one element type: levels, the per-mode
 // eigenvalues (null on the 3D path) and per-level x / b (level 0: z and r of
@@ -106,6 +121,8 @@ template <typename T>
 struct MGHier {
   std::vector<MGLevT<T>> lev;
   std::vector<MGFacT<T>> fac;  // per level
+  std::vector<MGEnds<T>> ends; // per level
+  MGTailEnds<T> tail_ends;
   const T *lam = nullptr;
   std::vector<T *> xl, bl;
   int tail0 = -1;           // first level handled by the fused tail kernel (-1: none)
@@ -116,8 +133,8 @@ struct MGHier {
 // V-cycle over the tail levels, one workgroup per mode (b of the first
 // tail level is given; x of every tail level is overwritten)
 template <typename T>
-void mg_tail(hipStream_t st, const MGTailT<T> &t, int nm, const T *lam, int pin_s, const int *singular,
-             const int *done);
+void mg_tail(hipStream_t st, const MGTailT<T> &t, int nm, const MGTailEnds<T> &E, const T *lam, int pin_s,
+             const int *singular, const int *done);
 // zebra line relaxation of the lines (m, a) with a % 2 == col_a (and, when
 // coupled, m % 2 == col_m); zero_nb: neighbouring lines read as zero;
 // pin_s >= 0: in singular groups row pin_s is replaced by x = 0; xc (FFT
@@ -125,7 +142,8 @@ void mg_tail(hipStream_t st, const MGTailT<T> &t, int nm, const T *lam, int pin_
 // next coarser level's x, cna columns) added, as mg_prolong would store it
 template <typename T>
 void mg_line(hipStream_t st, const MGLevT<T> &L, const T *lam, T *x, const T *b, int col_a, int col_m, int zero_nb,
-             int pin_s, const int *singular, const int *done, const T *xc = nullptr, int cna = 0);
+             int pin_s, const int *singular, const int *done, const T *xc = nullptr, int cna = 0,
+             const MGEnds<T> &E = MGEnds<T>());
 // the launched levels' line relaxation kernel: 0 reads each lane's rows
 // from memory directly, 1 stages the rows' right-hand sides and the new x
 // through LDS with coalesced loads and stores, 2 is 1 with a workgroup's
@@ -171,6 +189,11 @@ void mg_restrict_residual(hipStream_t st, const MGLevT<T> &F, const MGLevT<T> &C
 // coefficients and eigenvalues
 template <typename T>
 void mg_factor(hipStream_t st, const MGHier<T> &H, int nm, bool finest_only);
+// copies the end lines of the odd periodic axes to E: called before every
+// mg_line of their colour that reads its neighbours.  xc as xc0 of mg_line_fac
+template <typename T>
+void mg_save_ends(hipStream_t st, const MGLevT<T> &L, const MGEnds<T> &E, const T *x, const T *xc, int cna,
+                  const int *done);
 // mg_line with a level's factors; xc0: the coarse correction that lines of
 // this sweep's own colour still lack (read only across the ends of an odd
 // periodic axis)

@@ -11,21 +11,24 @@ __device__ __forceinline__ long vidx(const MGLevT<T> &L, int m, int a, int s) { 
 template <typename T>
 __device__ __forceinline__ long cidx(const MGLevT<T> &L, int m, int a, int s) { return m * L.qm + (long)a * L.ns + s; }
 
-// sum of the couplings to the neighbouring lines (a and m directions) times x
+// sum of the couplings to the neighbouring lines (a and m directions) times x;
+// wa, wm (a sweep on an odd periodic axis): row s of the line's entries of
+// MGEnds, which take the place of x across the axis' ends
 template <typename T>
-__device__ __forceinline__ T nb_sum(const MGLevT<T> &L, const T *__restrict__ x, int m, int a, long e, long q) {
+__device__ __forceinline__ T nb_sum(const MGLevT<T> &L, const T *__restrict__ x, int m, int a, long e, long q,
+                                    const T *wa = nullptr, const T *wm = nullptr) {
   T r = 0;
   const long sa = L.ns;
   if (a < L.na - 1) r += L.ca[q] * x[e + sa];
-  else if (L.per_a) r += L.ca[q] * x[e - (long)(L.na - 1) * sa];
+  else if (L.per_a) r += L.ca[q] * (wa ? wa[0] : x[e - (long)(L.na - 1) * sa]);
   if (a > 0) r += L.ca[q - sa] * x[e - sa];
-  else if (L.per_a) r += L.ca[q + (long)(L.na - 1) * sa] * x[e + (long)(L.na - 1) * sa];
+  else if (L.per_a) r += L.ca[q + (long)(L.na - 1) * sa] * (wa ? wa[sa] : x[e + (long)(L.na - 1) * sa]);
   if (L.coupled) {
     const long sm = (long)L.na * L.ns;
     if (m < L.nm - 1) r += L.cm[q] * x[e + sm];
-    else if (L.per_m) r += L.cm[q] * x[e - (long)(L.nm - 1) * sm];
+    else if (L.per_m) r += L.cm[q] * (wm ? wm[0] : x[e - (long)(L.nm - 1) * sm]);
     if (m > 0) r += L.cm[q - L.qm] * x[e - sm];
-    else if (L.per_m) r += L.cm[q + (long)(L.nm - 1) * L.qm] * x[e + (long)(L.nm - 1) * sm];
+    else if (L.per_m) r += L.cm[q + (long)(L.nm - 1) * L.qm] * (wm ? wm[sa] : x[e + (long)(L.nm - 1) * sm]);
   }
   return r;
 }

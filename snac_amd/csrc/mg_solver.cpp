@@ -532,6 +532,16 @@ void mg_plan(MGPlan &P, const Case &cs, int device, int comp) {
     }
     L.mlist = nullptr;
     L.mcount = nullptr;
+    const bool odd_a = h.per_a && h.na > 1 && h.na % 2 == 1, odd_m = h.per_m && h.nm > 1 && h.nm % 2 == 1;
+    auto ends = [&](auto &Hh, auto zero) {
+      using T = decltype(zero);
+      MGEnds<T> E;
+      if (odd_a) E.wa = dev_zeros<T>(P, (size_t)2 * h.nm * h.ns);
+      if (odd_m) E.wm = dev_zeros<T>(P, (size_t)2 * h.na * h.ns);
+      Hh.ends.push_back(E);
+    };
+    ends(P.h64, double());
+    ends(P.h32, float());
     P.h64.lev.push_back(L);
     MGLevT<float> Lf;
     Lf.nm = L.nm; Lf.na = L.na; Lf.ns = L.ns;
@@ -580,8 +590,8 @@ void mg_plan(MGPlan &P, const Case &cs, int device, int comp) {
       MGFacT<T> F;
       std::vector<int> cls, rep;
       if (!mg_fac_shape<T>(h.ns, F) || !column_classes<T>(h, cls, rep)) return;
-      // the unfactored kernels' bits need their split of the lines, and on an
-      // odd periodic axis their order of the two ends, which have one colour
+      // the unfactored kernels' bits need their split of the lines; FP32 has no
+      // factored sweep for the ends of an odd periodic axis
       if (sizeof(T) == 4 && (F.lpl != lpl || (h.per_a && h.na % 2 == 1 && h.na > 1))) return;
       F.ncls = (int)rep.size();
       const size_t n = (size_t)h.nm * F.ncls * mg_fac_entries(F.K, F.lpl) * F.lpl;
@@ -625,6 +635,7 @@ void mg_plan(MGPlan &P, const Case &cs, int device, int comp) {
     for (int q = 0; q < Hh.tail.nl; q++) {
       Hh.tail.lev[q] = Hh.lev[tail0 + q];
       Hh.tail.fac[q] = Hh.fac[tail0 + q];
+      Hh.tail_ends.wa[q] = Hh.ends[tail0 + q].wa;
       Hh.tail.x[q] = Hh.xl[tail0 + q];
       Hh.tail.b[q] = Hh.bl[tail0 + q];
       const int n = (Hh.lev[tail0 + q].na * Hh.lev[tail0 + q].ns + 3) / 4 * 4;  // 16-byte aligned blocks
@@ -695,7 +706,8 @@ void vcycle(MGPlan &P, MGHier<T> &H, hipStream_t st, size_t l) {
   const T *b = H.bl[l];
   if ((int)l == H.tail0) {  // the coarse end in one launch, one workgroup per mode
     if (P.mark_tail) P.mark_tail(true);
-    if (!mg_tail_fac(st, H.tail, P.ng, H.lam, P.done)) mg_tail(st, H.tail, P.ng, H.lam, P.pin_s, P.singular, P.done);
+    if (!mg_tail_fac(st, H.tail, P.ng, H.lam, P.done))
+      mg_tail(st, H.tail, P.ng, H.tail_ends, H.lam, P.pin_s, P.singular, P.done);
     if (P.mark_tail) P.mark_tail(false);
     return;
   }
@@ -721,13 +733,25 @@ void vcycle(MGPlan &P, MGHier<T> &H, hipStream_t st, size_t l) {
     mg_pair_up<T>(st, L, F, x, b, H.xl[l + 1], P.done);
     return;
   }
+  // a colour that holds both ends of an odd periodic axis, each the other's
+  // neighbour, is relaxed from their values before the sweep: a block Jacobi
+  // step within the colour (adjoint to the first sweep's from zero), and no
+  // line is read while it is written
+  const MGEnds<T> &E = H.ends[l];
+  auto save_ends = [&](const int (&cl)[2], const T *xc, int cna) {
+    if ((E.wa && cl[0] == 0) || (E.wm && cl[1] == 0)) mg_save_ends<T>(st, L, E, x, xc, cna, P.done);
+  };
   if (zero_first) mg_zero(st, (long)L.nm * L.na * L.ns, x);
   for (int k = 0; k < nc; k++) {
     const int znb = (!zero_first && k == 0) ? 1 : 0;
     const bool mk = l == 0 && znb == 0 && P.mark_line0;
     if (mk) P.mark_line0(true);
-    if (fac) mg_line_fac<T>(st, L, F, x, b, col[k][0], znb, P.done, nullptr, nullptr, 0);
-    else mg_line(st, L, H.lam, x, b, col[k][0], col[k][1], znb, -1, nullptr, P.done);
+    if (fac) {
+      mg_line_fac<T>(st, L, F, x, b, col[k][0], znb, P.done, nullptr, nullptr, 0);
+    } else {
+      if (!znb) save_ends(col[k], nullptr, 0);
+      mg_line(st, L, H.lam, x, b, col[k][0], col[k][1], znb, -1, nullptr, P.done, (const T *)nullptr, 0, E);
+    }
     if (mk) P.mark_line0(false);
   }
   // smooth_only: the finest level's symmetric zebra sweeps are the whole
@@ -753,12 +777,14 @@ void vcycle(MGPlan &P, MGHier<T> &H, hipStream_t st, size_t l) {
     const bool mk = l == 0 && P.mark_line0;
     if (mk) P.mark_line0(true);
     const bool pro = fuse && k == nc - 1;
-    if (fac)
+    if (fac) {
       mg_line_fac<T>(st, L, F, x, b, col[k][0], 0, P.done, pro ? (const T *)H.xl[l + 1] : nullptr,
                      coarse ? (const T *)H.xl[l + 1] : nullptr, coarse ? H.lev[l + 1].na : 0);
-    else
+    } else {
+      save_ends(col[k], fuse ? (const T *)H.xl[l + 1] : nullptr, fuse ? H.lev[l + 1].na : 0);
       mg_line(st, L, H.lam, x, b, col[k][0], col[k][1], 0, -1, nullptr, P.done, pro ? (const T *)H.xl[l + 1] : nullptr,
-              pro ? H.lev[l + 1].na : 0);
+              pro ? H.lev[l + 1].na : 0, E);
+    }
     if (mk) P.mark_line0(false);
   }
 }
