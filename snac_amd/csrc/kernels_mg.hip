@@ -828,18 +828,18 @@ __device__ __forceinline__ double wave_sum(double v) {
   return v;
 }
 
-// Group g's two sums from its chunks' partial sums, in the same order in
-// whichever kernel needs them: the CG passes reduce the partials of the pass
-// before them themselves (nchunk values, cache hits) instead of waiting for a
-// launch that does nothing else (4.3 us each, four per iteration).  Called by
-// every thread of the workgroup.
-__device__ __forceinline__ double2 part_sums(const double *__restrict__ part, int g, int nchunk) {
+// Group g's two sums from its n partial sums, in the same order in whichever
+// kernel needs them: the CG passes reduce the partials of the pass before
+// them themselves (cache hits) instead of waiting for a launch that does
+// nothing else, while there are few (MGPart).  Called by every thread of the
+// workgroup.
+__device__ __forceinline__ double2 part_sums(const double *__restrict__ part, int g, int n) {
   __shared__ double tot[2];
   if (threadIdx.x < 64) {
     double a = 0.0, b = 0.0;
-    for (int c = threadIdx.x; c < nchunk; c += 64) {
-      a += part[((long)g * nchunk + c) * 2];
-      b += part[((long)g * nchunk + c) * 2 + 1];
+    for (int c = threadIdx.x; c < n; c += 64) {
+      a += part[((long)g * n + c) * 2];
+      b += part[((long)g * n + c) * 2 + 1];
     }
     a = wave_sum(a);
     b = wave_sum(b);
@@ -1057,8 +1057,8 @@ __device__ __forceinline__ double cg_beta(int g, double rzn, const double *__res
 // group's ends forms its neighbour again.  Same values either way.
 template <typename TZ, typename TP, bool STAGE = false>
 __global__ __launch_bounds__(256) void k_dir_apply_dot(MGLev L, const double *__restrict__ lam, long gsize,
-                                                       const double *__restrict__ rzp, double *__restrict__ rzn,
-                                                       const double *__restrict__ rzo,
+                                                       const double *__restrict__ rzp, int nrz,
+                                                       double *__restrict__ rzn, const double *__restrict__ rzo,
                                                        const double *__restrict__ cross, const TZ *__restrict__ z,
                                                        const TP *__restrict__ pp, TP *__restrict__ p,
                                                        double *__restrict__ part, int nchunk,
@@ -1068,8 +1068,11 @@ __global__ __launch_bounds__(256) void k_dir_apply_dot(MGLev L, const double *__
   const int g = blockIdx.y;
   double s1 = 0.0;
   if (!done[g]) {
-    const double2 rz = part_sums(rzp, g, nchunk);
-    if (blockIdx.x == 0 && threadIdx.x == 0) { rzn[g * 2] = rz.x; rzn[g * 2 + 1] = rz.y; }  // for the passes after this one
+    const double2 rz = part_sums(rzp, g, nrz);
+    if (blockIdx.x == 0 && threadIdx.x == 0) {  // for the passes after this one
+      rzn[g * 2] = rz.x;
+      rzn[g * 2 + 1] = rz.y;
+    }
     const double be = cg_beta(g, rz.x, rzo, cross);
     auto pnew = [&](long e) -> double {
       if (be == 0.0) return (double)(TP)(double)z[e];
@@ -1141,8 +1144,8 @@ __global__ __launch_bounds__(256) void k_dir_apply_dot(MGLev L, const double *__
 // sums, as k_dir_apply_dot.
 template <typename TZ, typename TP>
 __global__ __launch_bounds__(256) void k_dir_apply_dot_lds(MGLev L, const double *__restrict__ lam, long gsize,
-                                                           const double *__restrict__ rzp, double *__restrict__ rzn,
-                                                           const double *__restrict__ rzo,
+                                                           const double *__restrict__ rzp, int nrz,
+                                                           double *__restrict__ rzn, const double *__restrict__ rzo,
                                                            const double *__restrict__ cross,
                                                            const TZ *__restrict__ z, const TP *__restrict__ pp,
                                                            TP *__restrict__ p, double *__restrict__ part, int nchunk,
@@ -1153,8 +1156,11 @@ __global__ __launch_bounds__(256) void k_dir_apply_dot_lds(MGLev L, const double
   const int g = blockIdx.y;
   double s1 = 0.0;
   if (!done[g]) {
-    const double2 rz = part_sums(rzp, g, nchunk);
-    if (blockIdx.x == 0 && threadIdx.x == 0) { rzn[g * 2] = rz.x; rzn[g * 2 + 1] = rz.y; }  // for the passes after this one
+    const double2 rz = part_sums(rzp, g, nrz);
+    if (blockIdx.x == 0 && threadIdx.x == 0) {  // for the passes after this one
+      rzn[g * 2] = rz.x;
+      rzn[g * 2 + 1] = rz.y;
+    }
     const double be = cg_beta(g, rz.x, rzo, cross);
     auto pn = [&](long e) -> TP {
       if (be == 0.0) return (TP)(double)z[e];
@@ -1213,8 +1219,8 @@ __global__ __launch_bounds__(256) void k_dir_apply_dot_lds(MGLev L, const double
 template <typename TP, bool STAGE = false>
 __global__ __launch_bounds__(256) void k_update_apply_dot(MGLev L, const double *__restrict__ lam, long gsize,
                                                           const double *__restrict__ rz,
-                                                          const double *__restrict__ pqp, double *__restrict__ x,
-                                                          const TP *__restrict__ p, double *__restrict__ r,
+                                                          const double *__restrict__ pqp, int npq,
+                                                          double *__restrict__ x, const TP *__restrict__ p, double *__restrict__ r,
                                                           float *__restrict__ rf, const float *__restrict__ zf,
                                                           double *__restrict__ part, int nchunk,
                                                           const int *__restrict__ done, int first) {
@@ -1223,7 +1229,7 @@ __global__ __launch_bounds__(256) void k_update_apply_dot(MGLev L, const double 
   const int g = blockIdx.y;
   double s1 = 0.0, s2 = 0.0;
   if (!done[g]) {
-    const double den = part_sums(pqp, g, nchunk).x;
+    const double den = part_sums(pqp, g, npq).x;
     // p.Mp > 0 for an SPD operator and p != 0; anything else (p = 0, or a
     // preconditioner output that is not usable) skips the step instead of
     // spreading an overflow or a NaN
@@ -1309,8 +1315,8 @@ __global__ __launch_bounds__(256) void k_update_apply_dot(MGLev L, const double 
 template <typename TP>
 __global__ __launch_bounds__(256) void k_update_apply_dot_lds(MGLev L, const double *__restrict__ lam, long gsize,
                                                               const double *__restrict__ rz,
-                                                              const double *__restrict__ pqp, double *__restrict__ x,
-                                                              const TP *__restrict__ p, double *__restrict__ r,
+                                                              const double *__restrict__ pqp, int npq,
+                                                              double *__restrict__ x, const TP *__restrict__ p, double *__restrict__ r,
                                                               float *__restrict__ rf, const float *__restrict__ zf,
                                                               double *__restrict__ part, int nchunk,
                                                               const int *__restrict__ done, int first) {
@@ -1320,7 +1326,7 @@ __global__ __launch_bounds__(256) void k_update_apply_dot_lds(MGLev L, const dou
   const int g = blockIdx.y;
   double s1 = 0.0, s2 = 0.0;
   if (!done[g]) {
-    const double den = part_sums(pqp, g, nchunk).x;
+    const double den = part_sums(pqp, g, npq).x;
     // as k_update_apply_dot: an unusable step length skips the step
     double al = den > 0.0 ? rz[g * 2] / den : 0.0;
     if (!(__builtin_fabs(al) < 1e300)) al = 0.0;
@@ -1529,7 +1535,8 @@ __global__ __launch_bounds__(FLAG_NT) void k_flags(int ng, const double *__restr
 // the null-space component that k_dot_rz takes off
 template <typename T>
 __global__ __launch_bounds__(256) void k_null_part(long gsize, const T *__restrict__ x, const int *__restrict__ glist,
-                                                   double *__restrict__ part, int nchunk, const int *__restrict__ done) {
+                                                   double *__restrict__ part, int nchunk,
+                                                   const int *__restrict__ done) {
   __shared__ double sh[4];
   const int g = glist[blockIdx.y];
   double s2 = 0.0;
@@ -1552,8 +1559,8 @@ __global__ __launch_bounds__(256) void k_null_part(long gsize, const T *__restri
 template <typename T>
 __global__ __launch_bounds__(256) void k_dot_rz(long gsize, const double *__restrict__ r, T *__restrict__ z,
                                                 double *__restrict__ part, int nchunk, const int *__restrict__ done,
-                                                const int *__restrict__ sing, const double *__restrict__ npart,
-                                                const double *__restrict__ nact,
+                                                const int *__restrict__ sing, const double *__restrict__ nullp,
+                                                int nnull, const double *__restrict__ nact,
                                                 const unsigned char *__restrict__ act) {
   __shared__ double sh[4];
   const int g = blockIdx.y;
@@ -1561,7 +1568,7 @@ __global__ __launch_bounds__(256) void k_dot_rz(long gsize, const double *__rest
   if (!(done && done[g])) {
     const long base = (long)g * gsize;
     if (sing && sing[g]) {
-      const T mean = (T)(part_sums(npart, g, nchunk).y / nact[g]);
+      const T mean = (T)(part_sums(nullp, g, nnull).y / nact[g]);
       for (long i = (long)blockIdx.x * 256 + threadIdx.x; i < gsize; i += (long)nchunk * 256) {
         T v = z[base + i];
         if (act[i]) {
@@ -1920,8 +1927,8 @@ void mg_cg_update_dot(hipStream_t st, int ng, long gsize, const double *rz, cons
 }
 
 template <typename TZ, typename TP>
-void mg_dir_apply_dot(hipStream_t st, const MGLev &L, const double *lam, int ng, long gsize, const double *rzp,
-                      double *rzn, const double *rzo, const double *cross, const TZ *z, const TP *p_prev, TP *p,
+void mg_dir_apply_dot(hipStream_t st, const MGLev &L, const double *lam, int ng, long gsize, MGPart rz, double *rzn,
+                      const double *rzo, const double *cross, const TZ *z, const TP *p_prev, TP *p,
                       double *part, int nchunk, const int *done) {
   // the LDS form where a level's coefficients do not depend on a, its rows
   // divide 256 and a chunk's lines with their two neighbours fit in 64 KB
@@ -1929,66 +1936,80 @@ void mg_dir_apply_dot(hipStream_t st, const MGLev &L, const double *lam, int ng,
   const size_t lds = L.ns > 0 ? (size_t)(csz / L.ns + 2) * L.ns * sizeof(TP) : 0;
   const size_t ldsg = (size_t)(csz + 2 * L.ns) * sizeof(TP);  // any 2D level: the chunk and a line on each side
   if (g_cg_lds && !L.coupled && L.auni && L.ns > 0 && 256 % L.ns == 0 && lds <= 64 * 1024)
-    hipLaunchKernelGGL((k_dir_apply_dot_lds<TZ, TP>), dim3(nchunk, ng), dim3(256), lds, st, L, lam, gsize, rzp, rzn, rzo,
-                       cross, z, p_prev, p, part, nchunk, done);
+    hipLaunchKernelGGL((k_dir_apply_dot_lds<TZ, TP>), dim3(nchunk, ng), dim3(256), lds, st, L, lam, gsize, rz.p,
+                       rz.n, rzn, rzo, cross, z, p_prev, p, part, nchunk, done);
   else if (g_cg_lds && !L.coupled && ldsg <= 64 * 1024)
-    hipLaunchKernelGGL((k_dir_apply_dot<TZ, TP, true>), dim3(nchunk, ng), dim3(256), ldsg, st, L, lam, gsize, rzp, rzn, rzo,
-                       cross, z, p_prev, p, part, nchunk, done);
+    hipLaunchKernelGGL((k_dir_apply_dot<TZ, TP, true>), dim3(nchunk, ng), dim3(256), ldsg, st, L, lam, gsize, rz.p,
+                       rz.n, rzn, rzo, cross, z, p_prev, p, part, nchunk, done);
   else
-    hipLaunchKernelGGL((k_dir_apply_dot<TZ, TP>), dim3(nchunk, ng), dim3(256), 0, st, L, lam, gsize, rzp, rzn, rzo, cross,
-                       z, p_prev, p, part, nchunk, done);
+    hipLaunchKernelGGL((k_dir_apply_dot<TZ, TP>), dim3(nchunk, ng), dim3(256), 0, st, L, lam, gsize, rz.p, rz.n,
+                       rzn, rzo, cross, z, p_prev, p, part, nchunk, done);
   SNAC_HIP(hipGetLastError());
 }
 
 template <typename TP>
 void mg_update_apply_dot(hipStream_t st, const MGLev &L, const double *lam, int ng, long gsize, const double *rz,
-                         const double *pqp, double *x, const TP *p, double *r, float *rf, const float *zf,
+                         MGPart pq, double *x, const TP *p, double *r, float *rf, const float *zf,
                          double *part, int nchunk, const int *done, bool first) {
   const long csz = ((gsize + nchunk - 1) / nchunk + 255) / 256 * 256;
   const size_t lds = L.ns > 0 ? (size_t)(csz / L.ns + 2) * L.ns * sizeof(TP) : 0;
   const size_t ldsg = (size_t)(csz + 2 * L.ns) * sizeof(TP);
   const int fi = first ? 1 : 0;
   if (g_cg_lds && !L.coupled && L.auni && L.ns > 0 && 256 % L.ns == 0 && lds <= 64 * 1024)
-    hipLaunchKernelGGL(k_update_apply_dot_lds<TP>, dim3(nchunk, ng), dim3(256), lds, st, L, lam, gsize, rz, pqp, x, p,
-                       r, rf, zf, part, nchunk, done, fi);
+    hipLaunchKernelGGL(k_update_apply_dot_lds<TP>, dim3(nchunk, ng), dim3(256), lds, st, L, lam, gsize, rz, pq.p,
+                       pq.n, x, p, r, rf, zf, part, nchunk, done, fi);
   else if (g_cg_lds && !L.coupled && ldsg <= 64 * 1024)
-    hipLaunchKernelGGL((k_update_apply_dot<TP, true>), dim3(nchunk, ng), dim3(256), ldsg, st, L, lam, gsize, rz, pqp, x,
-                       p, r, rf, zf, part, nchunk, done, fi);
+    hipLaunchKernelGGL((k_update_apply_dot<TP, true>), dim3(nchunk, ng), dim3(256), ldsg, st, L, lam, gsize, rz, pq.p,
+                       pq.n, x, p, r, rf, zf, part, nchunk, done, fi);
   else
-    hipLaunchKernelGGL(k_update_apply_dot<TP>, dim3(nchunk, ng), dim3(256), 0, st, L, lam, gsize, rz, pqp, x, p, r, rf,
-                       zf, part, nchunk, done, fi);
+    hipLaunchKernelGGL(k_update_apply_dot<TP>, dim3(nchunk, ng), dim3(256), 0, st, L, lam, gsize, rz, pq.p, pq.n,
+                       x, p, r, rf, zf, part, nchunk, done, fi);
   SNAC_HIP(hipGetLastError());
 }
 #define SNAC_INST(TZ, TP)                                                                                             \
-  template void mg_dir_apply_dot<TZ, TP>(hipStream_t, const MGLev &, const double *, int, long, const double *,       \
-                                         double *, const double *, const double *, const TZ *, const TP *, TP *,       \
-                                         double *, int, const int *);
+  template void mg_dir_apply_dot<TZ, TP>(hipStream_t, const MGLev &, const double *, int, long, MGPart, double *,     \
+                                         const double *, const double *, const TZ *, const TP *, TP *, double *,      \
+                                         int, const int *);
 SNAC_INST(double, double)
 SNAC_INST(float, double)
 SNAC_INST(float, float)
 #undef SNAC_INST
 template void mg_update_apply_dot<double>(hipStream_t, const MGLev &, const double *, int, long, const double *,
-                                          const double *, double *, const double *, double *, float *, const float *,
+                                          MGPart, double *, const double *, double *, float *, const float *,
                                           double *, int, const int *, bool);
 template void mg_update_apply_dot<float>(hipStream_t, const MGLev &, const double *, int, long, const double *,
-                                         const double *, double *, const float *, double *, float *, const float *,
+                                         MGPart, double *, const float *, double *, float *, const float *,
                                          double *, int, const int *, bool);
 
 template <typename T>
 void mg_dot_rz(hipStream_t st, const MGLev &L, int ng, long gsize, const double *r, T *z, double *part, int nchunk,
-               const int *done, const int *sing, const int *sing_list, int n_sing, double *npart, const double *nact) {
+               const int *done, const int *sing, const int *sing_list, int n_sing, double *npart, double *ntot,
+               const double *nact) {
+  MGPart nul;
   if (n_sing > 0) {
-    hipLaunchKernelGGL(k_null_part<T>, dim3(nchunk, n_sing), dim3(256), 0, st, gsize, z, sing_list, npart, nchunk, done);
+    hipLaunchKernelGGL(k_null_part<T>, dim3(nchunk, n_sing), dim3(256), 0, st, gsize, z, sing_list, npart, nchunk,
+                       done);
     SNAC_HIP(hipGetLastError());
+    nul = mg_gather(st, ng, npart, nchunk, ntot, done, sing);
   }
   hipLaunchKernelGGL(k_dot_rz<T>, dim3(nchunk, ng), dim3(256), 0, st, gsize, r, z, part, nchunk, done,
-                     n_sing > 0 ? sing : nullptr, npart, nact, L.act);
+                     n_sing > 0 ? sing : nullptr, nul.p, nul.n, nact, L.act);
   SNAC_HIP(hipGetLastError());
 }
-template void mg_dot_rz<double>(hipStream_t, const MGLev &, int, long, const double *, double *, double *, int,
-                                const int *, const int *, const int *, int, double *, const double *);
-template void mg_dot_rz<float>(hipStream_t, const MGLev &, int, long, const double *, float *, double *, int,
-                               const int *, const int *, const int *, int, double *, const double *);
+#define SNAC_INST(T)                                                                                                  \
+  template void mg_dot_rz<T>(hipStream_t, const MGLev &, int, long, const double *, T *, double *, int, const int *,   \
+                             const int *, const int *, int, double *, double *, const double *);
+SNAC_INST(double)
+SNAC_INST(float)
+#undef SNAC_INST
+
+MGPart mg_gather(hipStream_t st, int ng, const double *part, int nchunk, double *tot, const int *done,
+                 const int *only) {
+  if (nchunk <= MG_PART_MAX) return MGPart{part, nchunk};
+  hipLaunchKernelGGL(k_dot_final, dim3(ng), dim3(64), 0, st, part, nchunk, tot, done, only);
+  SNAC_HIP(hipGetLastError());
+  return MGPart{tot, 1};
+}
 
 void mg_set_shift(MGPlan &P, hipStream_t st, double shift) {
   if (P.comp < 0 || !P.lam_base) return;

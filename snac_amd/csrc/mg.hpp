@@ -239,27 +239,46 @@ void mg_warm_residual(hipStream_t st, int ng, long gsize, const double *bb, doub
 void mg_cg_update_dot(hipStream_t st, int ng, long gsize, const double *rz, const double *pq, double *x,
                       const double *p, double *r, const double *q, float *rf, const float *zf, double *part,
                       int nchunk, double *out, const int *done);
+// A group's partial sums as the next pass reads them, n per group.
+struct MGPart {
+  const double *p = nullptr;
+  int n = 0;
+};
+// The partials of a pass for the next one: as they are up to MG_PART_MAX per
+// group, where every workgroup of the next pass adds them up itself, beyond
+// that added up into tot by a launch of their own, in the same order.  The
+// workgroups' sums cost n loads in each of n workgroups of a group, the launch
+// and its one wavefront about 2 us; four such sums an iteration.  A group is
+// a mode's plane (32 partials at 512 x 128, 256 at 1024 x 512), or the whole
+// 3D problem without an FFT axis.  ms a step, the launch / the workgroups:
+// 64 partials (512 x 256, 4 modes) 4.67 / 4.47, 256 (16 modes) 20.0 / 19.7,
+// 288 (3D, 96 x 64 x 96) 86.9 / 86.0, 1024 143.2 / 142.7 (both within their
+// spread), 2048 201.1 / 202.0, 4096 (256 x 128 x 256) 359.6 / 369.6.
+constexpr int MG_PART_MAX = 1024;
+MGPart mg_gather(hipStream_t st, int ng, const double *part, int nchunk, double *tot, const int *done,
+                 const int *only = nullptr);
 // the preconditioned residual z freed of its null-space component (the
-// singular groups' mean over their active cells, partial sums in npart), and
-// the partial sums of r.z per group
+// singular groups' mean over their active cells, partial sums in npart, ntot
+// for mg_gather), and the partial sums of r.z per group
 template <typename T>
 void mg_dot_rz(hipStream_t st, const MGLev &L, int ng, long gsize, const double *r, T *z, double *part, int nchunk,
-               const int *done, const int *sing, const int *sing_list, int n_sing, double *npart, const double *nact);
+               const int *done, const int *sing, const int *sing_list, int n_sing, double *npart, double *ntot,
+               const double *nact);
 // the CG's direction update and operator in one pass: p = z + beta p_prev
 // (beta as mg_cg_dir; p stored as TP, p_prev and p distinct buffers) and the
-// partial sums of p . (M p) per group.  rzp: mg_dot_rz's partials, whose sums
-// are stored in rzn as well
+// partial sums of p . (M p) per group.  rz: mg_dot_rz's sums, stored in rzn
+// as well
 template <typename TZ, typename TP>
-void mg_dir_apply_dot(hipStream_t st, const MGLev &L, const double *lam, int ng, long gsize, const double *rzp,
-                      double *rzn, const double *rzo, const double *cross, const TZ *z, const TP *p_prev, TP *p,
+void mg_dir_apply_dot(hipStream_t st, const MGLev &L, const double *lam, int ng, long gsize, MGPart rz, double *rzn,
+                      const double *rzo, const double *cross, const TZ *z, const TP *p_prev, TP *p,
                       double *part, int nchunk, const int *done);
 // mg_cg_update_dot with q = M p recomputed from p instead of read, p.q from
-// mg_dir_apply_dot's partials pqp, and its sums left as partials (mg_flags
+// mg_dir_apply_dot's partials, and its sums left as partials (mg_flags
 // adds them up).  first: the solve's first step from x = 0, x not read (x =
 // alpha p) and set to 0 on the groups that are already done
 template <typename TP>
 void mg_update_apply_dot(hipStream_t st, const MGLev &L, const double *lam, int ng, long gsize, const double *rz,
-                         const double *pqp, double *x, const TP *p, double *r, float *rf, const float *zf,
+                         MGPart pq, double *x, const TP *p, double *r, float *rf, const float *zf,
                          double *part, int nchunk, const int *done, bool first = false);
 void mg_izero(hipStream_t st, long n, int *x);
 // dst = (float) src
@@ -356,6 +375,7 @@ struct MGPlan {
   double *pd[2] = {nullptr, nullptr};
   float *pf[2] = {nullptr, nullptr};
   double *part = nullptr, *part_rz = nullptr, *part_pq = nullptr, *part_null = nullptr;  // per chunk and group
+  double *tot = nullptr, *tot_rz = nullptr, *tot_pq = nullptr, *tot_null = nullptr;      // their sums (mg_gather)
   double *bb = nullptr, *rr = nullptr, *pq = nullptr, *rz[2] = {nullptr, nullptr}, *sums = nullptr;
   double *nact = nullptr;
   int *done = nullptr, *singular = nullptr, *left = nullptr, *left_host = nullptr;

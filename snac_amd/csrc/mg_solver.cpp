@@ -652,6 +652,10 @@ void mg_plan(MGPlan &P, const Case &cs, int device, int comp) {
   P.part_rz = dev_zeros<double>(P, (size_t)2 * P.ng * P.nchunk);
   P.part_pq = dev_zeros<double>(P, (size_t)2 * P.ng * P.nchunk);
   P.part_null = dev_zeros<double>(P, (size_t)2 * P.ng * P.nchunk);
+  P.tot = dev_zeros<double>(P, 2 * P.ng);
+  P.tot_rz = dev_zeros<double>(P, 2 * P.ng);
+  P.tot_pq = dev_zeros<double>(P, 2 * P.ng);
+  P.tot_null = dev_zeros<double>(P, 2 * P.ng);
   P.bb = dev_zeros<double>(P, 2 * P.ng);
   P.rr = dev_zeros<double>(P, 2 * P.ng);
   P.pq = dev_zeros<double>(P, 2 * P.ng);
@@ -811,11 +815,11 @@ void precondition(MGPlan &P, hipStream_t st, bool net, const double *rr) {
       vcycle(P, P.h32, st, 0);
     }
     mg_dot_rz<float>(st, L0, P.ng, P.gsize, P.r, P.zf, P.part_rz, P.nchunk, P.done, P.singular, P.sing_list,
-                     P.any_singular ? P.n_sing : 0, P.part_null, P.nact);
+                     P.any_singular ? P.n_sing : 0, P.part_null, P.tot_null, P.nact);
   } else {
     vcycle(P, P.h64, st, 0);
     mg_dot_rz<double>(st, L0, P.ng, P.gsize, P.r, P.z, P.part_rz, P.nchunk, P.done, P.singular, P.sing_list,
-                      P.any_singular ? P.n_sing : 0, P.part_null, P.nact);
+                      P.any_singular ? P.n_sing : 0, P.part_null, P.tot_null, P.nact);
   }
 }
 
@@ -843,33 +847,27 @@ void mg_iteration(MGPlan &P, hipStream_t st, MGRun &R) {
   // in FP32; the network's need not be (an untrained one's directions grow
   // past the FP32 range), so the learned mode keeps FP64 directions.
   const MGLev &L0 = P.h64.lev[0];
-  if (mixed && P.prec == 1) {
-    mg_dir_apply_dot<float, float>(st, L0, P.h64.lam, P.ng, P.gsize, P.part_rz, P.rz[R.cur], rzo, rzo ? P.rr : nullptr, P.zf,
-                                   P.pf[R.pc], P.pf[1 - R.pc], P.part_pq, P.nchunk, P.done);
+  const MGPart rz = mg_gather(st, P.ng, P.part_rz, P.nchunk, P.tot_rz, P.done);
+  double *rzn = P.rz[R.cur];
+  const double *cross = rzo ? P.rr : nullptr;
+  // the direction pass from z and the previous directions, then the update pass
+  auto passes = [&](auto *z, auto *const (&p)[2], const double *crs, float *rf, const float *zf) {
+    using TP = std::remove_pointer_t<std::remove_reference_t<decltype(p[0])>>;
+    mg_dir_apply_dot(st, L0, P.h64.lam, P.ng, P.gsize, rz, rzn, rzo, crs, z, p[R.pc], p[1 - R.pc], P.part_pq, P.nchunk,
+                     P.done);
     R.pc = 1 - R.pc;
+    const MGPart pq = mg_gather(st, P.ng, P.part_pq, P.nchunk, P.tot_pq, P.done);
     if (P.mark_update) P.mark_update(true);
-    mg_update_apply_dot<float>(st, L0, P.h64.lam, P.ng, P.gsize, P.rz[R.cur], P.part_pq, P.x, P.pf[R.pc], P.r, P.rf, P.zf,
-                               P.part, P.nchunk, P.done, R.x_unset);
+    mg_update_apply_dot<TP>(st, L0, P.h64.lam, P.ng, P.gsize, rzn, pq, P.x, p[R.pc], P.r, rf, zf, P.part, P.nchunk,
+                            P.done, R.x_unset);
     if (P.mark_update) P.mark_update(false);
-  } else if (mixed) {
-    mg_dir_apply_dot<float, double>(st, L0, P.h64.lam, P.ng, P.gsize, P.part_rz, P.rz[R.cur], rzo, rzo ? P.rr : nullptr, P.zf,
-                                    P.pd[R.pc], P.pd[1 - R.pc], P.part_pq, P.nchunk, P.done);
-    R.pc = 1 - R.pc;
-    if (P.mark_update) P.mark_update(true);
-    mg_update_apply_dot<double>(st, L0, P.h64.lam, P.ng, P.gsize, P.rz[R.cur], P.part_pq, P.x, P.pd[R.pc], P.r, P.rf,
-                                P.zf, P.part, P.nchunk, P.done, R.x_unset);
-    if (P.mark_update) P.mark_update(false);
-  } else {
-    mg_dir_apply_dot<double, double>(st, L0, P.h64.lam, P.ng, P.gsize, P.part_rz, P.rz[R.cur], rzo, nullptr, P.z, P.pd[R.pc],
-                                     P.pd[1 - R.pc], P.part_pq, P.nchunk, P.done);
-    R.pc = 1 - R.pc;
-    if (P.mark_update) P.mark_update(true);
-    mg_update_apply_dot<double>(st, L0, P.h64.lam, P.ng, P.gsize, P.rz[R.cur], P.part_pq, P.x, P.pd[R.pc], P.r, nullptr,
-                                nullptr, P.part, P.nchunk, P.done, R.x_unset);
-    if (P.mark_update) P.mark_update(false);
-  }
+  };
+  if (mixed && P.prec == 1) passes(P.zf, P.pf, cross, P.rf, P.zf);
+  else if (mixed) passes(P.zf, P.pd, cross, P.rf, P.zf);
+  else passes(P.z, P.pd, nullptr, nullptr, nullptr);
   R.x_unset = false;  // written by this iteration's update pass
-  mg_flags(st, P.ng, P.part, P.nchunk, P.rr, P.bb, P.tol * P.tol, P.done, P.left, P.mlist, R.it + 1);
+  const MGPart rr = mg_gather(st, P.ng, P.part, P.nchunk, P.tot, P.done);
+  mg_flags(st, P.ng, rr.p, rr.n, P.rr, P.bb, P.tol * P.tol, P.done, P.left, P.mlist, R.it + 1);
   if (R.net && P.fallback) launch_net_stall(st, P.ng, P.rr, P.rr_prev, P.done, P.stall_ratio * P.stall_ratio, P.stall);
   R.it++;
 }
