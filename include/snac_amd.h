@@ -356,7 +356,9 @@ int snac_mg_line_choices(snac_ctx *ctx, int *fp64, int *fp32, int n);
  * the next lower variant), a negative value (the default) each level's
  * fastest, timed when the MG-PCG plan is set up and kept per level shape
  * for the process; 0..2 compute the same values, 3 and 4 the same systems
- * in another elimination order.  No counterpart in the reference.          */
+ * in another elimination order.  While a variant is forced no level and no
+ * coarse end runs from precomputed line factors.  No counterpart in the
+ * reference.                                                               */
 /* SNAC_KV_MG_RCP (process-wide): 1 (the default) makes the mode-batched MG
  * line sweeps divide by refined hardware reciprocals (within a few ulp of
  * the IEEE quotient); 0 divides by IEEE quotients, as the other line kernels

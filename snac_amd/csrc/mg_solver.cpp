@@ -710,7 +710,7 @@ void vcycle(MGPlan &P, MGHier<T> &H, hipStream_t st, size_t l) {
   const T *b = H.bl[l];
   if ((int)l == H.tail0) {  // the coarse end in one launch, one workgroup per mode
     if (P.mark_tail) P.mark_tail(true);
-    if (!mg_tail_fac(st, H.tail, P.ng, H.lam, P.done))
+    if (mg_line_variant() >= 0 || !mg_tail_fac(st, H.tail, P.ng, H.lam, P.done))
       mg_tail(st, H.tail, P.ng, H.tail_ends, H.lam, P.pin_s, P.singular, P.done);
     if (P.mark_tail) P.mark_tail(false);
     return;
