@@ -330,12 +330,16 @@ int snac_get_timing(snac_ctx *ctx, double *ms, int *count);
  * above) and the best times in ms.  No
  * counterpart in the reference (its FFTW plans use FFTW_ESTIMATE).          */
 int snac_get_autotune(snac_ctx *ctx, int *choices, double *ms, int n);
-/* the MG-PCG line relaxation kernel each level runs (SNAC_KV_MG_LINE
- * numbering, chosen by timing when the MG-PCG plan is set up; 5: lines from
- * precomputed factors, FP64 levels with few kinds of columns), for levels
- * 0..n-1 of the FP64 and of the FP32 V-cycle; -1 for levels in the fused
- * coarse-end kernel, past the last level, or before the MG-PCG path is
- * planned (either pointer may be null).  No counterpart in the reference. */
+/* the MG-PCG line relaxation chosen for each level (SNAC_KV_MG_LINE
+ * numbering, by timing when the MG-PCG plan is set up), for levels 0..n-1 of
+ * the FP64 and of the FP32 V-cycle; -1 for levels in the fused coarse-end
+ * kernel, past the last level, or before the MG-PCG path is planned (either
+ * pointer may be null).  FP64 levels with few kinds of columns run from
+ * precomputed line factors and say 5.  The FP32 entries 0..2 name the kernel
+ * whose values are computed: a level with few kinds of columns computes them
+ * from factors.  Where all columns of a level are alike both colours share a
+ * launch, in either precision; SNAC_PH_MG_LINE0 then counts one interval a
+ * V-cycle instead of three.  No counterpart in the reference.              */
 int snac_mg_line_choices(snac_ctx *ctx, int *fp64, int *fp32, int n);
 /* overrides an autotuned kernel variant: SNAC_KV_RK_MOM (0..16, as above),
  * SNAC_KV_TRIDIAG (0: c' in LDS, lines up to 128; 1: c' in scratch; 2:
@@ -357,8 +361,9 @@ int snac_mg_line_choices(snac_ctx *ctx, int *fp64, int *fp32, int n);
  * fastest, timed when the MG-PCG plan is set up and kept per level shape
  * for the process; 0..2 compute the same values, 3 and 4 the same systems
  * in another elimination order.  While a variant is forced no level and no
- * coarse end runs from precomputed line factors.  No counterpart in the
- * reference.                                                               */
+ * coarse end runs from precomputed line factors; an MG-PCG plan set up
+ * meanwhile takes it as its levels' choice without timing.  No counterpart
+ * in the reference.                                                        */
 /* SNAC_KV_MG_RCP (process-wide): 1 (the default) makes the mode-batched MG
  * line sweeps divide by refined hardware reciprocals (within a few ulp of
  * the IEEE quotient); 0 divides by IEEE quotients, as the other line kernels

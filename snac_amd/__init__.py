@@ -412,9 +412,10 @@ class Context:
 
     def mg_line_choices(self):
         """Per level of the FP64 and of the FP32 V-cycle, the line relaxation
-        kernel it runs (set_mg_line_variant's numbering; 5: precomputed line
-        factors; -1: a level of the fused coarse end, or the MG-PCG path not
-        planned yet)."""
+        kernel chosen (set_mg_line_variant's numbering; 5: precomputed line
+        factors; FP32: the kernel whose values are computed, from factors where
+        the level has them; -1: a level of the fused coarse end, or the MG-PCG
+        path not planned yet)."""
         a = np.zeros(32, np.int32)
         b = np.zeros(32, np.int32)
         _check(lib.snac_mg_line_choices(self.h, a, b, 32), "mg_line_choices")
@@ -438,7 +439,8 @@ class Context:
         the same systems in another elimination order); a negative value
         (the default) restores each level's fastest, timed at set-up (FP64
         levels with few kinds of columns: their precomputed line factors,
-        reported as 5).  0..2 compute the same values."""
+        reported as 5).  0..2 compute the same values.  A plan set up while
+        a variant is forced takes it as its levels' choice."""
         _check(lib.snac_set_kernel_variant(self.h, 4, int(v)), "set_kernel_variant")
 
     def set_mg_tail_lds(self, on):

@@ -1027,6 +1027,18 @@ void tune_hier(MGPlan &P, MGHier<T> &H, hipStream_t st) {
   const int last = H.tail0 >= 0 ? H.tail0 : nl - 1;  // launched levels that relax lines and restrict
   int dev = 0;
   SNAC_HIP(hipGetDevice(&dev));
+  // the variant a level runs when v is asked for (the next lower one it allows)
+  auto runs_as = [&](int l, int v) {
+    while (v > 0 && !mg_line_variant_runs(H.lev[l], v)) v--;
+    return v;
+  };
+  // under a forced variant every candidate would run that kernel: it is the
+  // levels' choice, and nothing is timed or kept for later plans
+  if (const int forced = mg_line_variant(); forced >= 0) {
+    for (int l = 0; l < last; l++)
+      H.lev[l].lvar = sizeof(T) == 8 && H.fac[l].tab ? 5 : (H.lev[l].na >= 2 ? runs_as(l, forced) : -1);
+    return;
+  }
   std::lock_guard<std::mutex> lk(g_line_mu);
   const std::string key = hier_key(H, dev);
   auto it = g_line_choice.find(key);
@@ -1058,11 +1070,6 @@ void tune_hier(MGPlan &P, MGHier<T> &H, hipStream_t st) {
       float ms = 0.f;
       SNAC_HIP(hipEventElapsedTime(&ms, e0, e1));
       return ms;
-    };
-    // the variant a level runs when v is asked for (the next lower one it allows)
-    auto runs_as = [&](int l, int v) {
-      while (v > 0 && !mg_line_variant_runs(H.lev[l], v)) v--;
-      return v;
     };
     // untimed V-cycles first: the clocks of an idle GPU ramp up under load,
     // and latency-bound and throughput-bound kernels gain differently
