@@ -8,6 +8,7 @@
 // in 0.03 ms instead of 7.8 ms.
 #include "hostcopy.hpp"
 
+#include <climits>
 #include <cstring>
 #include <exception>
 #include <mutex>
@@ -58,7 +59,7 @@ void HostCopy::run(int device, hipStream_t st, double *dev, long pitch, long w, 
                    const double *from_host) {
   if (!to_host && !from_host) throw std::runtime_error("null host array");
   if (w <= 0 || rows <= 0) return;
-  if (w > CHUNK * 64) throw std::runtime_error("field copy: row too long");
+  if (w > INT_MAX) throw std::runtime_error("field copy: row too long");  // k_pack_rows counts within w + CHUNK in 32 bits
   const long n = w * rows, nchunk = (n + CHUNK - 1) / CHUNK;
   // one thread keeps up with the link while the caller's pages are mapped; a
   // fresh array's page faults take about 0.1 ms per MiB and thread, so from
