@@ -485,6 +485,15 @@ void plan_mg(snac_ctx *c) {
   finish_mg_plan(c, P);
 }
 
+// the transforms of the mixed and learned modes (their dense tables hold n^2
+// values where the length has no power-of-two FFT), made when such a mode is
+// first in use; not during graph capture
+void mg_row_plans(snac_ctx *c, MGPlan &P) {
+  if (!P.ok || c->device < 0 || P.fa < 0 || c->prec == SNAC_PREC_FP64) return;
+  P.fwd_row = r2r_plan(P.kind_fwd, P.ng, true);
+  P.bwd_row = r2r_plan(P.kind_bwd, P.ng, true);
+}
+
 // after mg_plan: each level's fastest line kernel, the FFT-axis transforms
 // and the bounding-box work array (a Helmholtz plan shares the pressure
 // plan's: the solves run one after the other on the context's stream)
@@ -495,8 +504,7 @@ void finish_mg_plan(snac_ctx *c, MGPlan &P) {
   // staggered along a bounded FFT axis)
   P.fwd = r2r_plan(P.kind_fwd, P.ng);
   P.bwd = r2r_plan(P.kind_bwd, P.ng);
-  P.fwd_row = r2r_plan(P.kind_fwd, P.ng, true);
-  P.bwd_row = r2r_plan(P.kind_bwd, P.ng, true);
+  mg_row_plans(c, P);
   if (P.comp >= 0) {
     plan_mg(c);
     if (c->mg.ok && c->mg.ph) {
@@ -1658,6 +1666,9 @@ int snac_set_precision(snac_ctx *c, int mode) {
     c->st32 = st32;
     c->prec = mode;
     c->mg.prec = mode;
+    if (c->mg_planned) mg_row_plans(c, c->mg);
+    for (auto &f : c->imp)
+      if (f.mg) mg_row_plans(c, *f.mg);
     c->mg.fixed_iters = 0;  // the graph's CG counts are measured again
     c->mg.max_seen = 0;
     for (auto &f : c->imp)
