@@ -1220,7 +1220,8 @@ template <typename TP, bool STAGE = false>
 __global__ __launch_bounds__(256) void k_update_apply_dot(MGLev L, const double *__restrict__ lam, long gsize,
                                                           const double *__restrict__ rz,
                                                           const double *__restrict__ pqp, int npq,
-                                                          double *__restrict__ x, const TP *__restrict__ p, double *__restrict__ r,
+                                                          double *__restrict__ x, const TP *__restrict__ p,
+                                                          double *__restrict__ r,
                                                           float *__restrict__ rf, const float *__restrict__ zf,
                                                           double *__restrict__ part, int nchunk,
                                                           const int *__restrict__ done, int first) {
@@ -1316,7 +1317,8 @@ template <typename TP>
 __global__ __launch_bounds__(256) void k_update_apply_dot_lds(MGLev L, const double *__restrict__ lam, long gsize,
                                                               const double *__restrict__ rz,
                                                               const double *__restrict__ pqp, int npq,
-                                                              double *__restrict__ x, const TP *__restrict__ p, double *__restrict__ r,
+                                                              double *__restrict__ x, const TP *__restrict__ p,
+                                                          double *__restrict__ r,
                                                               float *__restrict__ rf, const float *__restrict__ zf,
                                                               double *__restrict__ part, int nchunk,
                                                               const int *__restrict__ done, int first) {
@@ -1453,11 +1455,10 @@ __global__ __launch_bounds__(256) void k_sub_mean(MGLev L, T *__restrict__ x, co
 }
 
 // one workgroup: sums the groups' residual norms (part: the update pass's
-// partials, else rr holds them), updates the done flags, counts the groups
-// left and (list) writes them in increasing order, 1024 groups per round
-// (ballot + popcount positions within a wavefront, wavefront totals through
-// LDS).  Latency-bound: each wavefront has the loads of four groups in
-// flight, and the flags pass to the ballot through LDS.
+// partials, a wavefront per group; else rr holds them), updates the done
+// flags, counts the groups left and (list) writes them in increasing order,
+// 1024 groups per round (ballot + popcount positions within a wavefront,
+// wavefront totals through LDS).  Latency-bound.
 constexpr int FLAG_NT = 1024, FLAG_W = FLAG_NT / 64;
 __global__ __launch_bounds__(FLAG_NT) void k_flags(int ng, const double *__restrict__ part, int nchunk,
                                                    double *__restrict__ rr, const double *__restrict__ bb, double tol2,
@@ -1469,40 +1470,20 @@ __global__ __launch_bounds__(FLAG_NT) void k_flags(int ng, const double *__restr
   for (int g0 = 0; g0 < ng; g0 += FLAG_NT) {
     const int n = min(ng - g0, FLAG_NT);
     if (part) {
-      constexpr int U = 4;
-      for (int q0 = wv; q0 < n; q0 += FLAG_W * U) {
-        double a[U], b[U], lim[U];
-        int dn[U];
-#pragma unroll
-        for (int u = 0; u < U; u++) {
-          const int q = q0 + u * FLAG_W;
-          const long g = g0 + min(q, n - 1);
-          a[u] = b[u] = 0.0;
-          dn[u] = done[g];
-          lim[u] = tol2 * bb[g * 2];
-          if (lane < nchunk) {
-            a[u] = part[(g * nchunk + lane) * 2];
-            b[u] = part[(g * nchunk + lane) * 2 + 1];
-          }
+      for (int q = wv; q < n; q += FLAG_W) {
+        const long g = g0 + q;
+        double a = 0.0, b = 0.0;
+        for (int c = lane; c < nchunk; c += 64) {
+          a += part[(g * nchunk + c) * 2];
+          b += part[(g * nchunk + c) * 2 + 1];
         }
-        for (int c = lane + 64; c < nchunk; c += 64)
-#pragma unroll
-          for (int u = 0; u < U; u++) {
-            const long g = g0 + min(q0 + u * FLAG_W, n - 1);
-            a[u] += part[(g * nchunk + c) * 2];
-            b[u] += part[(g * nchunk + c) * 2 + 1];
-          }
-#pragma unroll
-        for (int u = 0; u < U; u++) {
-          const int q = q0 + u * FLAG_W, g = g0 + q;
-          const double ta = wave_sum(a[u]), tb = wave_sum(b[u]);
-          if (lane != 0 || q >= n) continue;
-          // a group that is done keeps its values
-          if (!dn[u]) { rr[g * 2] = ta; rr[g * 2 + 1] = tb; }
-          const bool now = !dn[u] && ta <= lim[u];
-          if (now) done[g] = 1;
-          live[q] = !dn[u] && !now;
-        }
+        a = wave_sum(a);
+        b = wave_sum(b);
+        if (lane != 0) continue;
+        const bool was = done[g], now = !was && a <= tol2 * bb[g * 2];
+        if (!was) { rr[g * 2] = a; rr[g * 2 + 1] = b; }  // a group that is done keeps its values
+        if (now) done[g] = 1;
+        live[q] = !was && !now;
       }
     } else if ((int)threadIdx.x < n) {
       const int g = g0 + threadIdx.x;
@@ -2004,8 +1985,8 @@ SNAC_INST(float)
 #undef SNAC_INST
 
 MGPart mg_gather(hipStream_t st, int ng, const double *part, int nchunk, double *tot, const int *done,
-                 const int *only) {
-  if (nchunk <= MG_PART_MAX) return MGPart{part, nchunk};
+                 const int *only, bool launch) {
+  if (!launch && nchunk <= MG_PART_MAX) return MGPart{part, nchunk};
   hipLaunchKernelGGL(k_dot_final, dim3(ng), dim3(64), 0, st, part, nchunk, tot, done, only);
   SNAC_HIP(hipGetLastError());
   return MGPart{tot, 1};

@@ -255,8 +255,13 @@ struct MGPart {
 // 288 (3D, 96 x 64 x 96) 86.9 / 86.0, 1024 143.2 / 142.7 (both within their
 // spread), 2048 201.1 / 202.0, 4096 (256 x 128 x 256) 359.6 / 369.6.
 constexpr int MG_PART_MAX = 1024;
+// mg_flags, one workgroup for all groups, adds up the norms of this many at
+// most; more take the launch (launch true).  ms a step, the launch / the
+// workgroup: 4 modes 4.51 / 4.49 (512 x 256), 8 equal, 16 5.69 / 5.78, 64 5.87
+// / 5.95 (512 x 128), 256 29.0 / 29.4 (512 x 256).
+constexpr int MG_FLAG_GROUPS = 8;
 MGPart mg_gather(hipStream_t st, int ng, const double *part, int nchunk, double *tot, const int *done,
-                 const int *only = nullptr);
+                 const int *only = nullptr, bool launch = false);
 // the preconditioned residual z freed of its null-space component (the
 // singular groups' mean over their active cells, partial sums in npart, ntot
 // for mg_gather), and the partial sums of r.z per group
@@ -375,7 +380,7 @@ struct MGPlan {
   double *pd[2] = {nullptr, nullptr};
   float *pf[2] = {nullptr, nullptr};
   double *part = nullptr, *part_rz = nullptr, *part_pq = nullptr, *part_null = nullptr;  // per chunk and group
-  double *tot = nullptr, *tot_rz = nullptr, *tot_pq = nullptr, *tot_null = nullptr;      // their sums (mg_gather)
+  double *tot_rz = nullptr, *tot_pq = nullptr, *tot_null = nullptr;                      // their sums (mg_gather)
   double *bb = nullptr, *rr = nullptr, *pq = nullptr, *rz[2] = {nullptr, nullptr}, *sums = nullptr;
   double *nact = nullptr;
   int *done = nullptr, *singular = nullptr, *left = nullptr, *left_host = nullptr;

@@ -652,7 +652,6 @@ void mg_plan(MGPlan &P, const Case &cs, int device, int comp) {
   P.part_rz = dev_zeros<double>(P, (size_t)2 * P.ng * P.nchunk);
   P.part_pq = dev_zeros<double>(P, (size_t)2 * P.ng * P.nchunk);
   P.part_null = dev_zeros<double>(P, (size_t)2 * P.ng * P.nchunk);
-  P.tot = dev_zeros<double>(P, 2 * P.ng);
   P.tot_rz = dev_zeros<double>(P, 2 * P.ng);
   P.tot_pq = dev_zeros<double>(P, 2 * P.ng);
   P.tot_null = dev_zeros<double>(P, 2 * P.ng);
@@ -866,8 +865,8 @@ void mg_iteration(MGPlan &P, hipStream_t st, MGRun &R) {
   else if (mixed) passes(P.zf, P.pd, cross, P.rf, P.zf);
   else passes(P.z, P.pd, nullptr, nullptr, nullptr);
   R.x_unset = false;  // written by this iteration's update pass
-  const MGPart rr = mg_gather(st, P.ng, P.part, P.nchunk, P.tot, P.done);
-  mg_flags(st, P.ng, rr.p, rr.n, P.rr, P.bb, P.tol * P.tol, P.done, P.left, P.mlist, R.it + 1);
+  const MGPart rr = mg_gather(st, P.ng, P.part, P.nchunk, P.rr, P.done, nullptr, P.ng > MG_FLAG_GROUPS);
+  mg_flags(st, P.ng, rr.p == P.rr ? nullptr : rr.p, rr.n, P.rr, P.bb, P.tol * P.tol, P.done, P.left, P.mlist, R.it + 1);
   if (R.net && P.fallback) launch_net_stall(st, P.ng, P.rr, P.rr_prev, P.done, P.stall_ratio * P.stall_ratio, P.stall);
   R.it++;
 }

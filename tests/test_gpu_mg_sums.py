@@ -21,3 +21,16 @@ def test_partial_sums(tmp_path, nz, prec):
     assert relres <= 1e-13
     # stops at 1e-13 of the right-hand side; the pressure's condition takes the rest
     assert np.linalg.norm(got - ref) <= 1e-10 * np.linalg.norm(ref), it
+
+
+@pytest.mark.parametrize("prec", ["fp64", "mixed"])
+@pytest.mark.parametrize("nz", [8, 9, 1030])
+def test_flags(tmp_path, nz, prec):
+    """the convergence flags of as many modes as their workgroup adds up itself, of one more, and of two rounds"""
+    n = (20, 12, nz)
+    with context(tmp_path, "t", n, "fp64", "tensor", 3) as ctx:
+        ref, _ = project(ctx)
+    with context(tmp_path, "m", n, prec, "mg", 3) as ctx:
+        got, (it, relres) = project(ctx)
+    assert relres <= 1e-13
+    assert np.linalg.norm(got - ref) <= 1e-10 * np.linalg.norm(ref), it
