@@ -297,7 +297,10 @@ enum {
   SNAC_PH_R2R_BWD = 5,  /* inverse transforms and normfft scaling           */
   SNAC_PH_CORREC = 6,   /* correc + updt_pressure                           */
   SNAC_PH_RK_SCAL = 7,  /* rk_scal + bulk forcing of the scalars            */
-  SNAC_PH_HELMHOLTZ = 8, /* implicit diffusion: the three Helmholtz solves  */
+  SNAC_PH_HELMHOLTZ = 8, /* implicit diffusion: the three Helmholtz solves,
+                           one interval a substage where the direct solver
+                           takes them side by side, else one per stage of
+                           each component's solve                            */
   SNAC_PH_MG_LINE0 = 9, /* MG-PCG: each finest-level zebra colour sweep that
                            reads its neighbour lines, or each descent of both
                            colours in one launch: either moves 1.5 vectors of

@@ -11,11 +11,11 @@
 // Bound: the sweeps by memory (b and x of half the lines, x of the other
 // half) where a level is large, by the latency of one line's solve where it
 // is small; the coarse end (k_tail_fac) by the chain of its line solves,
-// about twenty in a row.  Measured per launch, before and after: a channel of
-// 64 modes, 512 columns, 128 rows in FP64, the sweeps over its four launched
-// levels 15.1 -> 8.9 us on average, the coarse end 110 -> 36 us; 64 modes,
-// 256 x 256 in FP32 11.2 -> 6.1 and 163 -> 75 us; the step's 48 modes, 512 x
-// 80 in FP64 11.4 -> 6.9 and 110 -> 42 us.
+// about twenty in a row.  Measured per launch, unfactored and factored: the
+// step's 48 modes, 512 x 80 in FP64, the sweeps over its four launched levels
+// 11.4 -> 6.9 us on average, the coarse end 110 -> 42 us; the coarse end of 64
+// modes, 128 rows in FP64 110 -> 36 us, of 64 modes, 256 rows in FP32 163 ->
+// 75 us.  (Levels whose columns are all alike run kernels_mgpair.hip.)
 #include "mgline_device.hpp"
 
 namespace snac {

@@ -889,8 +889,10 @@ __global__ __launch_bounds__(512) void k_r2r_mfma(MArgs a) {
 // The dense product one output per thread: lengths past the matrix-core
 // form's LDS, and the mixed-precision mode's transforms.  There FP32
 // right-hand sides turn any change of rounding, however small, into
-// differences of about 2e-9 of the velocities within a few substages, so that
-// mode keeps its operations and their order.
+// differences of about 2e-9 of the velocities within a few substages (its own
+// error is 6.6e-8).  That mode was left with its operations, their order and
+// the coefficients of r2r_coef so that its results stay what they were, not for
+// their accuracy.
 __global__ __launch_bounds__(NT) void k_r2r_dense(Args a) {
   extern __shared__ double2 S[];
   double *R = reinterpret_cast<double *>(S);
@@ -1004,7 +1006,10 @@ void launch_rfft_swapped(bool inv, bool wave, dim3 grid, size_t lds, hipStream_t
 // the matrix product's 2 n^2 operations a line take longer than its memory
 // traffic (a 192x96x96 box: 96-point lines 16 -> 12-14 us, 192-point lines
 // 23-26 -> 12-15 us); at 48 points both take 8 us, and the product takes
-// several grid blocks in one launch.
+// several grid blocks in one launch.  These twelve lengths have instances and
+// no others: the remaining even lengths with factors 2, 3 and 5 would gain as
+// well, the more the longer, and take the product for now (64 x 64 lines of 180
+// points 12-13 us, 360 25-27, 576 50-57, 960 126-128; of 384 points here 13-15).
 bool rfft_mixed_split(int n, int &n1, int &n2) {
   static const int t[][3] = {{72, 9, 4},   {80, 5, 8},   {96, 6, 8},    {120, 15, 4},  {144, 9, 8},  {160, 10, 8},
                              {192, 12, 8}, {240, 15, 8}, {288, 9, 16}, {320, 10, 16}, {384, 12, 16}, {480, 15, 16}};

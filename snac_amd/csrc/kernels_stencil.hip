@@ -31,7 +31,8 @@ __device__ __forceinline__ void tile_of(int gx, int gy, int &bx, int &by, int &b
 }
 // Which grid block a workgroup of a launch over several works on: start[q] is
 // the first workgroup of block q (the last entries repeat the total).  Cases
-// of several small grid blocks are bound by their launches, about 4 us each.
+// of several small grid blocks are bound by their launches, about 2 us each in
+// a captured step.
 template <typename Args>
 __device__ __forceinline__ int block_of(const Args &A, int &bid, int &nblk) {
   int q = 0;
@@ -53,7 +54,14 @@ __device__ __forceinline__ long dto_index(const Geo &g, int i, int j, int k) {
 // BUOY: Boussinesq buoyancy of scalar 1, -f12*gacc*beta*(face average of s)
 // (rk.f90:104-108), gb = gacc*beta
 template <bool BUOY, bool IMP>
-__device__ __forceinline__ void rk_mom_cell(int nblk, int bid, Geo g, Metrics m, const double *__restrict__ u, const double *__restrict__ v, const double *__restrict__ w, const double *__restrict__ p, double *__restrict__ un, double *__restrict__ vn, double *__restrict__ wn, double *__restrict__ dtu, double *__restrict__ dtv, double *__restrict__ dtw, double f1, double f2, double f12, double visc, double bfx, double bfy, double bfz, const double *__restrict__ s1, double gbx, double gby, double gbz) {
+__device__ __forceinline__ void rk_mom_cell(int nblk, int bid, Geo g, Metrics m, const double *__restrict__ u,
+                                            const double *__restrict__ v, const double *__restrict__ w,
+                                            const double *__restrict__ p, double *__restrict__ un,
+                                            double *__restrict__ vn, double *__restrict__ wn,
+                                            double *__restrict__ dtu, double *__restrict__ dtv,
+                                            double *__restrict__ dtw, double f1, double f2, double f12, double visc,
+                                            double bfx, double bfy, double bfz, const double *__restrict__ s1,
+                                            double gbx, double gby, double gbz) {
   int bx, by, bz;
   tile_of(nblk, bid, (g.nx + TX - 1) / TX, (g.ny + TY - 1) / TY, bx, by, bz);
   const int i = bx * TX + threadIdx.x + 1;
@@ -151,7 +159,8 @@ __global__ __launch_bounds__(TX *TY) void k_rk_mom(Geo g, Metrics m, const doubl
                                                     double visc, double bfx, double bfy, double bfz,
                                                     const double *__restrict__ s1, double gbx, double gby,
                                                     double gbz) {
-  rk_mom_cell<BUOY, IMP>(gridDim.x, blockIdx.x, g, m, u, v, w, p, un, vn, wn, dtu, dtv, dtw, f1, f2, f12, visc, bfx, bfy, bfz, s1, gbx, gby, gbz);
+  rk_mom_cell<BUOY, IMP>(gridDim.x, blockIdx.x, g, m, u, v, w, p, un, vn, wn, dtu, dtv, dtw, f1, f2, f12, visc, bfx,
+                         bfy, bfz, s1, gbx, gby, gbz);
 }
 
 template <bool BUOY, bool IMP>
@@ -576,7 +585,11 @@ __global__ __launch_bounds__(TX *TY) void k_rk_scal(Geo g, Metrics m, const doub
   dso[q] = d;
 }
 
-__device__ __forceinline__ void fillps_cell(int nblk, int bid, Geo g, Metrics m, int fa, const double *__restrict__ u, const double *__restrict__ v, const double *__restrict__ w, double *__restrict__ pp, double idtrk, const double *rx0, const double *rx1, const double *ry0, const double *ry1, const double *rz0, const double *rz1) {
+__device__ __forceinline__ void fillps_cell(int nblk, int bid, Geo g, Metrics m, int fa, const double *__restrict__ u,
+                                            const double *__restrict__ v, const double *__restrict__ w,
+                                            double *__restrict__ pp, double idtrk, const double *rx0,
+                                            const double *rx1, const double *ry0, const double *ry1,
+                                            const double *rz0, const double *rz1) {
   int bx, by, bz;
   tile_of(nblk, bid, (g.nx + TX - 1) / TX, (g.ny + TY - 1) / TY, bx, by, bz);
   const int i = bx * TX + threadIdx.x + 1;
@@ -614,7 +627,11 @@ __global__ __launch_bounds__(TX *TY) void k_fillps(Geo g, Metrics m, int fa, con
 
 // correc over the whole ghosted box; cells outside the reference's loop
 // ranges (i <= nx for u, j <= ny for v, k <= nz for w) are copied
-__device__ __forceinline__ void correc_cell(int nblk, int bid, Geo g, Metrics m, const double *__restrict__ pp, const double *__restrict__ u, const double *__restrict__ v, const double *__restrict__ w, double *__restrict__ un, double *__restrict__ vn, double *__restrict__ wn, double dtrk, double *__restrict__ p) {
+__device__ __forceinline__ void correc_cell(int nblk, int bid, Geo g, Metrics m, const double *__restrict__ pp,
+                                            const double *__restrict__ u, const double *__restrict__ v,
+                                            const double *__restrict__ w, double *__restrict__ un,
+                                            double *__restrict__ vn, double *__restrict__ wn, double dtrk,
+                                            double *__restrict__ p) {
   int bx, by, bz;
   tile_of(nblk, bid, (g.nx + 2 + TX - 1) / TX, (g.ny + 2 + TY - 1) / TY, bx, by, bz);
   const int i = bx * TX + threadIdx.x;
