@@ -325,7 +325,7 @@ def run_form(name, d, b, args, cells, dt_ref):
                 out["roofline_line0"] = {
                     "bound": "hbm", "achieved": round(bytes_ / (avg * 1e-3) / 1e9, 1), "peak": HBM_PEAK_GBS,
                     "unit": "GB/s", "frac": round(bytes_ / (avg * 1e-3) / 1e9 / HBM_PEAK_GBS, 4),
-                    "traffic": None if pair else traffic_for("k_line", args.workload, args.size, name),
+                    "traffic": traffic_for("k_pair_down" if pair else "k_line", args.workload, args.size, name),
                     "kernel": f"{'k_pair_down, finest level, both zebra colours' if pair else 'k_line, finest level, one zebra colour'} "
                               f"({'FP32' if f32 else 'FP64'}; {2 if pair and f32 else 1.5} x {esz} B per unknown)", "avg_launch_ms": round(avg, 4),
                     "launches": l0_n, "ms_per_step": round(l0_ms / ne, 4)}
