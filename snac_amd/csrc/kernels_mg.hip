@@ -1668,15 +1668,15 @@ bool launch_line_modes(hipStream_t st, const MGLevT<T> &L, const T *lam, T *x, c
                          zero_nb, pin_s, singular, done, xc, cna, E);
     SNAC_HIP(hipGetLastError());
   };
-  auto with_ends = [&](auto kk, auto fu) {
-    if (E.wa) launch(kk, fu, std::true_type{});
-    else launch(kk, fu, std::false_type{});
+  auto go = [&](auto kk) {
+    if (E.wa) launch(kk, std::false_type{}, std::true_type{});
+    else launch(kk, std::false_type{}, std::false_type{});
   };
-  auto go = [&](auto kk) { with_ends(kk, std::false_type{}); };
-  // lines of exactly LP * K rows: the instance with compile-time chunks
+  // lines of exactly LP * K rows: the instance with compile-time chunks (odd
+  // periodic levels take the general one: the same values)
   auto full = [&](auto kk) {
-    if (L.ns != LP * decltype(kk)::value) return false;
-    with_ends(kk, std::true_type{});
+    if (E.wa || L.ns != LP * decltype(kk)::value) return false;
+    launch(kk, std::true_type{}, std::false_type{});
     return true;
   };
   if constexpr (LP == 32) {

@@ -62,7 +62,8 @@ def check(tmp_path, n, even, prec, fft_axis, variants):
 
 
 @pytest.mark.parametrize("prec", ["fp64", "mixed"])
-@pytest.mark.parametrize("n", [(33, 24, 4), (90, 5, 4), (37, 3, 4), (69, 72, 4), (45, 520, 4), (11, 24, 4)])
+@pytest.mark.parametrize("n", [(33, 24, 4), (90, 5, 4), (37, 3, 4), (69, 72, 4), (45, 520, 4), (11, 24, 4),
+                               (35, 256, 4)])
 def test_modes(tmp_path, n, prec):
     even = {90: 88}.get(n[0], n[0] - 1)
     check(tmp_path, n, (even,) + n[1:], prec, 3, (-1, 0, 1, 2, 3, 4))
